@@ -1,4 +1,5 @@
-// bf16-weight linear support for gfx950 (the GEMM itself is fused_linear.hip):
+// bf16-weight linear support for gfx950 (the GEMM itself is fused_linear.hip up to 32
+// rows, big_bf16.hip above):
 // y = bf16(x) @ W^T with fp32 accumulation, rounded to bf16 like the reference's
 // bf16 matmul output (backends/mlx_ops.py:122-125).
 //

@@ -507,6 +507,10 @@ __global__ __launch_bounds__(256) void big_qkv_epilogue_kernel(const FusedArgs a
 #pragma unroll
     for (int k = 1; k < KMAX; ++k)
       if (k < KS) sum += v[k][j];
+    if (a.rnd_bf16) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] = round_bf16(sum[e]);
+    }
     *(f32x4*)&tile[(threadIdx.x >> 5) + 8 * j][(threadIdx.x & 31) * 4] = sum;
   }
   __syncthreads();
@@ -517,7 +521,8 @@ __global__ __launch_bounds__(256) void big_qkv_epilogue_kernel(const FusedArgs a
 // y = sum of the KS slices (slice order) + bias, 4 floats per thread.
 __global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int KS,
                                                          int64_t n, const uint16_t* __restrict__ bias,
-                                                         int N, float* __restrict__ y) {
+                                                         int N, float* __restrict__ y,
+                                                         int rnd_bf16) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= n) return;
   f32x4 v[8];
@@ -527,6 +532,10 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict
 #pragma unroll
   for (int k = 1; k < 8; ++k)
     if (k < KS) sum += v[k];
+  if (rnd_bf16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[e] = round_bf16(sum[e]);
+  }
   if (bias) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sum[e] += bf16_bits_to_float(bias[(i + e) % N]);
@@ -610,11 +619,11 @@ void big_linear(const FusedArgs& a, int kind, int KS, hipStream_t s, float* tail
 }
 
 void sum_slices(const float* part, int KS, int64_t n, const uint16_t* bias, int N, float* y,
-                hipStream_t s) {
+                hipStream_t s, bool rnd_bf16) {
   require(KS >= 1 && KS <= 8 && n % 4 == 0 && N % 4 == 0, "sum_slices: 1..8 slices of n % 4 == 0");
   const int64_t blocks = (n / 4 + 255) / 256;
   hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)blocks), dim3(256), 0, s, part, KS, n,
-                     bias, N, y);
+                     bias, N, y, (int)rnd_bf16);
   DRT_HIP(hipGetLastError());
 }
 

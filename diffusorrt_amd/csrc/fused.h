@@ -102,6 +102,7 @@ struct FusedArgs {
 constexpr int SK_ROW_TILES = 2;
 
 namespace drt {
+int n_cu_of_current_device();
 void fused_linear(const FusedArgs& a, int kind, hipStream_t s);
 // The split-K skinny kernels for q4 weights and M <= 32 rows; returns false
 // (launching nothing) when the arguments do not fit them.
@@ -126,6 +127,19 @@ void big_linear(const FusedArgs& a, int kind, int KS, hipStream_t s, float* tail
                 size_t tail_part_floats = 0, int* tail_count = nullptr, int n_tail_count = 0);
 size_t big_tail_part_floats(int M, int N, int K, int n_cu);
 constexpr int BIG_TAIL_COUNTERS = 512;  // split tiles a runtime's counters cover
+// The large-M bf16-weight kernels (M > 32, K % 64 == 0; big_bf16.hip): ACT_BF16
+// activation in, kinds FL_QKV, FL_SWIGLU (ACT_BF16 out) and FL_STORE (rounded with
+// the bias; ks > 1, or without rnd_bf16: fp32 slices y + ks * M * N for a reduce pass).
+struct BigBf16Plan {
+  int tile = 0;  // tile shape
+  int ks = 1;    // K slices
+  int n256 = 0;  // leading columns on 256 x 256 tiles (a launch of their own)
+};
+bool big_bf16_supported(const FusedArgs& a, int kind);
+BigBf16Plan big_bf16_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+                          float reduce_us);
+void big_bf16_linear(const FusedArgs& a, int kind, const BigBf16Plan& p, hipStream_t s);
+void big_bf16_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s);
 // q|k|v projection + epilogue: split-K into `part` (when the tiles alone would
 // leave CUs idle and part_floats suffices) and a separate epilogue pass.
 void big_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s);
@@ -155,7 +169,8 @@ void swiglu_slices(const float* part, int KS, int M, int N, void* act, int* err,
 // hidden[M][N] += the KS slices, and the new rows' partial sums of squares ss[N / 32][32]
 void residual_slices(const float* part, int KS, int M, int N, float* hidden, float* ss,
                      hipStream_t s);
-// y[i] = sum_k part[k * n + i] (+ bias[i % N]) in slice order (the per-op linear's reduce)
+// y[i] = sum_k part[k * n + i] (+ bias[i % N]) in slice order (the per-op linear's
+// reduce); rnd_bf16: the sum rounded to bf16 before the bias
 void sum_slices(const float* part, int KS, int64_t n, const uint16_t* bias, int N, float* y,
-                hipStream_t s);
+                hipStream_t s, bool rnd_bf16 = false);
 }

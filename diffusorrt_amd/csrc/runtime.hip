@@ -460,6 +460,14 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     }
     rt->streaming = rt->q4 && stream_supported(32, n_qkv, d) && stream_supported(32, d, Hq * hd) &&
                  stream_supported(32, 2 * F, d) && stream_supported(32, d, F);
+    if (!rt->q4 && M > 32 * SK_ROW_TILES) {
+      rt->act2.alloc((size_t)M * widest * 2);
+      // slices of the widest split projection: one of every row, or up to eight of
+      // the row counts that need splitting to fill the chip
+      const size_t n_max = std::max(n_qkv, d);
+      rt->big_part_floats = std::max((size_t)M, (size_t)8 * std::min(M, 512)) * n_max;
+      rt->big_part.alloc(rt->big_part_floats * 4);
+    }
     if (rt->q4 && (M > 32 || rt->streaming)) {
       rt->act2.alloc((size_t)2 * M * widest * 2);
       size_t bf = 0;
@@ -717,10 +725,10 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
   // forwards of up to SK_ROW_TILES 32-row tiles use the split-K linears, which
   // carry the RMSNorm row statistics from each residual update to the next norm
   float* ss = M <= 32 * SK_ROW_TILES ? rt.sk_ss.as<float>() : nullptr;
-  // longer q4 forwards use the large-M kernels: each linear reads an ACT_F16P
-  // activation, the RMSNorms run as their own passes, fused with the split-K
-  // reduce and residual add of the projection before them
-  const bool big = rt.q4 && M > 32 * SK_ROW_TILES;
+  // longer forwards use the large-M kernels: each linear reads a ready activation
+  // (ACT_F16P, or ACT_BF16 for bf16 weights), the RMSNorms run as their own passes,
+  // fused with the split-K reduce and residual add of the projection before them
+  const bool big = M > 32 * SK_ROW_TILES;
   // <= 32-row forwards of 7B-class layers: the weight-streaming linears (fp32 K
   // slices, reduced by small passes: residual add + row statistics, q|k|v
   // epilogue, SwiGLU; the RMSNorms run inside the next linear's staging)
@@ -751,7 +759,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
   }
   if (big && L > 0)
     residual_norm(hidden, nullptr, 0, M, false, nullptr, false,
-                  rt.layers[0].in_norm.as<uint16_t>(), eps, d, ACT_F16P, rt.act.p, xs, M, s,
+                  rt.layers[0].in_norm.as<uint16_t>(), eps, d, fmt, rt.act.p, xs, M, s,
                   rt.placement_err.as<int>());
   // split-K projection (o_proj / down_proj) into partial slices, then
   // hidden += sum of the slices and the next norm's activation
@@ -767,6 +775,14 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       stream_linear(f, sp, s);
       return sp.KS;
     }
+    if (!rt.q4) {
+      f.rnd_bf16 = 0;  // the sum of the slices is rounded by the reduce pass
+      const BigBf16Plan bp =
+          big_bf16_plan(M, f.N, f.K, FL_STORE, max_ks, rt.big_part_floats, 0.f);
+      require((size_t)bp.ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
+      big_bf16_linear(f, FL_STORE, bp, s);
+      return bp.ks;
+    }
     const int ks = big_linear_splits(M, f.N, f.K, max_ks);
     require((size_t)ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
     big_linear(f, FL_STORE, ks, s);
@@ -775,7 +791,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
   auto big_resid = [&](FusedArgs f, const uint16_t* next_norm) {
     require(f.bias == nullptr, "o_proj / down_proj bias is not supported on this path");
     const int ks = slices(f, BG_RESID_MAX_KS);
-    residual_norm(hidden, bpart, ks, M, false, nullptr, true, next_norm, eps, d, ACT_F16P,
+    residual_norm(hidden, bpart, ks, M, !rt.q4, nullptr, true, next_norm, eps, d, fmt,
                   rt.act.p, xs, M, s, rt.placement_err.as<int>());
   };
   for (int l = 0; l < L; ++l) {
@@ -825,7 +841,8 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       }
       if (big) {
         f.act = rt.act.p;
-        big_qkv(f, bpart, rt.big_part_floats, s);
+        if (rt.q4) big_qkv(f, bpart, rt.big_part_floats, s);
+        else big_bf16_qkv(f, bpart, rt.big_part_floats, s);
       } else if (stream) {  // normed from the residual stream while staged
         qkv_epilogue_slices(f, bpart, slices(f, ST_QKV_MAX_KS), s);
       } else {
@@ -870,9 +887,12 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       FusedArgs fg = base(w.gu);
       fg.act = rt.act.p;
       fg.act_out = rt.act2.p;
-      fg.act_fmt = ACT_F16P;
-      big_linear(fg, FL_SWIGLU, 1, s, bpart, rt.big_part_floats, rt.big_tail_count.as<int>(),
-                 BIG_TAIL_COUNTERS);
+      fg.act_fmt = fmt;
+      if (rt.q4)
+        big_linear(fg, FL_SWIGLU, 1, s, bpart, rt.big_part_floats, rt.big_tail_count.as<int>(),
+                   BIG_TAIL_COUNTERS);
+      else
+        big_bf16_linear(fg, FL_SWIGLU, big_bf16_plan(M, fg.N, fg.K, FL_SWIGLU, 1, 0, 0.f), s);
       FusedArgs fd = base(w.down);
       fd.act = rt.act2.p;
       big_resid(fd, last ? nullptr : rt.layers[l + 1].in_norm.as<uint16_t>());
@@ -2359,9 +2379,12 @@ int32_t drt_op_bf16_repack(const void* w, int32_t n, int32_t k, void* wb, void* 
   });
 }
 
+constexpr float BB_OP_REDUCE_US = 4.f;  // the slice sum's own launch
+// (more than 32 rows: the split-K slices)
 size_t drt_op_bf16_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
-  (void)m; (void)n; (void)k;
-  return 256;
+  if (m <= 32 || n <= 0 || k <= 0 || n % 32 || k % 64) return 256;
+  const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, SIZE_MAX, BB_OP_REDUCE_US);
+  return p.ks > 1 ? (size_t)p.ks * m * n * 4 : 256;
 }
 
 int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, int32_t k,
@@ -2370,8 +2393,6 @@ int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, 
   return guarded([&] {
     require(wb && x && y && m > 0 && n > 0 && k > 0, "bad bf16_linear arguments");
     require(n % 32 == 0 && k % 16 == 0, "bf16_linear needs n % 32 == 0 and k % 16 == 0");
-    (void)workspace;
-    (void)workspace_bytes;
     FusedArgs f;
     f.wb = (const uint16_t*)wb;
     f.bias = (const uint16_t*)bias;
@@ -2381,7 +2402,22 @@ int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, 
     f.act = x;
     f.rnd_bf16 = 1;  // the bf16 matmul output is bf16; the bias is added after
     f.y = y;
-    fused_linear(f, FL_STORE, as_stream(stream));
+    hipStream_t st = as_stream(stream);
+    if (!big_bf16_supported(f, FL_STORE)) {
+      fused_linear(f, FL_STORE, st);
+      return;
+    }
+    // as many slices as the caller's workspace holds (none is needed)
+    const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS,
+                                        workspace ? workspace_bytes / 4 : 0, BB_OP_REDUCE_US);
+    if (p.ks > 1) {
+      float* part = (float*)workspace;
+      f.y = part;
+      big_bf16_linear(f, FL_STORE, p, st);
+      sum_slices(part, p.ks, (int64_t)m * n, (const uint16_t*)bias, n, y, st, true);
+    } else {
+      big_bf16_linear(f, FL_STORE, p, st);
+    }
   });
 }
 

@@ -492,6 +492,8 @@ constexpr int ST_MAX_KS = 8;  // K slices the slice reductions take
 size_t st_lds(int ch) {
   return (size_t)2 * 32 * (ch * 64 + ST_PAD) * 2 + (size_t)ch * 32 * 4 + 32 * 4;
 }
+}  // namespace
+
 // (the CU count of the first device asked; every device this library runs on
 // is the same part; 256 where no device answers, e.g. a workspace query made
 // without a GPU)
@@ -509,7 +511,6 @@ int n_cu_of_current_device() {
   }
   return cached;
 }
-}  // namespace
 
 bool stream_supported(int M, int N, int K) {
   return M >= 1 && M <= 32 && N % 128 == 0 && K % 64 == 0 &&

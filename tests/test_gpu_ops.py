@@ -165,6 +165,45 @@ def test_bf16_linear(m, n, k):
     assert rel < 1e-2
 
 
+# The large-M bf16 kernels: row and column remainders of every tile (64, 128, 256),
+# fewer 64-k stages than stage buffers, split K, whole rounds of 256 x 256 tiles with
+# the last columns on 128 x 128 ones (520 x 22400 on 256 CUs), and a K that is not
+# whole stages (the general kernel).
+@pytest.mark.parametrize("m,n,k,with_ws", [
+    (33, 32, 64, True), (64, 160, 128, True), (65, 992, 192, True), (129, 1024, 3072, True),
+    (129, 1024, 3072, False), (257, 4064, 1024, True), (520, 22400, 1024, True),
+    (70, 256, 80, True)])
+def test_bf16_linear_large_m(m, n, k, with_ws):
+    import ctypes as C
+
+    from diffusorrt_amd import _lib, kernels
+
+    _say("bf16_linear large M", m, n, k, "workspace" if with_ws else "no workspace")
+    gen = torch.Generator().manual_seed(12)
+    wt = (torch.randn((n, k), generator=gen) * 0.02).to(torch.bfloat16)
+    bias = torch.randn((n,), generator=gen).to(torch.bfloat16)
+    x = torch.randn((m, k), generator=gen)
+    w = kernels.DeviceBF16Weight(wt.cuda())
+    if with_ws:
+        y = kernels.linear(x.cuda(), w, bias.cuda())
+    else:  # the entry point needs no workspace: it then does not split K
+        xb, bd = x.to(torch.bfloat16).cuda(), bias.cuda()
+        y = torch.empty((m, n), device="cuda")
+        _lib.check(_lib.load().drt_op_bf16_linear(
+            C.c_void_p(w.wb.data_ptr()), C.c_void_p(xb.data_ptr()), m, n, k,
+            C.c_void_p(bd.data_ptr()), C.c_void_p(y.data_ptr()), None, 0,
+            C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    y = y.cpu().numpy().astype(np.float64)
+    exact = x.to(torch.bfloat16).double().numpy() @ wt.double().numpy().T
+    err = np.abs((y - bias.double().numpy()) - exact)
+    # half a bf16 ulp of the product (2^-8 of it), the fp32 sums' own error ahead of the
+    # rounding, and the fp32 addition of the bias
+    mag = np.abs(x.to(torch.bfloat16).double().numpy()) @ np.abs(wt.double().numpy()).T
+    bound = np.abs(exact) * 2.0 ** -8 + mag * k * 2.0 ** -24 + 2.0 ** -22 * (1 + np.abs(y))
+    _say(f"  worst error / bound {np.max(err / bound):.3f}")
+    assert (err <= bound).all()
+
+
 # ---------------------------------------------------------------- attention (config 2)
 
 def _attention_inputs(L, seed=1, rows=32, hq=16, hkv=8):
