@@ -380,6 +380,8 @@ BigBf16Plan big_bf16_plan(int M, int N, int K, int kind, int max_ks, size_t part
 }
 
 bool big_bf16_supported(const FusedArgs& a, int kind) {
+  // (16-byte loads straight into LDS: aligned operands only)
+  if ((((uintptr_t)a.wb | (uintptr_t)a.act) & 15) != 0) return false;
   if (!a.wb || a.qw || !a.act || a.M <= 32 || a.N % 32 || a.K % 64 || a.K < 64) return false;
   if (kind == FL_SWIGLU) return a.N % 128 == 0 && a.act_fmt == ACT_BF16;
   if (kind == FL_QKV) return a.N % 128 == 0;

@@ -518,29 +518,31 @@ __global__ __launch_bounds__(256) void big_qkv_epilogue_kernel(const FusedArgs a
   qkv_epilogue<T>(a, qt, head, mp, row0 + mp, rows, get, vbuf);
 }
 
-// y = sum of the KS slices (slice order) + bias, 4 floats per thread.
-__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int KS,
-                                                         int64_t n, const uint16_t* __restrict__ bias,
-                                                         int N, float* __restrict__ y,
-                                                         int rnd_bf16) {
+// y = sum of the KS slices (slice order) + bias, 4 floats per thread, every slice's load
+// issued before the first add (2 slices of 2048 x 3072, 75 MB: 12.6 -> 11.9 us, 2048 x 1024: 8.3 -> 5.4; always eight
+// loads, the last slice's repeated, before).
+template <int KS>
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int64_t n,
+                                                         const uint16_t* __restrict__ bias, int N,
+                                                         float* __restrict__ y, int rnd_bf16) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= n) return;
-  f32x4 v[8];
+  f32x4 v[KS];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) v[k] = *(const f32x4*)(part + (int64_t)min(k, KS - 1) * n + i);
+  for (int k = 0; k < KS; ++k) v[k] = *(const f32x4*)(part + k * n + i);
   f32x4 sum = v[0];
 #pragma unroll
-  for (int k = 1; k < 8; ++k)
-    if (k < KS) sum += v[k];
+  for (int k = 1; k < KS; ++k) sum += v[k];
   if (rnd_bf16) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sum[e] = round_bf16(sum[e]);
   }
-  if (bias) {
+  if (bias) {  // N % 4 == 0: the four columns are one row's
+    const int c = (int)(i % N);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sum[e] += bf16_bits_to_float(bias[(i + e) % N]);
+    for (int e = 0; e < 4; ++e) sum[e] += bf16_bits_to_float(bias[c + e]);
   }
-  *(f32x4*)(y + i) = sum;
+  *(f32x4_e*)(y + i) = sum;
 }
 
 template __global__ void big_qkv_epilogue_kernel<_Float16>(const FusedArgs, const float*, int);
@@ -622,8 +624,16 @@ void sum_slices(const float* part, int KS, int64_t n, const uint16_t* bias, int 
                 hipStream_t s, bool rnd_bf16) {
   require(KS >= 1 && KS <= 8 && n % 4 == 0 && N % 4 == 0, "sum_slices: 1..8 slices of n % 4 == 0");
   const int64_t blocks = (n / 4 + 255) / 256;
-  hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)blocks), dim3(256), 0, s, part, KS, n,
-                     bias, N, y, (int)rnd_bf16);
+#define DRT_SS(K)                                                                              \
+  case K:                                                                                      \
+    hipLaunchKernelGGL(sum_slices_kernel<K>, dim3((unsigned)blocks), dim3(256), 0, s, part, n, \
+                       bias, N, y, (int)rnd_bf16);                                             \
+    break;
+  switch (KS) {
+    DRT_SS(1) DRT_SS(2) DRT_SS(3) DRT_SS(4) DRT_SS(5) DRT_SS(6) DRT_SS(7)
+    DRT_SS(8)
+  }
+#undef DRT_SS
   DRT_HIP(hipGetLastError());
 }
 

@@ -19,6 +19,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// the same for tensors known only to be aligned to their element (views into a larger
+// buffer): one 16-byte access, which the hardware takes at any address
+typedef float f32x4_e __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_e __attribute__((ext_vector_type(4), aligned(2)));
 
 #define DRT_DEV __device__ __forceinline__
 

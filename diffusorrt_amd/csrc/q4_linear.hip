@@ -58,24 +58,48 @@ extern "C" __global__ void q4_repack_kernel(const uint32_t* __restrict__ w_q,
 }
 
 // fp32 (or bf16) activation rows -> ACT_F16P (hi plane, lo plane at + M*K) +
-// group sums of hi + lo. One wave per (row, group).
-extern "C" __global__ void q4_act_prep_kernel(const void* __restrict__ x, int x_is_bf16,
-                                              _Float16* __restrict__ xp,
-                                              float* __restrict__ xsum, int M, int K) {
-  const int G = K >> 6;
-  const int lane = threadIdx.x & 63;
-  const int64_t wid = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-  if (wid >= (int64_t)M * G) return;
-  const int64_t m = wid / G, g = wid % G;
-  const int k = (int)g * 64 + lane;
-  float v;
-  if (x_is_bf16) v = bf16_bits_to_float(((const uint16_t*)x)[m * K + k]);
-  else v = ((const float*)x)[m * K + k];
-  const _Float16 h = (_Float16)v, lo = f16_lo(v, h);
-  xp[m * K + f16p_index(k)] = h;
-  xp[(int64_t)M * K + m * K + f16p_index(k)] = lo;
-  const float s = wave_sum((float)h + (float)lo);
-  if (lane == 0) xsum[m * G + g] = s;
+// group sums of hi + lo. Bound by its bytes: a thread owns one 8-element chunk, so
+// every access is 16 bytes and a group's sum is over 8 lanes (2048 x 3072 fp32, 50 MB:
+// 19.2 -> 8.8 us).
+template <bool BF16>
+__global__ __launch_bounds__(256) void q4_act_prep_kernel(const void* __restrict__ x,
+                                                          _Float16* __restrict__ xp,
+                                                          float* __restrict__ xsum, int64_t chunks,
+                                                          int64_t plane) {
+  const int64_t c = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (c >= chunks) return;  // whole groups of 8 lanes (K % 64 == 0)
+  float v[8];
+  if (BF16) {
+    const u32x4 w = *(const u32x4_e*)((const uint16_t*)x + c * 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[2 * e] = bf16_bits_to_float(w[e] & 0xffffu);
+      v[2 * e + 1] = bf16_bits_to_float(w[e] >> 16);
+    }
+  } else {
+    const f32x4 a = *(const f32x4_e*)((const float*)x + c * 8);
+    const f32x4 b = *(const f32x4_e*)((const float*)x + c * 8 + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
+    }
+  }
+  _Float16 h[8], lo[8];
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const _Float16 he = (_Float16)v[e], le = f16_lo(v[e], he);
+    h[f16p_index(e)] = he;
+    lo[f16p_index(e)] = le;
+    s += (float)he + (float)le;
+  }
+  *(u32x4*)(xp + c * 8) = __builtin_bit_cast(u32x4, h);
+  *(u32x4*)(xp + plane + c * 8) = __builtin_bit_cast(u32x4, lo);
+  s += __shfl_xor(s, 1, 64);
+  s += __shfl_xor(s, 2, 64);
+  s += __shfl_xor(s, 4, 64);
+  if ((threadIdx.x & 7) == 0) xsum[c >> 3] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -95,9 +119,12 @@ void q4_repack(const uint32_t* w_q, const uint16_t* scales, const uint16_t* bias
 
 void q4_act_prep(const void* x, bool x_bf16, int M, int K, _Float16* xp, float* xsum,
                  hipStream_t s) {
-  const int64_t waves = (int64_t)M * (K / 64);
-  hipLaunchKernelGGL(q4_act_prep_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, x,
-                     (int)x_bf16, xp, xsum, M, K);
+  const int64_t plane = (int64_t)M * K, chunks = plane / 8;
+  const dim3 grid((unsigned)((chunks + 255) / 256));
+  if (x_bf16)
+    hipLaunchKernelGGL(q4_act_prep_kernel<true>, grid, dim3(256), 0, s, x, xp, xsum, chunks, plane);
+  else
+    hipLaunchKernelGGL(q4_act_prep_kernel<false>, grid, dim3(256), 0, s, x, xp, xsum, chunks, plane);
   DRT_HIP(hipGetLastError());
 }
 

@@ -523,3 +523,85 @@ def test_lm_head_sampling_matches_oracle_rule(kind, n, k):
                                       positions=positions.cpu().tolist())
     assert tokens.cpu().tolist() == t_ref
     np.testing.assert_allclose(scores.cpu().numpy(), s_ref, rtol=1e-6)
+
+
+# ---------------------------------------------------------------- per-op elementwise kernels
+
+# widths on both sides of every lanes-per-row step and off the 16-byte grid, tensors that
+# start off it too (views into a larger buffer), and cache tiles written in part
+@pytest.mark.parametrize("rows,d,off", [(1, 4, 0), (7, 128, 1), (3, 132, 0), (5, 516, 3), (2, 1028, 0),
+                                        (3, 2052, 0), (2, 4096, 1), (2, 4100, 0), (3, 130, 0)])
+def test_rms_norm_widths_and_offsets(rows, d, off):
+    from diffusorrt_amd import kernels
+
+    _say("rms_norm", rows, d, "offset", off)
+    gen = torch.Generator().manual_seed(31)
+    flat = torch.randn(rows * d + off, generator=gen) * 3
+    x = flat[off:].view(rows, d)
+    w = (1 + 0.1 * torch.randn(d, generator=gen)).to(torch.bfloat16)
+    y = kernels.rms_norm(flat.cuda()[off:].view(rows, d), w.cuda(), 1e-6).cpu().double()
+    xd = x.double()
+    ref = xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-6) * w.double()
+    # an fp32 sum of d squares (d * 2^-24 relative, halved by the square root) and six
+    # rounded operations after it
+    assert ((y - ref).abs() <= ref.abs() * (d + 12) * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("rows,h,hd,off", [(1, 1, 8, 0), (9, 3, 128, 1), (5, 2, 12, 0), (33, 16, 64, 0)])
+def test_rope_widths_and_offsets(rows, h, hd, off):
+    from diffusorrt_amd import kernels
+
+    _say("rope", rows, h, hd, "offset", off)
+    gen = torch.Generator().manual_seed(32)
+    flat = torch.randn(rows * h * hd + off, generator=gen)
+    c, s = torch.randn((rows, 1, hd), generator=gen), torch.randn((rows, 1, hd), generator=gen)
+    y = kernels.rope(flat.cuda()[off:].view(rows, h, hd), c.cuda(), s.cuda()).cpu().double()
+    x = flat[off:].view(rows, h, hd).double()
+    rot = torch.cat([-x[..., hd // 2:], x[..., :hd // 2]], -1)
+    a, b = x * c.double(), rot * s.double()
+    # two products and a sum, each rounded once
+    assert ((y - (a + b)).abs() <= (a.abs() + b.abs()) * 2.0 ** -22).all()
+
+
+@pytest.mark.parametrize("m,off", [(33, 0), (5, 3)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_q4_linear_activation_offsets(m, off, dtype):
+    from diffusorrt_amd import kernels
+
+    _say("q4_linear activation", m, dtype, "offset", off)
+    gen, q = _q4_case(4096, 2048, seed=33)
+    flat = torch.randn(m * 2048 + off, generator=gen)
+    flat = flat.to(torch.bfloat16) if dtype == "bf16" else flat
+    w = kernels.DeviceQ4Weight(q.w_q.cuda(), q.scales.cuda(), q.biases.cuda())
+    y = kernels.linear(flat.cuda()[off:].view(m, 2048), w).cpu()
+    # the same rows from an aligned tensor: the same kernels, bit for bit
+    assert torch.equal(y, kernels.linear(flat[off:].view(m, 2048).contiguous().cuda(), w).cpu())
+
+
+@pytest.mark.parametrize("pos0,n,src,kv", [(0, 32, "f32", "f16"), (5, 3, "f32", "f16"),
+                                           (30, 70, "bf16", "bf16"), (64, 33, "bf16", "f16"),
+                                           (17, 15, "f32", "bf16")])
+def test_kv_store_partial_tiles(pos0, n, src, kv):
+    from diffusorrt_amd.kernels import PrefixKVCache
+
+    _say("kv store", pos0, n, src, kv)
+    gen = torch.Generator().manual_seed(34)
+    hkv, tdt = 3, (torch.float16 if kv == "f16" else torch.bfloat16)
+    cache = PrefixKVCache(1, hkv, 128, dtype=kv)
+    k, v = (torch.randn((n, hkv, 128), generator=gen) for _ in range(2))
+    if src == "bf16":
+        k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    cache.data.fill_(7.0)
+    cache.store(0, k.cuda(), v.cuda(), pos0)
+    tiles = cache.data[0].cpu().view(hkv, -1, 2, 4096)
+    want = torch.full_like(tiles, 7.0)
+    hd = torch.arange(128)
+    for r in range(n):
+        t, kk = divmod(pos0 + r, 32)
+        q16 = kk & 15
+        ko = ((hd >> 3) * 32 + kk) * 8 + (hd & 7)
+        vo = ((((hd >> 5) * 2 + (kk >> 4)) * 2 + ((q16 >> 2) & 1)) * 32 + (hd & 31)) * 8 + \
+            (q16 & 3) + 4 * (q16 >> 3)
+        want[:, t, 0, ko] = k[r].to(tdt)
+        want[:, t, 1, vo] = v[r].to(tdt)
+    assert torch.equal(tiles, want)
