@@ -24,6 +24,8 @@
 #include "common.h"
 #include "launch.h"
 
+#include <cmath>
+
 namespace {
 
 template <typename T> struct MfmaT;
@@ -35,9 +37,7 @@ template <> struct MfmaT<_Float16> {
 template <> struct MfmaT<__bf16> {
   typedef bf16x8 vec;
   static DRT_DEV f32x16 mma(vec a, vec b, f32x16 c) { return mfma_bf16(a, b, c); }
-  static DRT_DEV __bf16 from_float(float f) {
-    return __builtin_bit_cast(__bf16, float_to_bf16_bits(f));
-  }
+  static DRT_DEV __bf16 from_float(float f) { return (__bf16)f; }
 };
 
 DRT_DEV int eff_block(int p, int prompt_len, int block) {
@@ -64,202 +64,299 @@ DRT_DEV float max_xor32(float v) {
 }
 
 
-template <typename T, int QW>
-__global__ __launch_bounds__(64 * QW) void attn_split_kernel(
+// Output of the long-query attention: eight consecutive columns c0 .. of a row, by
+// eight lanes per 64-column group. fmt: 0 = ACT_F16P (hi plane, lo plane at + n_rows *
+// D, group sums), 1 = ACT_BF16, 2 = fp32 plain, 3 = bf16 plain.
+struct AttnOut {
+  void* out;
+  float* xsum;
+  int* err;
+  int fmt;
+};
+DRT_DEV void store_attn8(const f32x4 v0, const f32x4 v1, int row, int n_rows, int c0, int D,
+                         int lane, const AttnOut& ao) {
+  const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+  if (ao.fmt == 0) {
+    _Float16 h[8], lo[8];
+    float gs = 0.f;
+    bool over = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const _Float16 he = (_Float16)v[e], le = f16_lo(v[e], he);
+      h[f16p_index(e)] = he;
+      lo[f16p_index(e)] = le;
+      gs += (float)he + (float)le;
+      over = over || f16_overflows(v[e]);
+    }
+    _Float16* o = (_Float16*)ao.out + (int64_t)row * D + c0;
+    *(u32x4*)o = __builtin_bit_cast(u32x4, h);
+    *(u32x4*)(o + (int64_t)n_rows * D) = __builtin_bit_cast(u32x4, lo);
+    if (over && ao.err) atomicOr(ao.err, DRT_ERR_F16_RANGE);
+    gs += __shfl_xor(gs, 1, 64);
+    gs += __shfl_xor(gs, 2, 64);
+    gs += __shfl_xor(gs, 4, 64);
+    if ((lane & 7) == 0) ao.xsum[(int64_t)row * (D >> 6) + (c0 >> 6)] = gs;
+  } else if (ao.fmt == 1 || ao.fmt == 3) {
+    uint16_t hb[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) hb[e] = float_to_bf16_bits(v[e]);
+    *(u32x4*)((uint16_t*)ao.out + (int64_t)row * D + c0) = __builtin_bit_cast(u32x4, hb);
+  } else {
+    float* o = (float*)ao.out + (int64_t)row * D + c0;
+    *(f32x4*)o = v0;
+    *(f32x4*)(o + 4) = v1;
+  }
+}
+
+// Long-query attention: a wave owns one 32-vector query tile, the QW waves of a
+// key group share 32-key K/V tiles, streamed by direct-to-LDS loads into a ring of
+// three 16 KiB slots (tile t + 2 is issued once tile t has arrived and every wave is
+// done with t - 1: one barrier per tile, no registers held by the loads). Two or three
+// waves per SIMD overlap one's softmax (VALU) with another's products (MFMA): either
+// alone takes about as long as the other. The
+// softmax is kept to a max, an fma, an exp2, an add and half a conversion per
+// score: the scale is folded into the exponent's fma and the mask is tested only in
+// tiles that not every row of the wave sees whole. LO: Q has a lo plane (without it
+// the products with it are left out).
+// OUT: a single split writes the attention itself (out_fmt as in
+// attn_combine_kernel) instead of a partial for the combine.
+// KG: key groups of a work-group, each with its own QW waves over a contiguous share of
+// the keys; their parts meet in LDS at the end.
+// 2048 rows x 16 heads over 4096 keys, bf16: 135 -> 77 us with the combine (671 TFLOP/s; K/V
+// staged through registers, products with a zero lo plane, a mask test per score before).
+template <typename T, int QW, int KG, bool LO, bool OUT>
+DRT_DEV void attn_split_tile(
     const T* __restrict__ q,       // [n_rows][Hq][128]
-    const T* __restrict__ q_lo,    // its lo plane (the same layout), or null (zero)
+    const T* __restrict__ q_lo,    // its lo plane (the same layout; LO)
     const T* __restrict__ kv,      // this layer: [Hkv][tile_cap][8192]
     int64_t kv_head_stride,        // elements between kv heads
     int n_rows, int Hq, int Hkv, int n_keys, int row_pos0,
     int mask_kind, int mask_prompt_len, int mask_block, int tiles_per_split,
     float* __restrict__ o_part,    // [splits][Hkv][n_qv][128]
     float* __restrict__ ml_part,   // [splits][Hkv][n_qv][2]
-    float scale) {
+    float scale, const AttnOut& ao) {
   typedef typename MfmaT<T>::vec vec;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int qw = wave % QW, kg = wave / QW;  // query tile and key group of this wave
   const int G = Hq / Hkv;
   const int n_qv = n_rows * G;
-  const int n_splits = gridDim.x / Hkv;
   const int split = blockIdx.x / Hkv;
   const int kvh = blockIdx.x - split * Hkv;
-  const int qt = blockIdx.y * QW + wave;
+  const int qt = blockIdx.y * QW + qw;
   const int n_tiles = (n_keys + 31) >> 5;
   const int t_begin = split * tiles_per_split;
   const int t_end = min(n_tiles, t_begin + tiles_per_split);
 
-  extern __shared__ __align__(16) char smem[];
-  T* lds = (T*)smem;  // [2][8192]
+  constexpr int TILE_BYTES = KV_TILE_ELEMS * 2;
+  static_assert(QW * 8192 <= 2 * TILE_BYTES, "a half head of every query must fit two slots");
+  // separate arrays: the compiler knows the slot being read is not one being filled
+  constexpr int SLOT = KG * TILE_BYTES;
+  __shared__ __align__(1024) char ring0[SLOT];
+  __shared__ __align__(1024) char ring1[SLOT];
+  __shared__ __align__(1024) char ring2[SLOT];
+  __shared__ float2 ml[KG > 1 ? KG * QW * 32 : 1];
 
   // This lane's query (B operand of S^T) and its absolute position.
   const int qv = qt * 32 + (lane & 31);
   const bool q_ok = qv < n_qv;
   const int qrow = q_ok ? qv / G : 0;
   const int qhead = kvh * G + (q_ok ? qv - (qv / G) * G : 0);
-  vec qf[8], qfl[8];  // Q hi / lo planes
+  vec qf[8], qfl[LO ? 8 : 1];  // Q hi / lo planes
   {
     const int64_t qo = ((int64_t)qrow * Hq + qhead) * 128 + 8 * (lane >> 5);
-    const T* qp = q + qo;
-    const T* qpl = (q_lo ? q_lo : q) + qo;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if (q_ok) {
-        qf[i] = *(const vec*)(qp + 16 * i);
-        qfl[i] = *(const vec*)(qpl + 16 * i);
-        if (!q_lo) qfl[i] = vec{};
-      } else {
-        qf[i] = qfl[i] = vec{};
-      }
+      qf[i] = *(const vec*)(q + qo + 16 * i);
+      if (LO) qfl[LO ? i : 0] = *(const vec*)(q_lo + qo + 16 * i);
     }
   }
-  const int qpos = row_pos0 + qrow;
   const float c = scale * 1.44269504088896340736f;  // scores to base-2 exponents
   // d2f_hybrid: a query sees exactly the keys before the end of its own block
   // (the whole prompt, then whole blocks up to its own), so visibility is one
-  // compare per key against q_key_end
-  int q_key_end = n_keys;
-  if (mask_kind == 1) {
-    const int e = eff_block(qpos, mask_prompt_len, mask_block);
-    q_key_end = min(n_keys, e < 0 ? mask_prompt_len : mask_prompt_len + (e + 1) * mask_block);
-  }
-  // Wave-uniform visibility bound: no key beyond the last visible key of the
-  // wave's rows needs loading into this wave's math.
-  int wave_key_end = n_keys;
-  if (mask_kind == 1) {
-    const int last_row = min(n_rows - 1, (qt * 32 + 31) / G);
-    const int e = eff_block(row_pos0 + last_row, mask_prompt_len, mask_block);
-    wave_key_end = min(n_keys, e < 0 ? mask_prompt_len : mask_prompt_len + (e + 1) * mask_block);
-  }
-  // WG-uniform bound (the last wave's rows are the latest).
-  int wg_key_end = n_keys;
-  if (mask_kind == 1) {
-    const int last_row = min(n_rows - 1, (blockIdx.y * QW * 32 + QW * 32 - 1) / G);
-    const int e = eff_block(row_pos0 + last_row, mask_prompt_len, mask_block);
-    wg_key_end = min(n_keys, e < 0 ? mask_prompt_len : mask_prompt_len + (e + 1) * mask_block);
-  }
-  const int t_stop = min(t_end, (wg_key_end + 31) >> 5);
+  // compare per key against the row's end, which never falls from row to row.
+  auto key_end = [&](int row) {
+    if (mask_kind != 1) return n_keys;
+    const int e = eff_block(row_pos0 + row, mask_prompt_len, mask_block);
+    return min(n_keys, e < 0 ? mask_prompt_len : mask_prompt_len + (e + 1) * mask_block);
+  };
+  const int q_key_end = key_end(qrow);
+  // uniform bounds: keys every row of the wave sees, keys any of them sees, and
+  // keys any row of the work-group sees (its last wave's rows are the latest)
+  const int wave_full = key_end(min(n_rows - 1, qt * 32 / G));
+  const int wave_end = key_end(min(n_rows - 1, (qt * 32 + 31) / G));
+  const int wg_end = key_end(min(n_rows - 1, ((int)blockIdx.y * QW * 32 + QW * 32 - 1) / G));
+  const int t_stop = min(t_end, (wg_end + 31) >> 5);
+  // this key group's tiles: a contiguous share of the split's (masked) range
+  const int per = mask_kind == 1 ? (max(0, t_stop - t_begin) + KG - 1) / KG : tiles_per_split / KG;
+  const int kt0 = t_begin + kg * per, kt1 = min(t_stop, kt0 + per);
+  const int n_it = min(per, t_stop - t_begin);  // iterations (every group's)
 
   float m_run = -INFINITY, l_run = 0.f;
   f32x16 o[4];
 #pragma unroll
   for (int hb = 0; hb < 4; ++hb) o[hb] = f32x16{};
 
-  const T* kvh_base = kv + (int64_t)kvh * kv_head_stride;
-  constexpr int VEC_PER_TILE = KV_TILE_ELEMS / 8;  // 16-byte vectors per tile
-  constexpr int PER_THREAD = VEC_PER_TILE / (64 * QW);
-  // K/V tiles go global -> registers -> LDS (double buffered), loaded two tiles
-  // ahead through two register stages (tile t + 2 is in flight while tile t is
-  // computed and tile t + 1 is stored), so a tile's memory latency overlaps two
-  // iterations' work instead of one.
-  u32x4 stage_a[PER_THREAD], stage_b[PER_THREAD];
-  auto load_tile = [&](u32x4 (&st)[PER_THREAD], int t) {
-    const u32x4* src = (const u32x4*)(kvh_base + (int64_t)t * KV_TILE_ELEMS);
+  const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(kv + (int64_t)kvh * kv_head_stride), 0, (uint32_t)n_tiles * TILE_BYTES, 0x00020000);
+  constexpr int LD = TILE_BYTES / 1024 / QW;  // 1 KiB loads per wave and slot
+  // tile it of this wave's key group (past the cache's last tile: zeros, never used)
+  auto issue = [&](int it, char* dst) {
 #pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) st[i] = src[threadIdx.x + i * 64 * QW];
+    for (int i = 0; i < LD; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src, (__attribute__((address_space(3))) void*)(dst + (wave * LD + i) * 1024), 16,
+          (uint32_t)((kt0 + it) * TILE_BYTES + (qw * LD + i) * 1024 + lane * 16), 0, 0, 0);
   };
-  auto store_tile = [&](const u32x4 (&st)[PER_THREAD], int buf) {
-    u32x4* dst = (u32x4*)(lds + buf * KV_TILE_ELEMS);
+  auto compute = [&](int it, const char* slot) {
+    const int t = kt0 + it, key0 = t * 32;
+    if (key0 >= wave_end || t >= kt1) return;
+    const T* kt = (const T*)(slot + kg * TILE_BYTES);
+    const T* vt = kt + 4096;
+    f32x16 s = f32x16{};
 #pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) dst[threadIdx.x + i * 64 * QW] = st[i];
-  };
-  auto compute = [&](int t, int buf) {
-    const int key0 = t * 32;
-    if (key0 < wave_key_end) {
-      const T* kt = lds + buf * KV_TILE_ELEMS;
-      const T* vt = kt + 4096;
-      f32x16 s = f32x16{};
+    for (int i = 0; i < 8; ++i) {
+      const vec kf = *(const vec*)(kt + (i * 64 + lane) * 8);
+      s = MfmaT<T>::mma(kf, qf[i], s);
+      if (LO) s = MfmaT<T>::mma(kf, qfl[LO ? i : 0], s);
+    }
+    if (key0 + 32 > wave_full) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const vec kf = *(const vec*)(kt + (i * 64 + lane) * 8);
-        s = MfmaT<T>::mma(kf, qf[i], s);
-        s = MfmaT<T>::mma(kf, qfl[i], s);
+      for (int r = 0; r < 16; ++r) s[r] = key0 + mfma_row(r, lane) < q_key_end ? s[r] : -INFINITY;
+    }
+    float tmax = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
+    tmax = max_xor32(tmax) * c;  // -inf: no visible key in the tile
+    const bool up = tmax > m_run + DEC_RESCALE_LOG2;
+    if (__ballot(up)) {  // some base has to rise (rare after the first tiles)
+      const float alpha = up ? __builtin_amdgcn_exp2f(m_run - tmax) : 1.f;  // 0 from -inf
+      if (__ballot(up && m_run != -INFINITY)) {
+#pragma unroll
+        for (int hb = 0; hb < 4; ++hb) o[hb] *= alpha;
       }
-      float tmax = -INFINITY;
+      l_run *= alpha;
+      m_run = up ? tmax : m_run;
+    }
+    const float base = m_run == -INFINITY ? 0.f : m_run;  // no key yet: p = 0
+    float psum = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[r] = key0 + mfma_row(r, lane) < q_key_end ? s[r] * c : -INFINITY;
-        tmax = fmaxf(tmax, s[r]);
+    for (int kh = 0; kh < 2; ++kh) {
+      vec pf;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[kh * 8 + j], c, -base));
+        psum += p;
+        pf[j] = MfmaT<T>::from_float(p);
       }
-      tmax = max_xor32(tmax);  // -inf: no visible key in the tile
-      const bool up = tmax > m_run + DEC_RESCALE_LOG2;
-      if (__ballot(up)) {  // some base has to rise (rare after the first tiles)
-        const float alpha = up ? __builtin_amdgcn_exp2f(m_run - tmax) : 1.f;  // 0 from -inf
-        if (__ballot(up && m_run != -INFINITY)) {
 #pragma unroll
-          for (int hb = 0; hb < 4; ++hb) o[hb] *= alpha;
-        }
-        l_run *= alpha;
-        m_run = up ? tmax : m_run;
-      }
-      const float base = m_run == -INFINITY ? 0.f : m_run;  // no key yet: p = 0
-      float psum = 0.f;
-      float p[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p[r] = __builtin_amdgcn_exp2f(s[r] - base);
-        psum += p[r];
-      }
-      l_run += psum;
-#pragma unroll
-      for (int kh = 0; kh < 2; ++kh) {
-        vec pf;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pf[j] = MfmaT<T>::from_float(p[kh * 8 + j]);
-#pragma unroll
-        for (int hb = 0; hb < 4; ++hb) {
-          const vec vf = *(const vec*)(vt + (((hb * 2 + kh) * 64) + lane) * 8);
-          o[hb] = MfmaT<T>::mma(vf, pf, o[hb]);
-        }
+      for (int hb = 0; hb < 4; ++hb) {
+        const vec vf = *(const vec*)(vt + (((hb * 2 + kh) * 64) + lane) * 8);
+        o[hb] = MfmaT<T>::mma(vf, pf, o[hb]);
       }
     }
+    l_run += psum;
   };
-
-  if (t_begin < t_stop) {
-    load_tile(stage_a, t_begin);
-    store_tile(stage_a, 0);
-  }
-  if (t_begin + 1 < t_stop) load_tile(stage_b, t_begin + 1);
-  __syncthreads();
-  // two tiles per pass: buffer 0 / stage_a for tiles t_begin + 2k, buffer 1 /
-  // stage_b for tiles t_begin + 2k + 1. A buffer is rewritten only after the
-  // barrier that follows its last read.
-  for (int t = t_begin; t < t_stop; t += 2) {
-    if (t + 2 < t_stop) load_tile(stage_a, t + 2);
-    compute(t, 0);
-    if (t + 1 >= t_stop) break;
-    store_tile(stage_b, 1);
-    __syncthreads();
-    if (t + 3 < t_stop) load_tile(stage_b, t + 3);
-    compute(t + 1, 1);
-    if (t + 2 >= t_stop) break;
-    store_tile(stage_a, 0);
-    __syncthreads();
+  // iteration it in slot it % 3; at most one later slot's loads are in flight while its
+  // own are awaited
+  auto step = [&](int it, char* here, char* two_on) {
+    if (it + 1 < n_it) __builtin_amdgcn_s_waitcnt(0x0F70 | LD);  // vmcnt(LD): its tile is here
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (it + 2 < n_it) issue(it + 2, two_on);
+    compute(it, here);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave is done reading the slot
+  };
+  if (n_it > 0) issue(0, ring0);
+  if (n_it > 1) issue(1, ring1);
+  asm volatile("" ::: "memory");
+  for (int it = 0; it < n_it; it += 3) {
+    step(it, ring0, ring2);
+    if (it + 1 >= n_it) break;
+    step(it + 1, ring1, ring0);
+    if (it + 2 >= n_it) break;
+    step(it + 2, ring2, ring1);
   }
   l_run += __shfl_xor(l_run, 32, 64);
 
-  // Transpose O^T through LDS so each query's 128 values are written contiguously.
-  __syncthreads();
-  float* ot = (float*)smem + wave * (32 * 132);
-#pragma unroll
-  for (int hb = 0; hb < 4; ++hb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) ot[(lane & 31) * 132 + hb * 32 + mfma_row(r, lane)] = o[hb][r];
-  __syncthreads();
+  // O^T through LDS, half a head (64 dims) at a time, so that eight lanes write a
+  // query's half: element (query, dim) at query * 64 + (dim ^ 4 * (query & 15)) of its
+  // wave's 8 KiB. The key groups' halves meet there: each group's waves write out a
+  // share of the queries, adding every group's part against the largest base.
+  __syncthreads();  // every wave is done with the ring
+  char* half0[2] = {ring0, ring1};  // QW waves of a key group over the two arrays
+  auto region = [&](int g) {
+    return (float*)(half0[qw >= (QW + 1) / 2] + (g * ((QW + 1) / 2) + qw % ((QW + 1) / 2)) * 8192);
+  };
+  float* ot = region(kg);
+  if (KG > 1 && lane < 32) ml[(kg * QW + qw) * 32 + lane] = make_float2(m_run, l_run);
   const int64_t part_base = ((int64_t)split * Hkv + kvh) * n_qv;
-  for (int i = lane; i < 32 * 32; i += 64) {
-    const int qq = i >> 5, c4 = (i & 31) * 4;
-    const int qv2 = qt * 32 + qq;
-    if (qv2 < n_qv) {
-      f32x4 v = {ot[qq * 132 + c4], ot[qq * 132 + c4 + 1], ot[qq * 132 + c4 + 2],
-                 ot[qq * 132 + c4 + 3]};
-      *(f32x4*)(o_part + (part_base + qv2) * 128 + c4) = v;
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    if (KG > 1 && hf) __syncthreads();  // the first half has been read
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        ot[(lane & 31) * 64 + ((b * 32 + mfma_row(r, lane)) ^ ((lane & 15) << 2))] = o[2 * hf + b][r];
+    // (one group: a wave's LDS operations complete in order, it sees its own writes)
+    if (KG > 1) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4 / KG; ++i) {
+      const int qq = (lane >> 3) + 8 * (kg * (4 / KG) + i), d8 = (lane & 7) * 8, sw = (qq & 15) << 2;
+      const int qv2 = qt * 32 + qq;
+      float mq, lq;
+      f32x4 v0, v1;
+      if (KG == 1) {
+        mq = __shfl(m_run, qq, 64);
+        lq = __shfl(l_run, qq, 64);
+        v0 = *(const f32x4*)(ot + qq * 64 + (d8 ^ sw));
+        v1 = *(const f32x4*)(ot + qq * 64 + ((d8 + 4) ^ sw));
+      } else {
+        mq = -INFINITY;
+        lq = 0.f;
+        v0 = v1 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int g = 0; g < KG; ++g) mq = fmaxf(mq, ml[(g * QW + qw) * 32 + qq].x);
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+          const float2 p = ml[(g * QW + qw) * 32 + qq];
+          const float w = p.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(p.x - mq);
+          const float* og = region(g) + qq * 64;
+          lq += w * p.y;
+          v0 += w * *(const f32x4*)(og + (d8 ^ sw));
+          v1 += w * *(const f32x4*)(og + ((d8 + 4) ^ sw));
+        }
+      }
+      if (qv2 >= n_qv) continue;  // (whole groups of eight lanes)
+      if (!OUT) {
+        float* p = o_part + (part_base + qv2) * 128 + hf * 64 + d8;
+        *(f32x4*)p = v0;
+        *(f32x4*)(p + 4) = v1;
+        if (hf == 0 && (lane & 7) == 0)
+          *(float2*)(ml_part + (part_base + qv2) * 2) = make_float2(mq, lq);
+      } else {
+        const float inv = 1.f / lq;
+        const int row = qv2 / G, D = Hq * 128;
+        const int c0 = (kvh * G + qv2 - row * G) * 128 + hf * 64 + d8;
+        store_attn8(v0 * inv, v1 * inv, row, n_rows, c0, D, lane, ao);
+      }
     }
   }
-  if (lane < 32 && q_ok) {
-    ml_part[(part_base + qv) * 2 + 0] = m_run;
-    ml_part[(part_base + qv) * 2 + 1] = l_run;
-  }
-  (void)n_splits;
+}
+
+// (the buffer resource type is not known to the host pass: the body is a device function)
+template <typename T, int QW, int KG, bool LO, bool OUT>
+__global__ __launch_bounds__(64 * QW * KG, QW * KG == 2 ? 1 : KG == 1 ? 3 : QW == 4 ? 2 : 1) void attn_split_kernel(
+    const T* __restrict__ q, const T* __restrict__ q_lo, const T* __restrict__ kv,
+    int64_t kv_head_stride, int n_rows, int Hq, int Hkv, int n_keys, int row_pos0, int mask_kind,
+    int mask_prompt_len, int mask_block, int tiles_per_split, float* __restrict__ o_part,
+    float* __restrict__ ml_part, float scale, const AttnOut ao) {
+  attn_split_tile<T, QW, KG, LO, OUT>(q, q_lo, kv, kv_head_stride, n_rows, Hq, Hkv, n_keys, row_pos0,
+                                  mask_kind, mask_prompt_len, mask_block, tiles_per_split, o_part,
+                                  ml_part, scale, ao);
 }
 
 // Decode attention: rows of one mask segment (every key in [0, n_keys) is
@@ -871,45 +968,8 @@ extern "C" __global__ __launch_bounds__(256) void attn_combine_kernel(
     M = mb;
   }
   const float inv = 1.f / L;
-  float v[8];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = a0[e] * inv;
-    v[e + 4] = a1[e] * inv;
-  }
-  const int D = Hq * 128;
-  const int c0 = head * 128 + 8 * ch;  // first column of this thread's chunk
-  if (out_fmt == 0) {  // ACT_F16P: hi plane, lo plane at + n_rows * D
-    _Float16 h[8], lo[8];
-    float gs = 0.f;
-    bool over = false;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const _Float16 he = (_Float16)v[e], le = f16_lo(v[e], he);
-      h[f16p_index(e)] = he;
-      lo[f16p_index(e)] = le;
-      gs += (float)he + (float)le;
-      over = over || f16_overflows(v[e]);
-    }
-    _Float16* o = (_Float16*)out + (int64_t)row * D + c0;
-    *(u32x4*)o = __builtin_bit_cast(u32x4, h);
-    *(u32x4*)(o + (int64_t)n_rows * D) = __builtin_bit_cast(u32x4, lo);
-    if (over && err) atomicOr(err, DRT_ERR_F16_RANGE);
-    // the 64-column group sums: eight threads of aligned lanes per group
-    gs += __shfl_xor(gs, 1, 64);
-    gs += __shfl_xor(gs, 2, 64);
-    gs += __shfl_xor(gs, 4, 64);
-    if ((ch & 7) == 0) xsum[(int64_t)row * (D >> 6) + (c0 >> 6)] = gs;
-  } else if (out_fmt == 1 || out_fmt == 3) {
-    uint16_t hb[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) hb[e] = float_to_bf16_bits(v[e]);
-    *(u32x4*)((uint16_t*)out + (int64_t)row * D + c0) = __builtin_bit_cast(u32x4, hb);
-  } else {
-    float* o = (float*)out + (int64_t)row * D + c0;
-    *(f32x4*)o = f32x4{v[0], v[1], v[2], v[3]};
-    *(f32x4*)(o + 4) = f32x4{v[4], v[5], v[6], v[7]};
-  }
+  store_attn8(a0 * inv, a1 * inv, row, n_rows, head * 128 + 8 * ch, Hq * 128, (int)threadIdx.x & 63,
+              AttnOut{out, xsum, err, out_fmt});
 }
 
 // Write K/V rows (logical [n][Hkv][128] fp32 or bf16) into the tiled cache of one
@@ -975,18 +1035,6 @@ __global__ __launch_bounds__(256) void kv_pack_kernel(const void* __restrict__ k
   }
 }
 
-template __global__ void attn_split_kernel<_Float16, 2>(const _Float16*, const _Float16*, const _Float16*, int64_t,
-                                                        int, int, int, int, int, int, int, int, int,
-                                                        float*, float*, float);
-template __global__ void attn_split_kernel<_Float16, 4>(const _Float16*, const _Float16*, const _Float16*, int64_t,
-                                                        int, int, int, int, int, int, int, int, int,
-                                                        float*, float*, float);
-template __global__ void attn_split_kernel<__bf16, 2>(const __bf16*, const __bf16*, const __bf16*, int64_t, int,
-                                                      int, int, int, int, int, int, int, int,
-                                                      float*, float*, float);
-template __global__ void attn_split_kernel<__bf16, 4>(const __bf16*, const __bf16*, const __bf16*, int64_t, int,
-                                                      int, int, int, int, int, int, int, int,
-                                                      float*, float*, float);
 template __global__ void attn_decode_kernel<_Float16, 1>(const _Float16*, const _Float16*, const _Float16*,
                                                           int64_t, int, int, int, int,
                                                           const StepDesc*, float*, float*, float,
@@ -1010,24 +1058,50 @@ template __global__ void attn_decode_kernel<__bf16, 2>(const __bf16*, const __bf
                                                         float*, float, int*);
 namespace drt {
 
-AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, size_t part_budget_bytes) {
+AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, int mask_kind,
+                        size_t part_budget_bytes) {
   AttnPlan p;
   const int G = Hq / Hkv;
   const int qtiles = (n_rows * G + 31) / 32;
   p.qw = qtiles <= 2 ? 2 : 4;
   p.qgroups = (qtiles + p.qw - 1) / p.qw;
   const int n_tiles = std::max(1, (n_keys + 31) / 32);
-  // two work-groups per CU for long key ranges; one for short ones (<= 2048 keys),
-  // where a split's fixed costs (Q staging, partial stores, the combine's reads)
-  // outweigh the extra parallelism (Dream's 512-key canvas: 18.7 + 8.4 ->
-  // 18.2 + 7.0 us per layer with two splits instead of four)
-  const int target_wgs = n_tiles <= 64 ? 256 : 512;
-  int splits = std::max(1, target_wgs / (Hkv * p.qgroups));
-  splits = std::min({splits, n_tiles, 64});  // the combine reads <= 64 splits
+  // Work-groups that fill the chip: one key group each, three per CU (448 work-groups,
+  // 2048 x 2048 keys: 75 us, 84 with two key groups). Fewer: two key groups, which
+  // overlap on one CU without partials in memory (256 work-groups, 4096 keys: 75 us, 92
+  // with two splits of one group), and as many splits as pay.
+  const int wgs = Hkv * p.qgroups;
+  int splits = 1;
+  if (mask_kind == 1) {
+    // one iteration over two tiles takes about 1.1 us, a split adds the combine's 8 us
+    // and its partials' bytes (1000 x 1000 keys: 24 us unsplit, 29 with two; 100 x 4100:
+    // 68 and 23 with eight)
+    p.kg = wgs > 256 ? 1 : 2;
+    const float iters = (float)((n_tiles + 1) / 2), part_us = (float)n_rows * Hq * 1024.f / 4e6f;
+    float best = 1.1f * iters;
+    for (int sp = 2; sp <= std::min({256 / wgs, (n_tiles + 1) / 2, 64}); ++sp) {
+      const float us = 1.1f * std::ceil(iters / sp) + 8.f + part_us * sp;  // (the combine reads <= 64)
+      if (us < best) {
+        best = us;
+        splits = sp;
+      }
+    }
+    splits *= p.kg;
+  } else {
+    // every row sees every key: as many equal key ranges as fill the chip with one
+    // work-group each (two for long key ranges), neighbouring pairs of them in one
+    // work-group (the ranges, and with them the rounding of the probabilities, are
+    // those of separate work-groups)
+    splits = std::max(1, (n_tiles <= 64 ? 256 : 512) / wgs);
+    splits = std::min({splits, n_tiles, 64});
+    p.kg = splits % 2 == 0 ? 2 : 1;
+  }
   // keep the fp32 partials within budget
   const size_t per_split = (size_t)Hkv * n_rows * G * 130 * 4;
-  if (per_split > 0) splits = (int)std::max<size_t>(1, std::min<size_t>(splits, part_budget_bytes / per_split));
-  p.tiles_per_split = (n_tiles + splits - 1) / splits;
+  if (per_split > 0)
+    splits = (int)std::max<size_t>(1, std::min<size_t>(splits, p.kg * (part_budget_bytes / per_split)));
+  if (splits % p.kg) p.kg = 1;
+  p.tiles_per_split = (n_tiles + splits - 1) / splits * p.kg;
   p.splits = (n_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
   return p;
 }
@@ -1045,30 +1119,40 @@ void attention(bool bf16, const void* q, const void* kv_layer, int64_t kv_head_s
   require(Hq % Hkv == 0, "attention needs Hq % Hkv == 0");
   require(n_keys >= 1 && n_rows >= 1, "attention needs at least one query row and key");
   const float scale = 1.0f / sqrtf(128.0f);
-  const size_t lds_kv = (size_t)2 * 8192 * 2;
-  const size_t lds = std::max(lds_kv, (size_t)plan.qw * 32 * 132 * 4);
+  require((size_t)((n_keys + 31) / 32) * 16384 <= 0xFFFFFFFFu, "attention: too many keys");
   const dim3 grid(plan.splits * Hkv, plan.qgroups);
-  const dim3 block(64 * plan.qw);
+  const dim3 block(64 * plan.qw * plan.kg);
+  const AttnOut ao{out, xsum, err, out_fmt};
   // algorithmic bytes of this launch: Q read + the K/V of n_keys keys
   const double bytes = 2.0 * n_rows * Hq * 128 + 4.0 * n_keys * Hkv * 128;
-#define DRT_ATTN(T, QW)                                                                         \
+#define DRT_ATTN4(T, QW, KG, LO, OUT)                                                           \
+  DRT_LAUNCH(Profiler::ATTN, bytes, (attn_split_kernel<T, QW, KG, LO, OUT>), grid, block, 0, s, \
+             (const T*)q, LO ? (const T*)q + (int64_t)n_rows * Hq * 128 : (const T*)nullptr,    \
+             (const T*)kv_layer, kv_head_stride, n_rows, Hq, Hkv, n_keys, row_pos0, mask_kind,  \
+             mask_prompt_len, mask_block, plan.tiles_per_split, o_part, ml_part, scale, ao)
+#define DRT_ATTN3(T, QW, KG)                                                                    \
   {                                                                                             \
-    auto fn = attn_split_kernel<T, QW>;                                                         \
-    static size_t granted = 0;                                                                  \
-    grant_lds((const void*)fn, lds, granted);                                                   \
-    DRT_LAUNCH(Profiler::ATTN, bytes, fn, grid, block, lds, s, (const T*)q,                     \
-               q_has_lo ? (const T*)q + (int64_t)n_rows * Hq * 128 : (const T*)nullptr,         \
-               (const T*)kv_layer, kv_head_stride, n_rows, Hq, Hkv, n_keys, row_pos0,           \
-               mask_kind, mask_prompt_len, mask_block, plan.tiles_per_split, o_part, ml_part,   \
-               scale);                                                                          \
+    if (q_has_lo) {                                                                             \
+      if (plan.splits == 1) DRT_ATTN4(T, QW, KG, true, true);                                   \
+      else DRT_ATTN4(T, QW, KG, true, false);                                                   \
+    } else {                                                                                    \
+      if (plan.splits == 1) DRT_ATTN4(T, QW, KG, false, true);                                  \
+      else DRT_ATTN4(T, QW, KG, false, false);                                                  \
+    }                                                                                           \
   }
-  if (bf16) {
-    if (plan.qw == 2) DRT_ATTN(__bf16, 2) else DRT_ATTN(__bf16, 4)
-  } else {
-    if (plan.qw == 2) DRT_ATTN(_Float16, 2) else DRT_ATTN(_Float16, 4)
+#define DRT_ATTN(T)                                                                             \
+  {                                                                                             \
+    if (plan.qw == 2 && plan.kg == 1) DRT_ATTN3(T, 2, 1)                                        \
+    else if (plan.qw == 2) DRT_ATTN3(T, 2, 2)                                                   \
+    else if (plan.kg == 1) DRT_ATTN3(T, 4, 1)                                                   \
+    else DRT_ATTN3(T, 4, 2)                                                                     \
   }
+  if (bf16) DRT_ATTN(__bf16) else DRT_ATTN(_Float16)
 #undef DRT_ATTN
+#undef DRT_ATTN3
+#undef DRT_ATTN4
   DRT_HIP(hipGetLastError());
+  if (plan.splits == 1) return;
   const int64_t threads = (int64_t)n_rows * Hq * 16;
   hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
                      o_part, ml_part, plan.splits, n_rows, Hq, Hkv, out, xsum, out_fmt, err);

@@ -176,9 +176,10 @@ void q4_act_prep(const void* x, bool x_bf16, int M, int K, _Float16* xp, float* 
 
 // Attention over the tiled cache of one layer.
 struct AttnPlan {
-  int qw = 2, qgroups = 1, splits = 1, tiles_per_split = 1;
+  int qw = 2, kg = 2, qgroups = 1, splits = 1, tiles_per_split = 1;
 };
-AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, size_t part_budget_bytes);
+AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, int mask_kind,
+                        size_t part_budget_bytes);
 size_t attention_part_bytes(const AttnPlan& p, int n_rows, int Hq, int Hkv);
 void attention(bool bf16, const void* q, const void* kv_layer, int64_t kv_head_stride,
                int n_rows, int Hq, int Hkv, int n_keys, int row_pos0, int mask_kind,

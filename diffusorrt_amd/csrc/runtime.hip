@@ -714,7 +714,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
     ranges = p.ranges > 0 ? p.ranges : attention_decode_ranges(a.n_keys, Hkv);
     apb = attention_decode_part_bytes(ranges, Hkv, M * G);
   } else {
-    ap = plan_attention(M, Hq, Hkv, a.n_keys, rt.attn_part_budget);
+    ap = plan_attention(M, Hq, Hkv, a.n_keys, a.mask_kind, rt.attn_part_budget);
     apb = attention_part_bytes(ap, M, Hq, Hkv);
   }
   require(apb <= rt.attn_part.bytes, "attention partials exceed the workspace");
@@ -2461,8 +2461,11 @@ int32_t drt_op_kv_pack(const void* k, const void* v, int32_t src_dtype, int32_t 
 
 size_t drt_op_attention_workspace_bytes(int32_t rows, int32_t hq, int32_t hkv, int32_t n_keys) {
   if (rows <= 0 || hq <= 0 || hkv <= 0 || hq % hkv || n_keys <= 0) return 0;
-  const AttnPlan p = plan_attention(rows, hq, hkv, n_keys, (size_t)256 << 20);
-  const size_t general = attention_part_bytes(p, rows, hq, hkv);
+  size_t general = 0;  // of either mask kind
+  for (int mask = 0; mask < 2; ++mask)
+    general = std::max(general, attention_part_bytes(plan_attention(rows, hq, hkv, n_keys, mask,
+                                                                    (size_t)256 << 20),
+                                                     rows, hq, hkv));
   const size_t decode = attention_decode_part_bytes(attention_decode_ranges(n_keys, hkv), hkv, rows * (hq / hkv));
   // + the kernels' Q operand: the caller's Q as the hi plane and a zero lo plane
   const size_t q_planes = ((size_t)2 * rows * hq * 128 * 2 + 255) / 256 * 256;
@@ -2504,7 +2507,7 @@ int32_t drt_op_attention(const void* q, const void* cache, int64_t head_stride, 
                        nullptr, ranges, o_part, out, nullptr, ofmt, as_stream(stream), nullptr,
                        false);
     } else {
-      const AttnPlan p = plan_attention(rows, hq, hkv, n_keys, (size_t)256 << 20);
+      const AttnPlan p = plan_attention(rows, hq, hkv, n_keys, fa.mask_kind, (size_t)256 << 20);
       float* ml_part = o_part + (size_t)p.splits * hkv * rows * (hq / hkv) * 128;
       attention(kv_dtype == DRT_BF16, q, cache, head_stride, rows, hq, hkv, n_keys, row_pos0,
                 fa.mask_kind, mask_prompt_len, fa.mask_block, p, o_part, ml_part, out, nullptr,

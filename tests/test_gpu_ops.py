@@ -284,6 +284,14 @@ def test_block_attention_many_key_ranges(hq, hkv):
 
 
 @pytest.mark.parametrize("kind,rows,pos0,L", [("d2f_hybrid", 96, 64, 160),
+                                              # one tile, a ragged last tile, an odd tile count,
+                                              # more key tiles than a key group's share
+                                              ("d2f_hybrid", 70, 0, 70),
+                                              ("d2f_hybrid", 97, 31, 128),
+                                              ("bidirectional", 65, 0, 65),
+                                              ("d2f_hybrid", 128, 4000, 4128),
+                                              ("d2f_hybrid", 1000, 24, 1024),
+                                              ("d2f_hybrid", 2100, 0, 2100),
                                               ("d2f_hybrid", 32, 8192, 8224),
                                               ("bidirectional", 100, 0, 100)])
 def test_attention_masks_f16(kind, rows, pos0, L):
