@@ -92,21 +92,22 @@ DRT_DEV void big_bf16_tile(const FusedArgs& a, int KS, int col0, int NX) {
     const int q = wave * B_LD + i;
     b_off[i] = (((uint32_t)(q >> 2) * KC + (q & 3)) << 10) + lane * 16;
   }
-  // load d of stage gi: A first, then B (past the last stage the last one is read
-  // again, into a buffer that nothing reads: no branch between the MFMAs). Buffer
+  // load d of stage gi: A first, then B (past the last stage out of the buffers' range:
+  // zeros without a memory access, and no branch between the MFMAs). Buffer
   // instructions: the compiler counts a global_load_lds as a flat access and then
   // waits for every LDS read in flight where some of them would do.
   auto issue = [&](int gi, char* dst, int d) {
     const int gc = g_lo + min(gi, n_g - 1);
+    const uint32_t past = gi < n_g ? 0u : 0x80000000u;
     if (d < A_LD)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           a_buf, (__attribute__((address_space(3))) void*)(dst + (wave + NW * d) * 1024), 16,
-          a_off[d < A_LD ? d : 0], gc * 128, 0, 0);
+          a_off[d < A_LD ? d : 0] + past, gc * 128, 0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           b_buf,
           (__attribute__((address_space(3))) void*)(dst + A_BYTES + (wave * B_LD + d - A_LD) * 1024),
-          16, b_off[d < A_LD ? 0 : d - A_LD], gc * 4096, 0, 0);
+          16, b_off[d < A_LD ? 0 : d - A_LD] + past, gc * 4096, 0, 0);
   };
 
   f32x16 acc[TM][TN];

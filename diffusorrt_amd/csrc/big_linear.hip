@@ -6,32 +6,36 @@
 // accumulators of the weight-streaming kernels, whose two FMAs per output and
 // group would cost as much VALU time as the MFMAs.
 //
-// Work-group tile: 128 rows x 256 columns, 4 waves side by side in N; a wave
-// owns 128 x 64 (4 x 2 MFMA 32x32x16 tiles, 128 fp32 accumulators per lane).
+// A work-group of 4 waves (WVM x WVN) owns 128 rows x 256 columns (1 x 4 waves of
+// 128 x 64) or 128 x 128 (2 x 2 of 64 x 64); two work-groups per CU hide each other's
+// waits.
 //   A (the ACT_F16P activation: hi and lo planes of [M][K]) is streamed per
-//     64-k group straight into LDS (global_load_lds, no registers held),
+//     64-k group straight into LDS (buffer loads to LDS, no registers held),
 //     double buffered: 2 planes x 128 rows x 128 B per group. Rows are stored
 //     unpadded with the 16-byte chunks of row r permuted (chunk c at position
 //     c ^ (r & 7) ^ ((r >> 3) & 1)), so the MFMA fragment reads of 8 consecutive
 //     rows hit 8 different 16-byte bank groups of a 128-byte row, and those of
 //     16 consecutive rows 16 different ones of two rows (256 bytes): no bank
 //     conflict whether the LDS serves 8 or 16 lanes of a 16-byte read per
-//     cycle. Each MFMA step multiplies hi and lo by the same B.
+//     cycle. Each MFMA step multiplies hi and lo by the same B. The two buffers
+//     are separate arrays, so the compiler can tell the one being read from the
+//     one being filled and waits for no load in flight.
 //   B (q4 tile layout: per 32-column n-tile and 64-k group, 1 KiB of words and
 //     32 scale|bias pairs) goes straight from global memory to registers and is
-//     dequantized there, one k step at a time: 2 n-tiles per wave per group.
-// Group g + 1's loads are issued right after the barrier that proves group g
-// in LDS, so they stream during g's MFMAs; two work-groups per CU (<= 256
-// registers per lane) hide each other's waits.
+//     dequantized there, one k step at a time.
+// k step t + 1's fragments are read, and its B dequantized a nibble pair at a time,
+// between step t's MFMAs; so are the loads of group g + 2 issued, between the MFMAs of
+// group g's last step, once group g + 1 is proven in LDS (in one batch ahead of the
+// MFMAs the loads and the VALU work held the wave's MFMAs up).
 // Split-K over blockIdx.z (KS slices) writes fp32 partial slices y + ks * M * N
 // that a reduce pass sums (residual_norm_kernel).
 // Split last round (tail.kt >= 2, one-dimensional grid): when the tiles fill the
-// device's work-group slots (two per CU) once with a few left over, the first
-// tail.full tiles run whole and each of the remaining ones is split into tail.kt
-// K ranges on as many work-groups of one XCD, so the last round takes a fraction
-// of a tile instead of leaving most CUs idle. The slices meet as in the split-K
-// decode linears: each writes its partial tile, counts its arrival in that XCD's
-// L2, and the last to arrive adds the slices in slice order and runs the epilogue.
+// device's work-group slots (two per CU) a whole number of times with some left over,
+// the first tail.full tiles run whole and each of the remaining ones is split into
+// tail.kt K ranges on as many work-groups of one XCD, so the last round takes a
+// fraction of a tile instead of leaving most CUs idle. The slices meet as in the
+// split-K decode linears: each writes its partial tile, counts its arrival in that
+// XCD's L2, and the last to arrive adds the slices in slice order and runs the epilogue.
 // Epilogues run on 32-row pieces of the tile staged through LDS:
 //   EPI_STORE : y (+ bias on slice 0)
 //   EPI_SWIGLU: [gate 64 | up 64] column blocks -> silu(g) * u -> ACT_F16P
@@ -47,83 +51,54 @@
 
 namespace {
 
-constexpr int BG_WM = 128;                     // rows per work-group
-constexpr int BG_WN = 256;                     // columns per work-group (4 waves x 64)
-constexpr int BG_PLANE_BYTES = BG_WM * 128;    // one plane of one group: 128 rows x 64 halves
+constexpr int BG_WM = 128;                        // rows per work-group
+constexpr int BG_PLANE_BYTES = BG_WM * 128;       // one plane of one group: 128 rows x 64 halves
 constexpr int BG_BUF_BYTES = 2 * BG_PLANE_BYTES;  // hi + lo planes of one group
-constexpr int BG_EROW = BG_WN + 4;             // floats per LDS row of an epilogue piece
-constexpr int BG_V_OFF = (32 * BG_EROW * 4 + 15) / 16 * 16;  // V tile half, after the piece
-constexpr int BG_LDS = 2 * BG_BUF_BYTES;       // two group buffers (the epilogue reuses them)
-static_assert(BG_V_OFF + 4096 * 2 <= BG_LDS, "epilogue piece + V tile must fit the A buffers");
-
-template <int S> struct Slot { static constexpr int value = S; };
+// column of element c of row r in an epilogue piece (float4s permuted by row, so that
+// reads down a column and along a row both hit distinct banks)
+DRT_DEV int bg_col(int r, int c) { return c ^ ((r & 31) << 2); }
+// s_waitcnt: no vector load and no LDS read in flight
+constexpr int BG_WAIT = 0x0070;
 
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 
-// fp16 B fragment of k step t of one 64-k group of one 32-column n-tile: word t
-// of the lane holds the 8 k of the step in the ACT_F16P order (0,4,1,5,2,6,3,7);
-// nibble pairs become (1024 + q) halves by bit placement, then q * s + b in one fma.
-DRT_DEV f16x8 dequant_q4_step(uint32_t wt, uint32_t sbv) {
-  const _Float16 s = (_Float16)bf16_bits_to_float(sbv & 0xffffu);
-  const _Float16 z = (_Float16)bf16_bits_to_float(sbv >> 16);
-  const h2v s2 = {s, s}, z2 = {z, z};
+// Nibble pair e of word wt of a k step (the lane's word t of the group holds the 8 k of
+// step t in the ACT_F16P order (0,4,1,5,2,6,3,7)) as fp16 weights s * q + z: (1024 + q)
+// halves by bit placement, then q * s + z in one fma.
+DRT_DEV uint32_t dequant_q4_pair(uint32_t wt, int e, h2v s2, h2v z2, uint32_t mask) {
   const h2v k2 = {(_Float16)-1024.f, (_Float16)-1024.f};
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const h2v h = __builtin_bit_cast(h2v, ((wt >> (4 * e)) & 0x000F000Fu) | 0x64006400u);
-    o[e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(h + k2, s2, z2));
-  }
-  return __builtin_bit_cast(f16x8, o);
-}
-
-// dequant_q4_step with the group's scale and bias already in fp16 pairs and
-// the nibble mask in a register (one v_and_or_b32 per nibble pair)
-DRT_DEV f16x8 dequant_q4_step_sz(uint32_t wt, h2v s2, h2v z2, uint32_t mask) {
-  const h2v k2 = {(_Float16)-1024.f, (_Float16)-1024.f};
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const h2v h = __builtin_bit_cast(h2v, ((wt >> (4 * e)) & mask) | 0x64006400u);
-    o[e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(h + k2, s2, z2));
-  }
-  return __builtin_bit_cast(f16x8, o);
-}
-
-// LDS fragment read the compiler does not see: a plain read after a
-// direct-to-LDS load makes it wait for every global load in flight first
-// (it cannot tell the group being read from the one being filled).
-DRT_DEV void lds_read16(f16x8& v, uint32_t addr) {
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr));
-}
-// ... at a constant byte offset from addr (the instruction's offset field)
-template <int OFF>
-DRT_DEV void lds_read16o(f16x8& v, uint32_t addr) {
-  static_assert(OFF >= 0 && OFF < 65536, "ds_read offset field");
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(OFF));
+  const h2v h = __builtin_bit_cast(h2v, ((wt >> (4 * e)) & mask) | 0x64006400u);
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(h + k2, s2, z2));
 }
 
 }  // namespace
 
 struct BgTail {
   int full = 0;            // whole tiles (the first work-groups, dealt in XCD runs)
+  int rest = 0;            // remaining tiles
   int kt = 0;              // K slices per remaining tile (0: the three-dimensional grid)
-  float* part = nullptr;   // [remaining tiles][kt][128 * 256] partial tiles
+  float* part = nullptr;   // [remaining tiles][kt][rows * columns of a tile] partial tiles
   int* count = nullptr;    // [remaining tiles] arrival counters, zero on entry and exit
 };
-constexpr int BG_TAIL_KT_MAX = 8;
+using drt::BG_TAIL_KT_MAX;
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int KS, const BgTail tail) {
+template <int EPI, int TM, int TN, int WVM, int WVN>
+DRT_DEV void big_q4_tile(const FusedArgs& a, int KS, const BgTail& tail) {
+  constexpr int BN = 32 * TN * WVN;
+  static_assert(WVM * WVN == 4 && 32 * TM * WVM == BG_WM && TN == 2, "four waves over 128 rows");
+  static_assert(WVM * 32 * BN * 4 == BG_BUF_BYTES, "an epilogue piece fills a buffer");
+  __shared__ __align__(1024) char buf0[BG_BUF_BYTES];
+  __shared__ __align__(1024) char buf1[BG_BUF_BYTES];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: LDS bases in SGPRs
+  const int wm = wave / WVN, wn = wave % WVN;
   const int M = a.M, N = a.N, K = a.K, G = K >> 6;
   // Tiles t = y + MT (x + NX z) (row tile y fastest), dealt to the XCDs in
   // contiguous runs: work-group b runs on XCD b % 8 and takes tile
   // (b % 8) * T8 / 8 + b / 8 (the last T - T8 tiles as they come), so an XCD's
   // L2 holds whole columns of row tiles: each weight tile is fetched by one XCD,
   // and a K slice of a split-K grid whose tiles fill an XCD's run stays on it.
-  const int MT = (M + BG_WM - 1) / BG_WM, NX = (N + BG_WN - 1) / BG_WN;
+  const int MT = (M + BG_WM - 1) / BG_WM, NX = (N + BN - 1) / BN;
   auto xcd_run = [](int b, int T) {
     const int T8 = T & ~7;
     return b < T8 ? (b & 7) * (T8 >> 3) + (b >> 3) : b;
@@ -136,7 +111,8 @@ __global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int K
     tile_x = (t / MT) % NX;
     ks = t / (MT * NX);
   }
-  if (EPI == EPI_SWIGLU && tail.kt) {
+  constexpr bool TAIL = EPI == EPI_SWIGLU || EPI == EPI_STORE;
+  if (TAIL && tail.kt) {
     // work-group b: tile b (the first full tiles in XCD runs), or K slice of a
     // remaining tile; the slices of one remaining tile share b % 8, i.e. one
     // XCD (full % 8 == 0)
@@ -157,186 +133,197 @@ __global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int K
         if (xcc != (b & 7))
           __hip_atomic_fetch_or(a.placement_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      if (tail_idx >= tail.rest) return;  // padding of the last eight tiles
     }
     tile_y = t % MT;
     tile_x = t / MT;
   }
-  const int n0 = tile_x * BG_WN, m0 = tile_y * BG_WM;
+  const int n0 = tile_x * BN, m0 = tile_y * BG_WM;
   const int g_lo = (int)((int64_t)G * ks / KS), g_hi = (int)((int64_t)G * (ks + 1) / KS);
   const int n_g = g_hi - g_lo;
   const int NT = N >> 5;
   // this wave's two n-tiles, clamped so that loads stay in bounds (columns
   // beyond N are computed from the last n-tile and never stored)
-  const int nt0 = min((n0 >> 5) + 2 * wave, NT - 1);
-  const int nt1 = min((n0 >> 5) + 2 * wave + 1, NT - 1);
-  extern __shared__ __align__(16) char smem[];
-  const _Float16* act = (const _Float16*)a.act;
+  const int nt0 = min((n0 >> 5) + TN * wn, NT - 1);
+  const int nt1 = min((n0 >> 5) + TN * wn + 1, NT - 1);
 
-  u32x4 wq[2][2];
-  uint32_t wsb[2][2];
-  // A of group g into buffer buf: plane pl, 8-row block blk = wave + 4i is one
-  // wave instruction (lane l: row blk*8 + (l >> 3), LDS position l & 7, which
-  // holds the row's chunk (l & 7) ^ (l >> 3) ^ (blk & 1), blk & 1 being
-  // wave & 1); rows past M re-read row M - 1,
-  // whose copies feed only outputs that are never stored. Addresses are a
-  // uniform base per group plus 32-bit lane offsets (activation < 4 GiB),
-  // recomputed at each issue (24-bit multiplies, from lane values made opaque
-  // there) instead of staying live across the loop.
-  const int row_l = m0 + wave * 8 + (lane >> 3);
-  const uint32_t col_l = (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (wave & 1)) * 16);
+  // A of a group: plane pl, 8-row block blk = wave + 4 i is one wave instruction
+  // (lane l: row blk * 8 + (l >> 3), LDS position l & 7, which holds the row's chunk
+  // (l & 7) ^ (l >> 3) ^ (blk & 1), blk & 1 being wave & 1), from a buffer per plane
+  // that ends with row M - 1: rows past it read zeros.
   const uint32_t K2 = (uint32_t)K * 2u;
-  const char* act_b = (const char*)act;
-  auto issue = [&](int g, int buf, auto slot) {
-    constexpr int S = decltype(slot)::value;
-    const char* ag = act_b + (size_t)g * 128;
-    int rl = row_l;
-    uint32_t cl = col_l;
-    asm volatile("" : "+v"(rl), "+v"(cl));
-#pragma unroll
-    for (int pl = 0; pl < 2; ++pl)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t m = (uint32_t)(min(rl + 32 * i, M - 1) + pl * M);
-        char* dst = smem + buf * BG_BUF_BYTES + pl * BG_PLANE_BYTES + (wave + 4 * i) * 1024;
-        __builtin_amdgcn_global_load_lds(
-            (__attribute__((address_space(1))) void*)(ag + (__umul24(m, K2) + cl)),
-            (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-      }
-    wq[S][0] = *q4_tile_words(a.qw, nt0, G, g, lane);
-    wq[S][1] = *q4_tile_words(a.qw, nt1, G, g, lane);
-    wsb[S][0] = q4_tile_sb(a.sb, nt0, G, g, lane);
-    wsb[S][1] = q4_tile_sb(a.sb, nt1, G, g, lane);
+  const uint32_t rows_bytes = (uint32_t)min(BG_WM, M - m0) * K2;
+  const char* act = (const char*)a.act + (size_t)m0 * K2;
+  const __amdgpu_buffer_rsrc_t hi_buf =
+      __builtin_amdgcn_make_buffer_rsrc((void*)act, 0, rows_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t lo_buf =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(act + (size_t)M * K2), 0, rows_bytes, 0x00020000);
+  const uint32_t a_off = (uint32_t)(wave * 8 + (lane >> 3)) * K2 +
+                         (uint32_t)(((lane & 7) ^ (lane >> 3) ^ (wave & 1)) * 16);
+  // load d (0 .. 7: block d & 3 of plane d >> 2) of group gi (past the last one out of
+  // the buffer's range: zeros without a memory access, and no branch between the MFMAs)
+  auto issue_a = [&](int gi, char* dst, int d) {
+    const int i = d & 3, pl = d >> 2;
+    const uint32_t past = gi < n_g ? 0u : 0x80000000u;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        pl ? lo_buf : hi_buf,
+        (__attribute__((address_space(3))) void*)(dst + pl * BG_PLANE_BYTES + (wave + 4 * i) * 1024),
+        16, a_off + ((uint32_t)(32 * i) * K2 + past), (g_lo + min(gi, n_g - 1)) * 128, 0, 0);
+  };
+  u32x4 wq[2][TN];
+  uint32_t wsb[2][TN];
+  auto issue_b = [&](int gi, int slot) {
+    const int g = g_lo + min(gi, n_g - 1);
+    wq[slot][0] = *q4_tile_words(a.qw, nt0, G, g, lane);
+    wq[slot][1] = *q4_tile_words(a.qw, nt1, G, g, lane);
+    wsb[slot][0] = q4_tile_sb(a.sb, nt0, G, g, lane);
+    wsb[slot][1] = q4_tile_sb(a.sb, nt1, G, g, lane);
   };
 
-  f32x16 acc[4][2];
+  f32x16 acc[TM][TN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i][0] = acc[i][1] = f32x16{};
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
 
-  // this lane's fragment row within each 32-row m-tile is lane & 31; its k
-  // chunk at step t is 4 * (lane >> 5) + t, stored at position
-  // chunk ^ (row & 7) ^ ((row >> 3) & 1) (row & 15 == lane & 15)
-  const uint32_t lds0 = (uint32_t)(uintptr_t)smem + (lane & 31) * 128;
-  // one k step's operands (A hi and lo fragments, the two dequantised B
-  // fragments); steps alternate between two sets, the next step's read and
-  // dequantised while the current step's MFMAs run
+  // one k step's operands (A hi and lo fragments, the dequantised B fragments); steps
+  // alternate between two sets
   struct Ops {
-    f16x8 h[4], l[4], b[2];
+    f16x8 h[TM], l[TM];
+    u32x4 b[TN];
   };
   uint32_t nib_mask = 0x000F000Fu;
   asm volatile("" : "+v"(nib_mask));  // in a register: v_and_or_b32 takes one constant
-  h2v gs2[2], gz2[2];                // the current group's scale and bias pairs
-  auto group_scales = [&](auto slot) {
-    constexpr int S = decltype(slot)::value;
+  h2v gs2[TN], gz2[TN];               // the current group's scale and bias pairs
+  auto group_scales = [&](int slot) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const _Float16 sc = (_Float16)bf16_bits_to_float(wsb[S][j] & 0xffffu);
-      const _Float16 zb = (_Float16)bf16_bits_to_float(wsb[S][j] >> 16);
+    for (int j = 0; j < TN; ++j) {
+      const _Float16 sc = (_Float16)bf16_bits_to_float(wsb[slot][j] & 0xffffu);
+      const _Float16 zb = (_Float16)bf16_bits_to_float(wsb[slot][j] >> 16);
       gs2[j] = h2v{sc, sc};
       gz2[j] = h2v{zb, zb};
     }
   };
-  auto load_ops = [&](Ops& o, int buf, int t, auto slot) {
-    constexpr int S = decltype(slot)::value;
-    // m-tile i of the hi plane at + 4096 i, of the lo plane at + BG_PLANE_BYTES + 4096 i
-    const uint32_t ab =
-        lds0 + buf * BG_BUF_BYTES +
-        (uint32_t)(((4 * (lane >> 5) + t) ^ (lane & 7) ^ ((lane >> 3) & 1)) * 16);
-    lds_read16o<0>(o.h[0], ab);
-    lds_read16o<BG_PLANE_BYTES>(o.l[0], ab);
-    lds_read16o<4096>(o.h[1], ab);
-    lds_read16o<BG_PLANE_BYTES + 4096>(o.l[1], ab);
-    lds_read16o<8192>(o.h[2], ab);
-    lds_read16o<BG_PLANE_BYTES + 8192>(o.l[2], ab);
-    lds_read16o<12288>(o.h[3], ab);
-    lds_read16o<BG_PLANE_BYTES + 12288>(o.l[3], ab);
+  // this lane's fragment row within each 32-row m-tile is lane & 31; its k chunk at
+  // step t is 4 * (lane >> 5) + t
+  const uint32_t a_row = (uint32_t)(wm * TM * 4096 + (lane & 31) * 128);
+  const uint32_t a_swz = (uint32_t)((lane & 7) ^ ((lane >> 3) & 1));
+  auto load_h = [&](Ops& o, const char* src, int t) {
+    const char* p = src + a_row + (((uint32_t)(4 * (lane >> 5) + t) ^ a_swz) * 16);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) o.b[j] = dequant_q4_step_sz(wq[S][j][t], gs2[j], gz2[j], nib_mask);
+    for (int i = 0; i < TM; ++i) o.h[i] = *(const f16x8*)(p + i * 4096);
   };
-  auto lds_wait = [](Ops& o) {
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(o.h[0]), "+v"(o.h[1]), "+v"(o.h[2]), "+v"(o.h[3]), "+v"(o.l[0]),
-                   "+v"(o.l[1]), "+v"(o.l[2]), "+v"(o.l[3]));
+  auto load_l = [&](Ops& o, const char* src, int t) {
+    const char* p = src + a_row + (((uint32_t)(4 * (lane >> 5) + t) ^ a_swz) * 16);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) o.l[i] = *(const f16x8*)(p + BG_PLANE_BYTES + i * 4096);
   };
   Ops X, Y;
-  if (n_g > 0) {
-    issue(g_lo, 0, Slot<0>{});
-    if (n_g > 1) issue(g_lo + 1, 1, Slot<1>{});
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();                     // group g_lo is in LDS in every wave
-    group_scales(Slot<0>{});
-    load_ops(X, 0, 0, Slot<0>{});
-    lds_wait(X);
-  }
-  // k step t of group gi (buffer and B slot S = gi & 1) on `cur`, the next
-  // step's operands into `nxt`; at the last step, once group gi + 1 is in LDS
-  // in every wave (and every wave is done with buffer S), group gi + 2 is
-  // issued into buffer and slot S
-  auto kstep = [&](Ops& cur, Ops& nxt, int gi, int t, auto slot) {
-    constexpr int S = decltype(slot)::value;
-    bool more = true;
+#pragma unroll
+  for (int d = 0; d < 8; ++d) issue_a(0, buf0, d);
+  issue_b(0, 0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int d = 0; d < 8; ++d) issue_a(1, buf1, d);
+  issue_b(1, 1);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (8 + 2 * TN));  // group 0 has arrived
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  group_scales(0);
+  load_h(X, buf0, 0);
+  load_l(X, buf0, 0);
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) X.b[j][e] = dequant_q4_pair(wq[0][j][0], e, gs2[j], gz2[j], nib_mask);
+  // k step t of group gi (in `here`, B slot S = gi & 1) on `cur`, the next step's
+  // operands into `nxt`; at the last step, once group gi + 1 is in LDS in every wave and
+  // this wave's reads of `here` are done, group gi + 2 goes into `here` and slot S (past
+  // the last group the operands read are unused)
+  auto kstep = [&](Ops& cur, Ops& nxt, int gi, int t, auto slot, char* here, char* there) {
+    constexpr int S = decltype(slot)::value, SN = 2 * TM;  // MFMA rows: hi, then lo
     if (t < 3) {
-      load_ops(nxt, S, t + 1, Slot<S>{});
-    } else if (gi + 1 < n_g) {
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-      __syncthreads();
-      if (gi + 2 < n_g) issue(g_lo + gi + 2, S, Slot<S>{});
-      group_scales(Slot<S ^ 1>{});
-      load_ops(nxt, S ^ 1, 0, Slot<S ^ 1>{});
+      load_h(nxt, here, t + 1);
     } else {
-      more = false;
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(BG_WAIT);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      load_h(nxt, there, 0);
+      group_scales(S ^ 1);
+      if (gi + 2 < n_g) issue_b(gi + 2, S);
     }
-    // the hi products of the step, then the lo ones (a tile's two MFMAs eight apart)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[i][0] = mfma_f16(cur.h[i], cur.b[0], acc[i][0]);
-      acc[i][1] = mfma_f16(cur.h[i], cur.b[1], acc[i][1]);
-    }
+    for (int s = 0; s < SN; ++s) {
+      const int i = s % TM;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[i][0] = mfma_f16(cur.l[i], cur.b[0], acc[i][0]);
-      acc[i][1] = mfma_f16(cur.l[i], cur.b[1], acc[i][1]);
+      for (int j = 0; j < TN; ++j)
+        acc[i][j] = mfma_f16(s < TM ? cur.h[i] : cur.l[i], __builtin_bit_cast(f16x8, cur.b[j]), acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+      // (the lo fragments once the current hi ones are spent: 16 registers fewer)
+      if (s == TM - 1) load_l(nxt, t < 3 ? here : there, (t + 1) & 3);
+#pragma unroll
+      for (int q = 0; q < 4 * TN / SN; ++q) {
+        const int p = s * (4 * TN / SN) + q, j = p >> 2, e = p & 3;
+        nxt.b[j][e] = dequant_q4_pair(t < 3 ? wq[S][j][t < 3 ? t + 1 : 0] : wq[S ^ 1][j][0], e, gs2[j],
+                                      gz2[j], nib_mask);
+      }
+      if (t == 3) {
+#pragma unroll
+        for (int q = 0; q < 8 / SN; ++q) issue_a(gi + 2, here, s * (8 / SN) + q);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (more) lds_wait(nxt);
   };
-  auto group = [&](int gi, auto slot) {
-    kstep(X, Y, gi, 0, slot);
-    kstep(Y, X, gi, 1, slot);
-    kstep(X, Y, gi, 2, slot);
-    kstep(Y, X, gi, 3, slot);
+  auto group = [&](int gi, auto slot, char* here, char* there) {
+    kstep(X, Y, gi, 0, slot, here, there);
+    kstep(Y, X, gi, 1, slot, here, there);
+    kstep(X, Y, gi, 2, slot, here, there);
+    kstep(Y, X, gi, 3, slot, here, there);
   };
-  for (int gb = 0; gb < n_g; gb += 2) {
-    group(gb, Slot<0>{});
-    if (gb + 1 < n_g) group(gb + 1, Slot<1>{});
+  int g = 0;
+  for (; g + 1 < n_g; g += 2) {
+    group(g, std::integral_constant<int, 0>{}, buf0, buf1);
+    group(g + 1, std::integral_constant<int, 1>{}, buf1, buf0);
   }
-  if (EPI == EPI_SWIGLU && tail_idx >= 0) {  // (the split last round is used for gate|up)
+  if (g < n_g) group(g, std::integral_constant<int, 0>{}, buf0, buf1);
+  __builtin_amdgcn_s_waitcnt(BG_WAIT);  // the epilogue reuses the buffers
+  // (the thread index made opaque: the epilogue's addresses are not computed ahead of
+  // the main loop and kept, or spilled, across it)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+
+  if (TAIL && tail_idx >= 0) {
     // a K slice of a remaining tile: store it as 16-byte chunks (chunk c = four
     // consecutive accumulators of thread t at (c * 256 + t) * 4), and let the
     // last slice to arrive add them all in slice order, two chunks of every
     // slice in flight at a time
-    constexpr int TILE = BG_WM * BG_WN;
+    constexpr int TILE = BG_WM * BN;
     float* pt = tail.part + (size_t)tail_idx * tail.kt * TILE;
-    f32x4* mine = (f32x4*)(pt + (size_t)ks * TILE) + threadIdx.x;
+    f32x4* mine = (f32x4*)(pt + (size_t)ks * TILE) + tid;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          mine[((i * 2 + j) * 4 + q) * 256] =
+          mine[((i * TN + j) * 4 + q) * 256] =
               f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
     __shared__ int last_flag;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();  // every store of the work-group is in this XCD's L2
-    if (threadIdx.x == 0)
+    if (tid == 0)
       last_flag = __hip_atomic_fetch_add(&tail.count[tail_idx], 1, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_WORKGROUP) == tail.kt - 1;
     __syncthreads();
     if (!last_flag) return;
-    const f32x4* pv = (const f32x4*)pt + threadIdx.x;
+    const f32x4* pv = (const f32x4*)pt + tid;
 #pragma unroll
-    for (int c0 = 0; c0 < 32; c0 += 2) {
+    for (int c0 = 0; c0 < 4 * TM * TN; c0 += 2) {
       f32x4 v[2][BG_TAIL_KT_MAX];
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc)
@@ -345,7 +332,7 @@ __global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int K
           v[cc][k] = pv[(size_t)min(k, tail.kt - 1) * (TILE / 4) + (c0 + cc) * 256];
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
-        const int c = c0 + cc, i = c >> 3, j = (c >> 2) & 1, q = c & 3;
+        const int c = c0 + cc, i = c / (4 * TN), j = (c >> 2) % TN, q = c & 3;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float sum = 0.f;
@@ -356,37 +343,40 @@ __global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int K
         }
       }
     }
-    if (threadIdx.x == 0) tail.count[tail_idx] = 0;
+    if (tid == 0) tail.count[tail_idx] = 0;
+    ks = 0;
   }
-  __syncthreads();  // every wave's last fragment reads are done: the epilogue reuses the LDS
 
-  // Epilogue in 32-row pieces (MFMA m-tile p of every wave) through LDS.
-  float* e = (float*)smem;  // [32][BG_EROW]
-  uint16_t* vbuf = (uint16_t*)(smem + BG_V_OFF);
+  // Epilogue through LDS in pieces: MFMA row tile p of every wave, 32 rows per wave row.
+  float* e = (float*)buf0;  // [32 * WVM][BN]
+  uint16_t* vbuf = (uint16_t*)buf1;
   const int row0 = a.desc ? a.desc->row0 : 0;
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int mp = m0 + 32 * p;  // forward row of local row 0
-    if (mp >= M) break;          // uniform
+  for (int p = 0; p < TM; ++p) {
+    if (m0 + 32 * p >= M) break;  // uniform
+    __syncthreads();  // the last fragment reads, then the previous piece's, are done
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        e[mfma_row(r, lane) * BG_EROW + wave * 64 + j * 32 + (lane & 31)] = acc[p][j][r];
+      for (int r = 0; r < 16; ++r) {
+        const int rr = mfma_row(r, tid & 63);
+        e[(wm * 32 + rr) * BN + bg_col(rr, (wn * TN + j) * 32 + (tid & 31))] = acc[p][j][r];
+      }
     __syncthreads();
+    auto row_of = [&](int rr) { return m0 + ((rr >> 5) * TM + p) * 32 + (rr & 31); };
     if (EPI == EPI_STORE) {
       float* y = a.y + (int64_t)ks * M * N;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int c = threadIdx.x + 256 * i;
-        const int r = c >> 6, n = n0 + (c & 63) * 4;
-        if (mp + r < M && n < N) {
-          f32x4 v = *(const f32x4*)(e + r * BG_EROW + (c & 63) * 4);
+        const int c = tid + 256 * i;
+        const int rr = c / (BN / 4), cc = c % (BN / 4) * 4, n = n0 + cc, m = row_of(rr);
+        if (m < M && n < N) {
+          f32x4 v = *(const f32x4*)(e + rr * BN + bg_col(rr, cc));
           if (a.bias && ks == 0) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] += bf16_bits_to_float(a.bias[n + k]);
           }
-          *(f32x4*)(y + (int64_t)(mp + r) * N + n) = v;
+          *(f32x4*)(y + (int64_t)m * N + n) = v;
         }
       }
     } else if (EPI == EPI_SWIGLU) {
@@ -396,41 +386,51 @@ __global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int K
       bool over = false;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const int c = threadIdx.x + 256 * i;
-        const int r = c >> 4, q = c & 15, blk = q >> 3, c8 = (q & 7) * 8;
-        if (mp + r < M && n0 + blk * 128 < N) {
+        const int c = tid + 256 * i;
+        const int rr = c / (BN / 16), q = c % (BN / 16), blk = q >> 3, c8 = (q & 7) * 8;
+        const int m = row_of(rr);
+        if (m < M && n0 + blk * 128 < N) {
+          const float* er = e + rr * BN;
+          float gv[8], uv[8];
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const f32x4 g4 = *(const f32x4*)(er + bg_col(rr, blk * 128 + c8 + 4 * hf));
+            const f32x4 u4 = *(const f32x4*)(er + bg_col(rr, blk * 128 + 64 + c8 + 4 * hf));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              gv[4 * hf + k] = g4[k];
+              uv[4 * hf + k] = u4[k];
+            }
+          }
           _Float16 h[8], lo[8];
 #pragma unroll
           for (int k = 0; k < 8; ++k) {
-            const float g = e[r * BG_EROW + blk * 128 + c8 + k];
-            const float u = e[r * BG_EROW + blk * 128 + 64 + c8 + k];
-            const float y = g * (1.f / (1.f + expf(-g))) * u;
+            const float y = gv[k] * (1.f / (1.f + expf(-gv[k]))) * uv[k];
             const _Float16 hk = (_Float16)y;
             h[f16p_index(k)] = hk;
             lo[f16p_index(k)] = f16_lo(y, hk);
             over = over || f16_overflows(y);
           }
-          _Float16* dst = (_Float16*)a.act_out + (int64_t)(mp + r) * F + (n0 >> 1) + blk * 64 + c8;
+          _Float16* dst = (_Float16*)a.act_out + (int64_t)m * F + (n0 >> 1) + blk * 64 + c8;
           *(u32x4*)dst = __builtin_bit_cast(u32x4, h);
           *(u32x4*)(dst + (int64_t)M * F) = __builtin_bit_cast(u32x4, lo);
         }
       }
       if (over) raise_range(a);
     } else if (EPI == EPI_LMSTAT) {
-      // lane: row lane & 31 of the piece, the 32 columns half of its wave's 64
-      // (the rows of 8 consecutive lanes sit in 8 different 16-byte bank groups)
-      const int r = lane & 31, half = lane >> 5;
-      const int col0 = n0 + wave * 64 + half * 32, row = mp + r;
-      const bool valid = row < M && n0 + wave * 64 < N;  // (N % 64 == 0)
+      // lane: row lane & 31 of its wave's piece, the 32 columns half of its wave's 64
+      const int r = tid & 31, half = (tid >> 5) & 1;
+      const int col0 = n0 + wn * 64 + half * 32, row = m0 + (wm * TM + p) * 32 + r;
+      const bool valid = row < M && n0 + wn * 64 < N;  // (N % 64 == 0)
       const float temperature = a.desc ? a.desc->temperature : a.lm_temp;
       const uint64_t seed = a.desc ? a.desc->seed : a.lm_seed;
       const int step = a.desc ? a.desc->step : a.lm_step;
       const int excl = a.desc ? a.desc->exclude_col : a.lm_excl;
       float v[32];
-      const float* src = e + r * BG_EROW + wave * 64 + half * 32;
+      const float* src = e + (wm * 32 + r) * BN;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const f32x4 t4 = *(const f32x4*)(src + 4 * q);
+        const f32x4 t4 = *(const f32x4*)(src + bg_col(r, wn * 64 + half * 32 + 4 * q));
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[4 * q + k] = t4[k];
       }
@@ -452,28 +452,33 @@ __global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int K
       other.sarg = __shfl_xor(mine.sarg, 32, 64);
       other.sl = __shfl_xor(mine.sl, 32, 64);
       if (half == 0 && valid)
-        ((LmStat*)a.lm_stats)[(int64_t)row * (N >> 6) + (n0 >> 6) + wave] = lm_join64(mine, other);
+        ((LmStat*)a.lm_stats)[(int64_t)row * (N >> 6) + (n0 >> 6) + wn] = lm_join64(mine, other);
     } else if (EPI == EPI_QKV) {
-      const int rows = min(32, M - mp);
 #pragma unroll
-      for (int hl = 0; hl < 2; ++hl) {
-        const int head = (n0 >> 7) + hl;
-        if (head * 128 >= N) break;  // uniform
-        if (hl) __syncthreads();     // the V tile buffer of head 0 has been copied out
-        auto get = [&](int m, int d) { return e[m * BG_EROW + hl * 128 + d]; };
-        const QkvTables qt = qkv_tables(a, head, row0 + mp, rows);
-        if (a.kv_bf16) qkv_epilogue<__bf16>(a, qt, head, mp, row0 + mp, rows, get, vbuf);
-        else qkv_epilogue<_Float16>(a, qt, head, mp, row0 + mp, rows, get, vbuf);
+      for (int w = 0; w < WVM; ++w) {
+        const int mp = m0 + (w * TM + p) * 32;
+        if (mp >= M) break;  // uniform
+        const int rows = min(32, M - mp);
+#pragma unroll
+        for (int hl = 0; hl < BN / 128; ++hl) {
+          const int head = (n0 >> 7) + hl;
+          if (head * 128 >= N) break;    // uniform
+          if (w || hl) __syncthreads();  // the V tile buffer of the last head has been copied out
+          auto get = [&](int m, int d) { return e[(w * 32 + m) * BN + bg_col(m, hl * 128 + d)]; };
+          const QkvTables qt = qkv_tables(a, head, row0 + mp, rows);
+          if (a.kv_bf16) qkv_epilogue<__bf16>(a, qt, head, mp, row0 + mp, rows, get, vbuf);
+          else qkv_epilogue<_Float16>(a, qt, head, mp, row0 + mp, rows, get, vbuf);
+        }
       }
     }
-    __syncthreads();  // the piece's LDS is read before the next piece is written
   }
 }
 
-template __global__ void big_q4_kernel<EPI_STORE>(const FusedArgs, int, const BgTail);
-template __global__ void big_q4_kernel<EPI_SWIGLU>(const FusedArgs, int, const BgTail);
-template __global__ void big_q4_kernel<EPI_QKV>(const FusedArgs, int, const BgTail);
-template __global__ void big_q4_kernel<EPI_LMSTAT>(const FusedArgs, int, const BgTail);
+// (the buffer resource type is not known to the host pass: the body is a device function)
+template <int EPI, int TM, int TN, int WVM, int WVN>
+__global__ __launch_bounds__(256, 2) void big_q4_kernel(const FusedArgs a, int KS, const BgTail tail) {
+  big_q4_tile<EPI, TM, TN, WVM, WVN>(a, KS, tail);
+}
 
 // The QKV epilogue of a split-K q|k|v projection: work-group (head, 32-row
 // block) sums the KS fp32 partial slices of its head's 128 columns (bias
@@ -550,18 +555,77 @@ template __global__ void big_qkv_epilogue_kernel<__bf16>(const FusedArgs, const 
 
 namespace drt {
 
-// K slices for a large-M q4 linear of M x N x K: enough work-groups for two per
-// CU (the kernel's register budget), at most max_ks slices and at least 8 groups
-// of 64 k per slice.
+// K slices the workspaces of a large-M q4 linear are sized for: enough work-groups for
+// two per CU, at most max_ks and at least 6 groups of 64 k each.
 int big_linear_splits(int M, int N, int K, int max_ks) {
-  const int tiles = ((M + BG_WM - 1) / BG_WM) * ((N + BG_WN - 1) / BG_WN);
+  const int tiles = ((M + BG_WM - 1) / BG_WM) * ((N + 255) / 256);
   if (tiles >= 384) return 1;
-  // the most slices that keep the grid within one round of two work-groups per
-  // CU (512 slots on 256 CUs: a CU holding two work-groups while others hold one
-  // sets the time), each slice at least 6 groups of 64 k
   int ks = std::min(max_ks, std::max(1, 512 / tiles));
   ks = std::min(ks, std::max(1, (K / 64) / 6));
   return std::max(1, ks);
+}
+
+namespace {
+// Estimated us of n work-groups of g groups of 64 k. Measured us per group for a few
+// work-groups (the loads' latency), for one per CU, for a few CUs with two (the others
+// wait for them) and for two on every CU: 128 x 256 tiles 1.22 / 1.70 / 2.55 / 3.35, 128 x
+// 128 tiles 0.85 / 1.00 / 1.45 / 1.95; and about 4 us to start and store a round.
+float bg_cost(bool wide, int n, float g, int n_cu) {
+  const float few = wide ? 1.22f : 0.85f, one = wide ? 1.70f : 1.00f;
+  const float over = wide ? 2.55f : 1.45f, two = wide ? 3.35f : 1.95f;
+  const int rounds = n / (2 * n_cu), rest = n - rounds * 2 * n_cu;
+  float us = rounds * (two * g + 4.f);
+  if (rest > n_cu) us += (over + (two - over) * (rest - n_cu) / n_cu) * g + 4.f;
+  else if (rest > 0) us += (few + (one - few) * rest / n_cu) * g + 4.f;
+  return us;
+}
+}  // namespace
+
+// The cheapest estimate over the two tiles and, for plain stores, the K slices (each at
+// least four groups; reduce_us: what the reduce pass costs besides its bytes), and for
+// unsplit stores and gate|up the split last round: the tiles past whole rounds of one
+// or two work-groups per CU over at most one K slice per CU. part_floats bounds the
+// slices and the split tiles' partials. Measured (hi + lo MFMA rates in brackets):
+// 512 x 18944 x 3584, 296 wide tiles: 155 us as they are, 156 as 592 narrow ones, 119
+// with the last 40 tiles in six slices (1165 TFLOP/s); 512 x 37888 x 3584: 294 and 232 (80
+// tiles in three slices; 246 in six, the last slice's adding outweighing the shorter
+// round); 41 x 18944 x 3584: 73 unsplit, 32 in three slices; 2048 x 1024 x 1024: 21 us in
+// two slices of wide tiles (+ 5 to add them), 21 unsplit narrow.
+BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+                      float reduce_us, bool tail_ok) {
+  const int n_cu = n_cu_of_current_device(), G = K / 64, MT = (M + BG_WM - 1) / BG_WM;
+  BigQ4Plan best;
+  float best_us = 1e30f;
+  auto take = [&](float us, const BigQ4Plan& p) {
+    if (us < best_us) {
+      best_us = us;
+      best = p;
+    }
+  };
+  for (int w = 1; w >= 0; --w) {
+    const bool wide = w == 1;
+    const int bn = wide ? 256 : 128, T = MT * ((N + bn - 1) / bn);
+    for (int ks = 1; ks <= max_ks; ++ks) {
+      if (ks > 1 && (kind != FL_STORE || G / ks < 4 || (size_t)ks * M * N > part_floats)) break;
+      float us = bg_cost(wide, T * ks, (float)((G + ks - 1) / ks), n_cu);
+      if (ks > 1) us += reduce_us + (2 * ks + 1) * 0.5e-6f * M * N;  // 4 bytes each at 8 TB/s
+      take(us, BigQ4Plan{wide, ks, 0, 0});
+    }
+    if (!tail_ok || (kind != FL_STORE && kind != FL_SWIGLU)) continue;
+    for (int unit = 1; unit <= 2; ++unit) {
+      const int full = T / (unit * n_cu) * (unit * n_cu), rest = T - full;
+      if (rest == 0 || rest > BIG_TAIL_COUNTERS || full % 8) continue;
+      const int kt = std::min({BG_TAIL_KT_MAX, n_cu / rest, G / 2});
+      if (kt < 2 || (size_t)rest * kt * BG_WM * bn > part_floats) continue;
+      const float whole = bg_cost(wide, full, (float)G, n_cu);
+      // an odd round of one per CU leaves the slices the second slots
+      const bool beside = full % (2 * n_cu) != 0;
+      const float us = beside ? whole + bg_cost(wide, rest * kt, (float)G / kt, n_cu) * 0.2f + 5.f
+                              : whole + bg_cost(wide, rest * kt, (float)G / kt, n_cu) + 4.f;
+      take(us, BigQ4Plan{wide, 1, full, kt});
+    }
+  }
+  return best;
 }
 
 bool big_linear_supported(const FusedArgs& a, int kind) {
@@ -572,45 +636,39 @@ bool big_linear_supported(const FusedArgs& a, int kind) {
   return kind == FL_QKV || kind == FL_SWIGLU || kind == FL_STORE;
 }
 
-size_t big_tail_part_floats(int M, int N, int K, int n_cu) {
-  const int tx = (N + BG_WN - 1) / BG_WN, T = tx * ((M + BG_WM - 1) / BG_WM), S = 2 * n_cu;
-  if (n_cu < 1 || T <= S) return 0;
-  const int full = T / S * S, rest = T - full;
-  const int kt = std::min(BG_TAIL_KT_MAX, std::min(S / std::max(rest, 1), K / 64));
-  if (rest % 8 || kt < 2) return 0;
-  return (size_t)rest * kt * BG_WM * BG_WN;
-}
-
-void big_linear(const FusedArgs& a, int kind, int KS, hipStream_t s, float* tail_part,
-                size_t tail_part_floats, int* tail_count, int n_tail_count) {
+void big_linear(const FusedArgs& a, int kind, const BigQ4Plan& p, hipStream_t s, float* tail_part,
+                int* tail_count) {
   require(big_linear_supported(a, kind), "large-M linear: unsupported shape or kind");
+  const int KS = p.ks;
+  const bool wide = p.wide;
   require(KS >= 1 && KS <= a.K / 64 && (KS == 1 || kind == FL_STORE),
           "large-M linear: split-K only for plain stores");
-  dim3 grid((a.N + BG_WN - 1) / BG_WN, (a.M + BG_WM - 1) / BG_WM, KS);
+  const int bn = wide ? 256 : 128;
+  dim3 grid((a.N + bn - 1) / bn, (a.M + BG_WM - 1) / BG_WM, KS);
   BgTail tail;
-  if (kind == FL_SWIGLU && KS == 1 && tail_part && tail_count && !a.fenced && a.n_xcc == 8) {
-    // the tiles past the last whole round of two work-groups per CU, split by K
-    int dev = 0, n_cu = 0;
-    DRT_HIP(hipGetDevice(&dev));
-    DRT_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-    const size_t need = big_tail_part_floats(a.M, a.N, a.K, n_cu);
-    const int T = (int)(grid.x * grid.y), S = 2 * n_cu;
-    if (need && need <= tail_part_floats && T - T / S * S <= n_tail_count) {
-      tail.full = T / S * S;
-      tail.kt = std::min(BG_TAIL_KT_MAX, std::min(S / (T - tail.full), a.K / 64));
-      tail.part = tail_part;
-      tail.count = tail_count;
-      grid = dim3((unsigned)(tail.full + (T - tail.full) * tail.kt), 1, 1);
-    }
+  if (p.kt > 0) {
+    const int T = (int)(grid.x * grid.y);
+    require(KS == 1 && (kind == FL_STORE || kind == FL_SWIGLU) && tail_part && tail_count &&
+                !a.fenced && a.n_xcc == 8 && p.full % 8 == 0 && p.full < T && p.kt >= 2 &&
+                p.kt <= BG_TAIL_KT_MAX && p.kt <= a.K / 64 && T - p.full <= BIG_TAIL_COUNTERS,
+            "large-M linear: split last round");
+    tail.full = p.full;
+    tail.rest = T - p.full;
+    tail.kt = p.kt;
+    tail.part = tail_part;
+    tail.count = tail_count;
+    grid = dim3((unsigned)(p.full + (tail.rest + 7) / 8 * 8 * p.kt), 1, 1);
   }
   const double bytes = (double)a.N * a.K / 2 + (double)a.N * a.K / 16 + 2.0 * a.M * a.K +
                        (kind == FL_STORE ? 4.0 * KS : 2.0) * a.M * a.N;
-#define DRT_BG(E)                                                                        \
-  {                                                                                      \
-    auto fn = big_q4_kernel<E>;                                                          \
-    static size_t granted = 0;                                                           \
-    grant_lds((const void*)fn, BG_LDS, granted);                                         \
-    DRT_LAUNCH(Profiler::GEMM, bytes, fn, grid, dim3(256), BG_LDS, s, a, KS, tail);      \
+#define DRT_BG(E)                                                                            \
+  {                                                                                          \
+    if (wide)                                                                                \
+      DRT_LAUNCH(Profiler::GEMM, bytes, (big_q4_kernel<E, 4, 2, 1, 4>), grid, dim3(256), 0, s, \
+                 a, KS, tail);                                                               \
+    else                                                                                     \
+      DRT_LAUNCH(Profiler::GEMM, bytes, (big_q4_kernel<E, 2, 2, 2, 2>), grid, dim3(256), 0, s, \
+                 a, KS, tail);                                                               \
   }
   if (kind == FL_QKV) DRT_BG(EPI_QKV)
   else if (kind == FL_SWIGLU) DRT_BG(EPI_SWIGLU)
@@ -638,16 +696,19 @@ void sum_slices(const float* part, int KS, int64_t n, const uint16_t* bias, int 
 }
 
 void big_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s) {
-  const int ks = big_linear_splits(a.M, a.N, a.K, BG_QKV_MAX_KS);
-  if (ks == 1 || ks > BG_QKV_MAX_KS || !part || (size_t)ks * a.M * a.N > part_floats) {
-    big_linear(a, FL_QKV, 1, s);
+  const BigQ4Plan whole = big_q4_plan(a.M, a.N, a.K, FL_QKV, 1, 0, 0.f, false);
+  // (the epilogue pass: its own launch and 6 us besides its bytes)
+  const BigQ4Plan split =
+      big_q4_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, part ? part_floats : 0, 6.f, false);
+  if (split.ks == 1) {
+    big_linear(a, FL_QKV, whole, s);
     return;
   }
   FusedArgs g = a;
   g.bias = nullptr;  // the epilogue adds it
   g.y = part;
-  big_linear(g, FL_STORE, ks, s);
-  qkv_epilogue_slices(a, part, ks, s);
+  big_linear(g, FL_STORE, split, s);
+  qkv_epilogue_slices(a, part, split.ks, s);
 }
 
 void qkv_epilogue_slices(const FusedArgs& a, const float* part, int ks, hipStream_t s) {

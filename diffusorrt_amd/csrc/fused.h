@@ -120,13 +120,20 @@ bool skinny_supported(int kind, int N, int K);
 // y + ks * M * N for a reduce pass).
 bool big_linear_supported(const FusedArgs& a, int kind);
 int big_linear_splits(int M, int N, int K, int max_ks);
-// tail_part / tail_count (optional): the workspace of the split last round (see
-// big_linear.hip), big_tail_part_floats() floats and one counter per split tile,
-// zero on entry and left zero.
-void big_linear(const FusedArgs& a, int kind, int KS, hipStream_t s, float* tail_part = nullptr,
-                size_t tail_part_floats = 0, int* tail_count = nullptr, int n_tail_count = 0);
-size_t big_tail_part_floats(int M, int N, int K, int n_cu);
-constexpr int BIG_TAIL_COUNTERS = 512;  // split tiles a runtime's counters cover
+// The plan of one: the tile (128 x 256 or 128 x 128), K slices, and the split last round
+// (see big_linear.hip; kt > 0): the first `full` tiles whole, the rest in kt K slices that
+// meet in tail_part ((tiles - full) * kt * 128 * 256 floats at most, within the plan's
+// part_floats) through one counter each, zero on entry and left zero.
+struct BigQ4Plan {
+  bool wide = true;
+  int ks = 1, full = 0, kt = 0;
+};
+BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+                      float reduce_us, bool tail_ok);
+void big_linear(const FusedArgs& a, int kind, const BigQ4Plan& p, hipStream_t s,
+                float* tail_part = nullptr, int* tail_count = nullptr);
+constexpr int BIG_TAIL_COUNTERS = 512;  // split tiles a caller's counters cover
+constexpr int BG_TAIL_KT_MAX = 8;       // K slices of one
 // The large-M bf16-weight kernels (M > 32, K % 64 == 0; big_bf16.hip): ACT_BF16
 // activation in, kinds FL_QKV, FL_SWIGLU (ACT_BF16 out) and FL_STORE (rounded with
 // the bias; ks > 1, or without rnd_bf16: fp32 slices y + ks * M * N for a reduce pass).

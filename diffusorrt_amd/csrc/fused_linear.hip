@@ -408,7 +408,7 @@ void fused_linear(const FusedArgs& a, int kind, hipStream_t s) {
   require(a.N % 32 == 0, "fused linear needs N % 32 == 0");
   if (skinny_linear(a, kind, s)) return;
   if (kind == FL_STORE && big_linear_supported(a, kind)) {  // > 32 rows, q4
-    big_linear(a, FL_STORE, 1, s);
+    big_linear(a, FL_STORE, big_q4_plan(a.M, a.N, a.K, FL_STORE, 1, 0, 0.f, false), s);
     return;
   }
   require(a.K % (a.qw ? 64 : 16) == 0, "fused linear needs K % 64 (q4) or K % 16 (bf16)");

@@ -772,7 +772,7 @@ void lmhead(const LinearW& w, const void* act, const float* xsum, int M, float* 
     f.lm_seed = seed;
     f.lm_step = step;
     f.lm_excl = exclude_col;
-    big_linear(f, FL_LMSTAT, 1, s);
+    big_linear(f, FL_LMSTAT, big_q4_plan(M, w.N, w.K, FL_LMSTAT, 1, 0, 0.f, false), s);
   } else {
   const size_t lds = (size_t)(w.q4 ? 2 : 1) * 32 * (chunk_k + 8) * 2 +
                      (size_t)32 * (chunk_k / 64) * 4 + (size_t)WAVES * 32 * 65 * 4;

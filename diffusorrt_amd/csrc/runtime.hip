@@ -486,10 +486,7 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
       }
       // the gate|up projection's split last round shares the workspace (it runs
       // between the q|k|v and down projections, which use it too)
-      int n_cu = 0;
-      DRT_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, rt->device));
-      for (int mt = 1; mt <= (M + 127) / 128; ++mt)
-        bf = std::max(bf, big_tail_part_floats(std::min(M, mt * 128), 2 * F, d, n_cu));
+      bf = std::max(bf, (size_t)n_cu_of_current_device() * 128 * 256);
       rt->big_part_floats = bf;
       rt->big_part.alloc(bf * 4);
       rt->big_tail_count.alloc((size_t)BIG_TAIL_COUNTERS * 4);
@@ -783,10 +780,10 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       big_bf16_linear(f, FL_STORE, bp, s);
       return bp.ks;
     }
-    const int ks = big_linear_splits(M, f.N, f.K, max_ks);
-    require((size_t)ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
-    big_linear(f, FL_STORE, ks, s);
-    return ks;
+    const BigQ4Plan bp = big_q4_plan(M, f.N, f.K, FL_STORE, max_ks, rt.big_part_floats, 0.f, false);
+    require((size_t)bp.ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
+    big_linear(f, FL_STORE, bp, s);
+    return bp.ks;
   };
   auto big_resid = [&](FusedArgs f, const uint16_t* next_norm) {
     require(f.bias == nullptr, "o_proj / down_proj bias is not supported on this path");
@@ -889,8 +886,10 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       fg.act_out = rt.act2.p;
       fg.act_fmt = fmt;
       if (rt.q4)
-        big_linear(fg, FL_SWIGLU, 1, s, bpart, rt.big_part_floats, rt.big_tail_count.as<int>(),
-                   BIG_TAIL_COUNTERS);
+        big_linear(fg, FL_SWIGLU,
+                   big_q4_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats, 0.f,
+                               !rt.fenced && rt.n_xcc == 8),
+                   s, bpart, rt.big_tail_count.as<int>());
       else
         big_bf16_linear(fg, FL_SWIGLU, big_bf16_plan(M, fg.N, fg.K, FL_SWIGLU, 1, 0, 0.f), s);
       FusedArgs fd = base(w.down);
@@ -2321,7 +2320,6 @@ static void q4_linear_into(const void* qw, const void* sb, const void* x, int32_
     f.act = xp;
     f.act_xsum = xs;
     f.y = y;
-    const int ks = m > 32 ? big_linear_splits(m, n, k, BG_OP_MAX_KS) : 1;
     if (sp.KS >= 1) {
       // large weights, <= 32 rows: streamed in fp32 K slices, summed (+ bias) into y
       float* part = (float*)(ws + q4_op_act_bytes(m, k));
@@ -2330,14 +2328,29 @@ static void q4_linear_into(const void* qw, const void* sb, const void* x, int32_
       g.y = part;
       stream_linear(g, sp, st);
       sum_slices(part, sp.KS, (int64_t)m * n, (const uint16_t*)bias, n, y, st);
-    } else if (ks > 1 && big_linear_supported(f, FL_STORE)) {
-      // split-K slices in the workspace, summed (+ bias) into y in a fixed order
+    } else if (m > 32) {
+      // planned within the slices the workspace rule provides (the same plan whichever
+      // workspace is passed); the split last round needs a counter block of this stream,
+      // which a graph capture cannot own (its replays may run beside the stream's calls)
       float* part = (float*)(ws + q4_op_act_bytes(m, k));
+      const size_t part_floats = (size_t)big_linear_splits(m, n, k, BG_OP_MAX_KS) * m * n;
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      DRT_HIP(hipStreamIsCapturing(st, &cap));
       FusedArgs g = f;
-      g.bias = nullptr;
-      g.y = part;
-      big_linear(g, FL_STORE, ks, st);
-      sum_slices(part, ks, (int64_t)m * n, (const uint16_t*)bias, n, y, st);
+      int* count = nullptr;
+      bool fenced = true;
+      if (cap == hipStreamCaptureStatusNone) count = op_counters_for(st, g.n_xcc, fenced);
+      g.fenced = fenced ? 1 : 0;
+      const BigQ4Plan p = big_q4_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, part_floats, 2.5f,
+                                      count && !fenced && g.n_xcc == 8);
+      if (p.ks > 1) {  // slices, summed (+ bias) into y in a fixed order
+        g.bias = nullptr;
+        g.y = part;
+        big_linear(g, FL_STORE, p, st);
+        sum_slices(part, p.ks, (int64_t)m * n, (const uint16_t*)bias, n, y, st);
+      } else {
+        big_linear(g, FL_STORE, p, st, part, count);
+      }
     } else {
       fused_linear(f, FL_STORE, st);
     }

@@ -204,6 +204,48 @@ def test_bf16_linear_large_m(m, n, k, with_ws):
     assert (err <= bound).all()
 
 
+# The large-M q4 kernels: both tiles, unsplit and split, the split last round beside one
+# work-group per CU (296 wide tiles on 256 CUs) with a row remainder, fewer groups than
+# buffers, and the same call inside a graph capture (no split last round there).
+@pytest.mark.parametrize("m,n,k", [(33, 32, 64), (65, 160, 128), (129, 1024, 192), (41, 18944, 3584),
+                                   (2048, 1024, 1024), (500, 18944, 1024), (300, 4608, 3584)])
+def test_q4_linear_large_m_plans(m, n, k):
+    from diffusorrt_amd import kernels
+
+    _say("q4_linear large M", m, n, k)
+    gen, q = _q4_case(n, k, seed=35)
+    x = torch.randn((m, k), generator=gen)
+    bias = torch.randn((n,), generator=gen).to(torch.bfloat16)
+    w = kernels.DeviceQ4Weight(q.w_q.cuda(), q.scales.cuda(), q.biases.cuda())
+    xd, bd = x.cuda(), bias.cuda()
+    y = kernels.linear(xd, w, bd).double()
+    # the operands the kernels multiply: each weight rounded once to fp16, x as hi + lo
+    shifts = torch.arange(8, dtype=torch.int32, device="cuda") * 4
+    nib = ((q.w_q.cuda().unsqueeze(-1) >> shifts) & 15).reshape(n, -1, 64).double()
+    w16 = (nib * q.scales.cuda().double().unsqueeze(-1) +
+           q.biases.cuda().double().unsqueeze(-1)).reshape(n, -1).half().double()
+    exact = xd.double() @ w16.t()
+    mag = xd.double().abs() @ w16.abs().t()
+    # an fp32 sum of k / 16 MFMA results and the slices (k / 8 * 2^-24 of the magnitudes
+    # at most), the pair's 2^-22, and the rounding of the bias addition
+    bound = mag * ((k / 8) * 2.0 ** -24 + 2.0 ** -21) + 2.0 ** -23 * (y.abs() + bd.double().abs())
+    err = (y - (exact + bd.double())).abs()
+    _say(f"  worst error / bound {float((err / bound).max()):.3f}")
+    assert bool((err <= bound).all())
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        kernels.linear(xd, w, bd)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        yg = kernels.linear(xd, w, bd)
+    for _ in range(3):
+        yg.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool(((yg.double() - (exact + bd.double())).abs() <= bound).all())
+
+
 # ---------------------------------------------------------------- attention (config 2)
 
 def _attention_inputs(L, seed=1, rows=32, hq=16, hkv=8):
