@@ -15,13 +15,14 @@ struct FusedArgs {
   const uint16_t* wb = nullptr;
   const uint16_t* bias = nullptr;
   int M = 0, N = 0, K = 0;
-  // XCDs of the device (work-group i runs on XCD i % n_xcc) and the flag a
+  // XCDs of the device (work-group i runs on XCD (i + xcc_rot) % n_xcc) and the flag a
   // work-group sets if it finds itself on another XCD (next to M, N, K: the
   // skinny kernels fetch these first, in one scalar load)
   int n_xcc = 1;
   // 1: the placement above is not assumed; split-K slices meet through
   // device-scope fences and atomics instead of one XCD's L2
   int fenced = 0;
+  int xcc_rot = 0;
   int* placement_err = nullptr;
   // PRO_ACT: activation [M][K] (ACT_F16P + xsum[M][K/64], or ACT_BF16); for
   // the split-K q4 store kernel also fp32 (x_in 1) or bf16 (x_in 2) rows
@@ -109,8 +110,13 @@ void fused_linear(const FusedArgs& a, int kind, hipStream_t s);
 bool skinny_linear(const FusedArgs& a, int kind, hipStream_t s);
 // Workspace the skinny kernels need for a linear of N outputs and K inputs.
 size_t skinny_part_floats(int N, int K);
-// One probe launch: does work-group i run on XCD i % n_xcc? (scratch_dev: >= 256 ints)
-bool probe_round_robin(int n_xcc, int* scratch_dev, hipStream_t s);
+// One probe launch: the rotation r for which work-group i runs on XCD (i + r) % n_xcc, or
+// -1 where there is none (scratch_dev: >= 256 ints). It is the hardware queue's: 0 in a
+// process with one queue, another for each queue once there are several.
+int probe_round_robin(int n_xcc, int* scratch_dev, hipStream_t s);
+// What a work-group that finds itself on XCD xcc, a launch's rotation r away from its
+// place x, reports besides the placement bit.
+constexpr int placement_bit(int r) { return 1 << (8 + r); }
 int skinny_counters(int N);
 // Whether the split-K kernels take a linear of this kind and shape (given
 // workspaces sized by skinny_part_floats / skinny_counters).

@@ -152,6 +152,11 @@ struct Runtime {
   int sk_n_counters = 0;
   int n_xcc = 1;
   bool fenced = false;           // split-K exchange through device-scope fences (no placement assumed)
+  // rotation of this stream's work-groups over the XCDs (probe_round_robin), its probe's
+  // scratch, and whether it was probed (not overridden)
+  int xcc_rot = 0;
+  DevBuf xcc_probe;
+  bool xcc_probed = false;
   DevBuf placement_err;          // int, set by a kernel that finds itself on an unexpected XCD
   int* placement_host = nullptr; // pinned copy, read after each synchronized forward
   // pinned landing area of a forward's scores and tokens, written by the LM head's
@@ -498,15 +503,20 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     rt->n_xcc = std::max(1, nx);
     // DRT_N_XCC overrides the XCD count the split-K grids are laid out for (a
     // test hook: a wrong count must surface as the placement error); otherwise
-    // one probe launch checks the round-robin placement, and where it does not
-    // hold the split-K exchange runs fenced (DRT_SPLITK_FENCED=1 forces that).
+    // one probe launch finds the round-robin placement's rotation - another for each
+    // hardware queue of a process with several (5, 6, 7 and 0 seen), which took the whole
+    // runtime to the fenced exchange when only 0 was taken (a step over 8192 keys 1565
+    // against 1255 us) - and where there is none the split-K exchange runs fenced
+    // (DRT_SPLITK_FENCED=1 forces that).
     const char* nx_env = getenv("DRT_N_XCC");
     if (nx_env && atoi(nx_env) >= 1) {
       rt->n_xcc = atoi(nx_env);
     } else {
-      DevBuf probe;
-      probe.alloc(256 * sizeof(int));
-      rt->fenced = !probe_round_robin(rt->n_xcc, probe.as<int>(), s);
+      rt->xcc_probe.alloc(256 * sizeof(int));
+      const int rot = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s);
+      rt->fenced = rot < 0;
+      rt->xcc_rot = std::max(0, rot);
+      rt->xcc_probed = true;
     }
     if (getenv("DRT_SPLITK_FENCED") != nullptr) rt->fenced = true;
     rt->placement_err.alloc(4);
@@ -812,6 +822,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       f.sk_row_tiles = SK_ROW_TILES;
       f.n_xcc = rt.n_xcc;
       f.fenced = rt.fenced ? 1 : 0;
+      f.xcc_rot = rt.xcc_rot;
       f.placement_err = rt.placement_err.as<int>();
       return f;
     };
@@ -956,14 +967,25 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
   }
 }
 
-// The split-K linears rely on work-group i running on XCD i % n_xcc; a kernel
+// The split-K linears rely on work-group i running on XCD (i + r) % n_xcc; a kernel
 // that observed otherwise left a flag (read back with the forward's results).
 // Bit 2 of the same flag: a wave of the decode attention gave up waiting for a K/V
 // tile (its bounded wait ran out), so that forward's attention is not valid.
-void check_placement(const Runtime& rt) {
+void check_placement(Runtime& rt) {
   // the placement first: a split-K exchange across XCDs produces garbage, which
   // may also trip the other two checks
-  const int e = *rt.placement_host;
+  int e = *rt.placement_host;
+  if ((e & 1) && rt.xcc_probed && !rt.fenced) {
+    // Another rotation throughout (every report the same, and what the stream has now): a
+    // hardware queue created since moved this one. What the exchange needs, equal i %
+    // n_xcc on one XCD, held all along.
+    const int r = probe_round_robin(rt.n_xcc, rt.xcc_probe.as<int>(), rt.stream);
+    if (r >= 0 && (e & ~(1 | placement_bit(r))) == 0 && (e & placement_bit(r))) {
+      rt.xcc_rot = r;
+      DRT_HIP(hipMemsetAsync(rt.placement_err.p, 0, 4, rt.stream));
+      e = *rt.placement_host = 0;
+    }
+  }
   if (e & 1)
     fail(INTERNAL_ERROR,
          "a split-K linear ran on an unexpected XCD (work-group placement is not the "
@@ -2225,15 +2247,15 @@ int* op_counters_for(hipStream_t stream, int& n_xcc, bool& fenced) {
     d.n_xcc = std::max(1, nx);
     hipStream_t ps = nullptr;
     DRT_HIP(hipStreamCreateWithFlags(&ps, hipStreamNonBlocking));
-    bool rr = false;
+    int rot = -1;
     try {
-      rr = probe_round_robin(d.n_xcc, (int*)pr, ps);
+      rot = probe_round_robin(d.n_xcc, (int*)pr, ps);
     } catch (...) {
       (void)hipStreamDestroy(ps);
       throw;
     }
     DRT_HIP(hipStreamDestroy(ps));
-    d.fenced = !rr;
+    d.fenced = rot < 0;  // (any rotation keeps equal i % n_xcc on one XCD, on any stream)
     d.counters = (int*)c;
   }
   n_xcc = d.n_xcc;

@@ -17,7 +17,7 @@
 // dimension: each tile's work-groups repeat the weight slices (the second read
 // mostly from L2) and keep partials, counters and row statistics of their own.
 //
-// The exchange stays inside one XCD's L2: work-group i runs on XCD i % n_xcc
+// The exchange stays inside one XCD's L2: work-group i runs on XCD (i + r) % n_xcc
 // (the dispatcher's round-robin), so the grid is laid out to give every slice
 // of block b the XCD b % n_xcc. Plain stores, the L2 atomic and plain loads are
 // then coherent with each other, with no device-wide fence (an L2 writeback and
@@ -77,14 +77,17 @@ constexpr int SK_SS_PER_THREAD = 14; // K / 32 <= 8 * 14 = 112 partial sums (d <
 // loads: an early return would let the compiler sink the loads, and the kernel
 // argument fetches they need, behind the branch - one more round trip for
 // every work-group.) n_xcc and perr are the pinned a.n_xcc, a.placement_err.
-DRT_DEV bool sk_place(int n_xcc, int fenced, int* perr, int n_blocks, int KS, int& blk,
+DRT_DEV bool sk_place(int n_xcc, int fenced, int rot, int* perr, int n_blocks, int KS, int& blk,
                       int& ks) {
   const int i = blockIdx.x, x = i % n_xcc, j = i / n_xcc;
   blk = x + n_xcc * (j / KS);
   ks = j - (j / KS) * KS;
   if (n_xcc > 1 && !fenced && threadIdx.x == 0 && perr) {
     const int xcc = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xf);  // HW_REG_XCC_ID
-    if (xcc != x) __hip_atomic_fetch_or(perr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int r = (xcc - x) & 7;
+    if (r != rot)
+      __hip_atomic_fetch_or(perr, 1 | drt::placement_bit(r), __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_AGENT);
   }
   const bool live = blk < n_blocks;
   blk = live ? blk : 0;
@@ -157,16 +160,17 @@ DRT_DEV void sk_wide_sum_slices(const float* pbase, int KS, float* red, bool rnd
 // Everything the first loads need is in the leading scalar arguments, which
 // arrive in scalar registers at wave start (kernel-argument preloading, 16
 // dwords): the sizes packed as dims0 = N | K << 16 and dims1 = M | KS << 8 |
-// n_xcc << 16 | fenced << 24. The rest of the arguments (`a`) are fetched
+// n_xcc << 16 | fenced << 24 | rot << 25. The rest of the arguments (`a`) are fetched
 // while the first loads are in flight.
 DRT_DEV void sk_dims(uint32_t dims0, uint32_t dims1, int& M, int& N, int& K, int& KS, int& n_xcc,
-                     int& fenced) {
+                     int& fenced, int& rot) {
   N = (int)(dims0 & 0xffffu);
   K = (int)(dims0 >> 16);
   M = (int)(dims1 & 0xffu);
   KS = (int)((dims1 >> 8) & 0xffu);
   n_xcc = (int)((dims1 >> 16) & 0xffu);
-  fenced = (int)(dims1 >> 24);
+  fenced = (int)((dims1 >> 24) & 1u);
+  rot = (int)(dims1 >> 25);
 }
 
 // PRE: the input is pre-scaled ACT_F16P planes (see FusedArgs::pre_out):
@@ -182,8 +186,8 @@ __global__ __launch_bounds__(256) void skinny_wide_kernel(
   constexpr bool BF = WK == W_BF16;
   static_assert(!PRE || !BF, "pre-scaled planes feed the q4 kernels only");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int M, N, K, KS, n_xcc, fenced;
-  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced);
+  int M, N, K, KS, n_xcc, fenced, rot;
+  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced, rot);
   // 32-row tile of this work-group: rows m0 .. m0 + M - 1 of the forward
   const int mt = blockIdx.y, m0 = 32 * mt, M_all = M;
   M = min(32, M_all - m0);
@@ -195,7 +199,7 @@ __global__ __launch_bounds__(256) void skinny_wide_kernel(
   int* counters = a.counters + (size_t)mt * a.n_counters;
   const int G = K >> 6;
   int grp, ks;
-  const bool live = sk_place(n_xcc, fenced, perr, N / 128, KS, grp, ks);
+  const bool live = sk_place(n_xcc, fenced, rot, perr, N / 128, KS, grp, ks);
   const int nt = grp * 4 + wave;
   const int u0 = ks * U, kc0 = u0 * 64;
   // absolute position of row 0 (the q|k|v epilogue's rotary tables), read at
@@ -477,8 +481,8 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
   static_assert(XIN == 0 || WK == W_Q4, "fp32 / bf16 rows feed the q4 kernels only");
   constexpr bool BF = WK == W_BF16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int M, N, K, KS, n_xcc, fenced;
-  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced);
+  int M, N, K, KS, n_xcc, fenced, rot;
+  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced, rot);
   // 32-row tile of this work-group: rows m0 .. m0 + M - 1 of the forward
   const int mt = blockIdx.y, m0 = 32 * mt, M_all = M;
   M = min(32, M_all - m0);
@@ -487,7 +491,7 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
   const int G = K >> 6;
   const int U = G / KS;
   int nt, ks;
-  const bool live = sk_place(n_xcc, fenced, perr, N / 32, KS, nt, ks);
+  const bool live = sk_place(n_xcc, fenced, rot, perr, N / 32, KS, nt, ks);
   const int u_lo = ks * U + (U * wave) / 4, u_hi = ks * U + (U * (wave + 1)) / 4;
   extern __shared__ __align__(16) char smem[];
   float* red = (float*)smem;  // [4][32][33]
@@ -762,9 +766,9 @@ __global__ __launch_bounds__(512) void skinny_gu_kernel(
   constexpr int K = G * 64, ROW = K + 8, CPR = G / 8, UPW = G / 8, RH = GU_RH;
   constexpr int RS = GU_RS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int M, N, Kd, KS, n_xcc, fenced;
-  sk_dims(dims0, dims1, M, N, Kd, KS, n_xcc, fenced);
-  (void)Kd, (void)KS, (void)n_xcc, (void)fenced, (void)perr;
+  int M, N, Kd, KS, n_xcc, fenced, rot;
+  sk_dims(dims0, dims1, M, N, Kd, KS, n_xcc, fenced, rot);
+  (void)Kd, (void)KS, (void)n_xcc, (void)fenced, (void)rot, (void)perr;
   // rows m0 .. m0 + M - 1 of the forward: half hr of 32-row tile mt
   const int mt = blockIdx.y >> 1, hr = blockIdx.y & 1, tr0 = RH * hr;
   const int m0 = 32 * mt + tr0, M_all = M;
@@ -968,10 +972,10 @@ int narrow_slices(int N, int K) {
 
 }  // namespace
 
-// Whether work-group i of a launch runs on XCD i % n_xcc (the layout the
+// The rotation r for which work-group i of a launch runs on XCD (i + r) % n_xcc (the layout the
 // split-K exchange assumes), from one probe launch of 4 * 64 work-groups.
-bool probe_round_robin(int n_xcc, int* scratch_dev, hipStream_t s) {
-  if (n_xcc <= 1) return true;
+int probe_round_robin(int n_xcc, int* scratch_dev, hipStream_t s) {
+  if (n_xcc <= 1) return 0;
   constexpr int WGS = 256;
   hipLaunchKernelGGL(xcc_probe_kernel, dim3(WGS), dim3(64), 0, s, scratch_dev);
   DRT_HIP(hipGetLastError());
@@ -979,8 +983,8 @@ bool probe_round_robin(int n_xcc, int* scratch_dev, hipStream_t s) {
   DRT_HIP(hipMemcpyAsync(xcc.data(), scratch_dev, WGS * sizeof(int), hipMemcpyDeviceToHost, s));
   DRT_HIP(hipStreamSynchronize(s));
   for (int i = 0; i < WGS; ++i)
-    if (xcc[i] != i % n_xcc) return false;
-  return true;
+    if (xcc[i] != (i + xcc[0]) % n_xcc) return -1;
+  return xcc[0];
 }
 
 size_t skinny_part_floats(int N, int K) {
@@ -1008,7 +1012,7 @@ bool skinny_supported(int kind, int N, int K) {
 namespace {
 uint32_t sk_dims1(const FusedArgs& a, int KS) {
   return (uint32_t)a.M | ((uint32_t)KS << 8) | ((uint32_t)a.n_xcc << 16) |
-         ((uint32_t)(a.fenced ? 1 : 0) << 24);
+         ((uint32_t)(a.fenced ? 1 : 0) << 24) | ((uint32_t)a.xcc_rot << 25);
 }
 }  // namespace
 

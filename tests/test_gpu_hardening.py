@@ -6,6 +6,8 @@ kernel still runs to completion:
   raises, and the GPU is then fine for a new runtime;
 * the fenced split-K exchange (``DRT_SPLITK_FENCED=1``, what a runtime falls
   back to when its placement probe fails) gives bit-identical results;
+* hardware queues that come into being after a runtime and move where its stream's
+  work-groups land: the same results as before;
 * the fp16 range of the activations: a first-layer norm weight that pushes the
   normalized activation past 65504 raises the range error, one that keeps it
   near 4e4 (checked on the CPU) does not.
@@ -13,6 +15,8 @@ kernel still runs to completion:
 from __future__ import annotations
 
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -74,6 +78,44 @@ def test_fenced_split_k_exchange_is_bit_identical():
     s1, t1, f1 = _propose(model, {"DRT_SPLITK_FENCED": "1"})
     assert (t1, f1) == (t0, f0)
     assert np.array_equal(np.asarray(s1), np.asarray(s0))
+
+
+_LATER_QUEUES = """
+import sys
+sys.path[:0] = [%r, %r]
+import numpy as np, torch
+from diffusorrt_amd import synthetic as syn
+from diffusorrt_amd.runtime import Runtime, bd3_session_config
+from helpers import tiny_geometry
+model = syn.build_model(tiny_geometry(), "q4", seed=54)
+g = model.geometry
+rt = Runtime(model, max_forward_rows=256, max_positions=512)
+x = list(range(64)) + [g.mask_token_id] * 32
+with rt.session(bd3_session_config(32, 8, len(x))) as s:
+    s.start_device(x, prompt_len=0, block_size=32, mask_token_id=g.mask_token_id,
+                   exact_kv=False, steps=8)
+    def once():
+        return s.propose_device(list(range(64, 96)), window_end=96, frozen_prefix=64)[:2]
+    first = [once() for _ in range(3)]  # eager, captured, replayed
+    streams = [torch.cuda.Stream() for _ in range(8)]
+    for st in streams:
+        with torch.cuda.stream(st):
+            torch.zeros(1, device="cuda")
+    torch.cuda.synchronize()
+    later = [once() for _ in range(3)]
+assert all(np.array_equal(np.asarray(a[0]), np.asarray(first[0][0])) and a[1] == first[0][1]
+           for a in first + later)
+rt.close()
+print("same")
+"""
+
+
+def test_queues_created_after_the_runtime():
+    _say("later hardware queues")
+    here = os.path.dirname(os.path.abspath(__file__))
+    out = subprocess.run([sys.executable, "-c", _LATER_QUEUES % (os.path.dirname(here), here)],
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.strip().endswith("same"), out.stdout + out.stderr
 
 
 def test_fp16_range_flag():
