@@ -53,12 +53,14 @@ extern "C" __global__ __launch_bounds__(256) void embed_kernel(
     float* __restrict__ hidden, int M, int d, float* __restrict__ ss_out,
     const StepDesc* __restrict__ row_desc, const uint16_t* __restrict__ pre_norm, float eps,
     uint16_t* __restrict__ pre, float* __restrict__ pre_xs, float* __restrict__ pre_sc,
-    int* __restrict__ err) {
+    int* __restrict__ err, int* __restrict__ rot) {
   // thread c owns columns 32c .. 32c + 31 (d % 32 == 0, d <= 32 * 256); every
   // load is issued before the first store (a wait for a load also waits for the
   // stores issued before it)
   const int m = blockIdx.x, c = threadIdx.x, ng = d >> 5;
   const bool live = c < ng;
+  if (rot && m == 0 && c == 0)  // where this launch's work-group 0 runs (see probe_round_robin)
+    *rot = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0x7);  // HW_REG_XCC_ID
   if (row_desc) tokens += row_desc->row0;
   float* ss_row = ss_out ? ss_out + (int64_t)(m >> 5) * d + (m & 31) : nullptr;
   float* xs_row = pre ? pre_xs + (int64_t)(m >> 5) * d + (m & 31) : nullptr;
@@ -424,7 +426,7 @@ extern "C" __global__ void swiglu_rows_kernel(const float* __restrict__ g,
 namespace drt {
 
 void embed(const int32_t* tokens, const uint16_t* table, float* hidden, int M, int d,
-           float* ss_out, hipStream_t s, const StepDesc* row_desc, const PreOut* pre) {
+           float* ss_out, hipStream_t s, const StepDesc* row_desc, const PreOut* pre, int* rot) {
   require(d % 32 == 0 && d <= 32 * 256, "embed needs d % 32 == 0 and d <= 8192");
   require(!pre || ss_out, "pre-scaled planes need the row statistics");
   // with ss_out, whole 32-row tiles are launched so unused rows get zero partials
@@ -432,7 +434,7 @@ void embed(const int32_t* tokens, const uint16_t* table, float* hidden, int M, i
   hipLaunchKernelGGL(embed_kernel, dim3(grid), dim3(256), 0, s, tokens, table, hidden, M, d,
                      ss_out, row_desc, pre ? pre->norm : nullptr, pre ? pre->eps : 0.f,
                      pre ? pre->planes : nullptr, pre ? pre->xs : nullptr,
-                     pre ? pre->sc : nullptr, pre ? pre->err : nullptr);
+                     pre ? pre->sc : nullptr, pre ? pre->err : nullptr, rot);
   DRT_HIP(hipGetLastError());
 }
 

@@ -15,14 +15,14 @@ struct FusedArgs {
   const uint16_t* wb = nullptr;
   const uint16_t* bias = nullptr;
   int M = 0, N = 0, K = 0;
-  // XCDs of the device (work-group i runs on XCD (i + xcc_rot) % n_xcc) and the flag a
-  // work-group sets if it finds itself on another XCD (next to M, N, K: the
-  // skinny kernels fetch these first, in one scalar load)
+  // XCDs of the device (work-group i runs on XCD (i + r) % n_xcc) and the flag a
+  // work-group sets if it finds itself on another XCD, with this forward's r in the
+  // word after it (next to M, N, K: the skinny kernels fetch these first, in one
+  // scalar load)
   int n_xcc = 1;
   // 1: the placement above is not assumed; split-K slices meet through
   // device-scope fences and atomics instead of one XCD's L2
   int fenced = 0;
-  int xcc_rot = 0;
   int* placement_err = nullptr;
   // PRO_ACT: activation [M][K] (ACT_F16P + xsum[M][K/64], or ACT_BF16); for
   // the split-K q4 store kernel also fp32 (x_in 1) or bf16 (x_in 2) rows

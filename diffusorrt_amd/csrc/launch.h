@@ -201,6 +201,7 @@ void kv_pack(bool kv_bf16, const void* k, const void* v, bool src_bf16, int n, i
              void* kv_layer, int64_t kv_head_stride, hipStream_t s);
 
 // Epilogues.
+// rot (optional): receives the XCD rotation of the launch (see probe_round_robin).
 // ss_out (optional, M <= 32): per-32-column partial sums of squares of the rows,
 // [d/32][32], the row statistics of the first decoder layer's RMSNorm.
 // The first layer's pre-scaled norm input that embed() writes with the residual
@@ -216,7 +217,7 @@ struct PreOut {
 };
 void embed(const int32_t* tokens, const uint16_t* table, float* hidden, int M, int d,
            float* ss_out, hipStream_t s, const StepDesc* row_desc = nullptr,
-           const PreOut* pre = nullptr);
+           const PreOut* pre = nullptr, int* rot = nullptr);
 void residual_norm(float* hidden, const float* part, int splits, int M_part, bool rnd_bf16,
                    const int32_t* src_rows, bool write_hidden, const uint16_t* norm_w, float eps,
                    int d, int fmt, void* act, float* xsum, int n_out_rows, hipStream_t s,

@@ -152,12 +152,11 @@ struct Runtime {
   int sk_n_counters = 0;
   int n_xcc = 1;
   bool fenced = false;           // split-K exchange through device-scope fences (no placement assumed)
-  // rotation of this stream's work-groups over the XCDs (probe_round_robin), its probe's
-  // scratch, and whether it was probed (not overridden)
-  int xcc_rot = 0;
+  // scratch of the placement's probe, and whether it was probed (not overridden)
   DevBuf xcc_probe;
   bool xcc_probed = false;
-  DevBuf placement_err;          // int, set by a kernel that finds itself on an unexpected XCD
+  DevBuf placement_err;          // int, set by a kernel that finds itself on an unexpected XCD,
+                                 // and this forward's rotation (written by its embedding)
   int* placement_host = nullptr; // pinned copy, read after each synchronized forward
   // pinned landing area of a forward's scores and tokens, written by the LM head's
   // last kernel (the caller's arrays are pageable)
@@ -503,24 +502,23 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     rt->n_xcc = std::max(1, nx);
     // DRT_N_XCC overrides the XCD count the split-K grids are laid out for (a
     // test hook: a wrong count must surface as the placement error); otherwise
-    // one probe launch finds the round-robin placement's rotation - another for each
-    // hardware queue of a process with several (5, 6, 7 and 0 seen), which took the whole
-    // runtime to the fenced exchange when only 0 was taken (a step over 8192 keys 1565
-    // against 1255 us) - and where there is none the split-K exchange runs fenced
-    // (DRT_SPLITK_FENCED=1 forces that).
+    // one probe launch checks the placement for a round-robin of any rotation - another
+    // for each hardware queue of a process with several (5, 6, 7 and 0 seen), which took
+    // the whole runtime to the fenced exchange when only 0 was taken (a step over 8192
+    // keys 1565 against 1255 us) - and where there is none the split-K exchange runs
+    // fenced (DRT_SPLITK_FENCED=1 forces that). The rotation itself is taken anew by each
+    // forward's first kernel: queues created later move it.
     const char* nx_env = getenv("DRT_N_XCC");
     if (nx_env && atoi(nx_env) >= 1) {
       rt->n_xcc = atoi(nx_env);
     } else {
       rt->xcc_probe.alloc(256 * sizeof(int));
-      const int rot = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s);
-      rt->fenced = rot < 0;
-      rt->xcc_rot = std::max(0, rot);
+      rt->fenced = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s) < 0;
       rt->xcc_probed = true;
     }
     if (getenv("DRT_SPLITK_FENCED") != nullptr) rt->fenced = true;
-    rt->placement_err.alloc(4);
-    DRT_HIP(hipMemsetAsync(rt->placement_err.p, 0, 4, s));
+    rt->placement_err.alloc(8);
+    DRT_HIP(hipMemsetAsync(rt->placement_err.p, 0, 8, s));
     DRT_HIP(hipHostMalloc((void**)&rt->placement_host, 4, hipHostMallocCoherent));
     *rt->placement_host = 0;
   }
@@ -762,7 +760,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       po.err = rt.placement_err.as<int>();
     }
     embed(p.tokens_rel, rt.embed.as<uint16_t>(), hidden, M, d, ss, s,
-          p.tokens_at_row0 ? desc : nullptr, pre ? &po : nullptr);
+          p.tokens_at_row0 ? desc : nullptr, pre ? &po : nullptr, rt.placement_err.as<int>() + 1);
   }
   if (big && L > 0)
     residual_norm(hidden, nullptr, 0, M, false, nullptr, false,
@@ -822,7 +820,6 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       f.sk_row_tiles = SK_ROW_TILES;
       f.n_xcc = rt.n_xcc;
       f.fenced = rt.fenced ? 1 : 0;
-      f.xcc_rot = rt.xcc_rot;
       f.placement_err = rt.placement_err.as<int>();
       return f;
     };
@@ -976,12 +973,11 @@ void check_placement(Runtime& rt) {
   // may also trip the other two checks
   int e = *rt.placement_host;
   if ((e & 1) && rt.xcc_probed && !rt.fenced) {
-    // Another rotation throughout (every report the same, and what the stream has now): a
-    // hardware queue created since moved this one. What the exchange needs, equal i %
-    // n_xcc on one XCD, held all along.
+    // Another rotation from some kernel on (every report the same, and what the stream has
+    // now): a hardware queue created during the forward moved this one. What the exchange
+    // needs, equal i % n_xcc on one XCD, held all along.
     const int r = probe_round_robin(rt.n_xcc, rt.xcc_probe.as<int>(), rt.stream);
     if (r >= 0 && (e & ~(1 | placement_bit(r))) == 0 && (e & placement_bit(r))) {
-      rt.xcc_rot = r;
       DRT_HIP(hipMemsetAsync(rt.placement_err.p, 0, 4, rt.stream));
       e = *rt.placement_host = 0;
     }

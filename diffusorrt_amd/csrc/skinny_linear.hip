@@ -76,22 +76,29 @@ constexpr int SK_SS_PER_THREAD = 14; // K / 32 <= 8 * 14 = 112 partial sums (d <
 // block 0 and must leave before their first store. (They run on past their
 // loads: an early return would let the compiler sink the loads, and the kernel
 // argument fetches they need, behind the branch - one more round trip for
-// every work-group.) n_xcc and perr are the pinned a.n_xcc, a.placement_err.
-DRT_DEV bool sk_place(int n_xcc, int fenced, int rot, int* perr, int n_blocks, int KS, int& blk,
-                      int& ks) {
+// every work-group.) n_xcc is the pinned a.n_xcc.
+DRT_DEV bool sk_place(int n_xcc, int n_blocks, int KS, int& blk, int& ks) {
   const int i = blockIdx.x, x = i % n_xcc, j = i / n_xcc;
   blk = x + n_xcc * (j / KS);
   ks = j - (j / KS) * KS;
-  if (n_xcc > 1 && !fenced && threadIdx.x == 0 && perr) {
-    const int xcc = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xf);  // HW_REG_XCC_ID
-    const int r = (xcc - x) & 7;
-    if (r != rot)
-      __hip_atomic_fetch_or(perr, 1 | drt::placement_bit(r), __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-  }
   const bool live = blk < n_blocks;
   blk = live ? blk : 0;
   return live;
+}
+
+// In a work-group that has arrived and is not the last: is it where this forward's
+// rotation (written after the error word by its embedding kernel) puts it? If not, it
+// reports the rotation it sees. Here the read of the rotation delays nothing (read at the
+// start, it cost each kernel 0.3 us); the last work-group of a block counted every other
+// arrival in its own XCD's L2.
+DRT_DEV void sk_check(int n_xcc, int fenced, int* perr) {
+  if (n_xcc > 1 && !fenced && threadIdx.x == 0 && perr) {
+    const int xcc = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xf);  // HW_REG_XCC_ID
+    const int r = (xcc - (int)blockIdx.x % n_xcc) & 7;
+    if (r != perr[1])
+      __hip_atomic_fetch_or(perr, 1 | drt::placement_bit(r), __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // Called after this work-group stored its partial: returns true in the last
@@ -160,17 +167,16 @@ DRT_DEV void sk_wide_sum_slices(const float* pbase, int KS, float* red, bool rnd
 // Everything the first loads need is in the leading scalar arguments, which
 // arrive in scalar registers at wave start (kernel-argument preloading, 16
 // dwords): the sizes packed as dims0 = N | K << 16 and dims1 = M | KS << 8 |
-// n_xcc << 16 | fenced << 24 | rot << 25. The rest of the arguments (`a`) are fetched
+// n_xcc << 16 | fenced << 24. The rest of the arguments (`a`) are fetched
 // while the first loads are in flight.
 DRT_DEV void sk_dims(uint32_t dims0, uint32_t dims1, int& M, int& N, int& K, int& KS, int& n_xcc,
-                     int& fenced, int& rot) {
+                     int& fenced) {
   N = (int)(dims0 & 0xffffu);
   K = (int)(dims0 >> 16);
   M = (int)(dims1 & 0xffu);
   KS = (int)((dims1 >> 8) & 0xffu);
   n_xcc = (int)((dims1 >> 16) & 0xffu);
-  fenced = (int)((dims1 >> 24) & 1u);
-  rot = (int)(dims1 >> 25);
+  fenced = (int)(dims1 >> 24);
 }
 
 // PRE: the input is pre-scaled ACT_F16P planes (see FusedArgs::pre_out):
@@ -186,8 +192,8 @@ __global__ __launch_bounds__(256) void skinny_wide_kernel(
   constexpr bool BF = WK == W_BF16;
   static_assert(!PRE || !BF, "pre-scaled planes feed the q4 kernels only");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int M, N, K, KS, n_xcc, fenced, rot;
-  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced, rot);
+  int M, N, K, KS, n_xcc, fenced;
+  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced);
   // 32-row tile of this work-group: rows m0 .. m0 + M - 1 of the forward
   const int mt = blockIdx.y, m0 = 32 * mt, M_all = M;
   M = min(32, M_all - m0);
@@ -199,7 +205,7 @@ __global__ __launch_bounds__(256) void skinny_wide_kernel(
   int* counters = a.counters + (size_t)mt * a.n_counters;
   const int G = K >> 6;
   int grp, ks;
-  const bool live = sk_place(n_xcc, fenced, rot, perr, N / 128, KS, grp, ks);
+  const bool live = sk_place(n_xcc, N / 128, KS, grp, ks);
   const int nt = grp * 4 + wave;
   const int u0 = ks * U, kc0 = u0 * 64;
   // absolute position of row 0 (the q|k|v epilogue's rotary tables), read at
@@ -405,7 +411,10 @@ __global__ __launch_bounds__(256) void skinny_wide_kernel(
 #pragma unroll
     for (int jj = 0; jj < 4; ++jj)
       *(f32x4*)(pw + 256 * jj) = f32x4{acc[4 * jj], acc[4 * jj + 1], acc[4 * jj + 2], acc[4 * jj + 3]};
-    if (!last_to_arrive(&counters[grp], KS, flag, a.fenced)) return;
+    if (!last_to_arrive(&counters[grp], KS, flag, a.fenced)) {
+      sk_check(n_xcc, fenced, perr);
+      return;
+    }
     const float* pbase = part + (size_t)grp * KS * 4096;
     const bool rnd = BF && a.rnd_bf16;
     if (KS <= 2) sk_wide_sum_slices<2>(pbase, KS, red, rnd);
@@ -481,8 +490,8 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
   static_assert(XIN == 0 || WK == W_Q4, "fp32 / bf16 rows feed the q4 kernels only");
   constexpr bool BF = WK == W_BF16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int M, N, K, KS, n_xcc, fenced, rot;
-  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced, rot);
+  int M, N, K, KS, n_xcc, fenced;
+  sk_dims(dims0, dims1, M, N, K, KS, n_xcc, fenced);
   // 32-row tile of this work-group: rows m0 .. m0 + M - 1 of the forward
   const int mt = blockIdx.y, m0 = 32 * mt, M_all = M;
   M = min(32, M_all - m0);
@@ -491,7 +500,7 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
   const int G = K >> 6;
   const int U = G / KS;
   int nt, ks;
-  const bool live = sk_place(n_xcc, fenced, rot, perr, N / 32, KS, nt, ks);
+  const bool live = sk_place(n_xcc, N / 32, KS, nt, ks);
   const int u_lo = ks * U + (U * wave) / 4, u_hi = ks * U + (U * (wave + 1)) / 4;
   extern __shared__ __align__(16) char smem[];
   float* red = (float*)smem;  // [4][32][33]
@@ -655,7 +664,10 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
            red[(96 + m) * 33 + c0 + e];
   if (KS > 1) {
     *(f32x4*)(part + (size_t)(nt * KS + ks) * 1024 + m * 32 + c0) = v;
-    if (!last_to_arrive(&counters[nt], KS, flag, a.fenced)) return;
+    if (!last_to_arrive(&counters[nt], KS, flag, a.fenced)) {
+      sk_check(n_xcc, fenced, perr);
+      return;
+    }
     const float* pp = part + (size_t)nt * KS * 1024 + m * 32 + c0;
     f32x4 pv[SK_KS_MAX];
 #pragma unroll
@@ -766,9 +778,9 @@ __global__ __launch_bounds__(512) void skinny_gu_kernel(
   constexpr int K = G * 64, ROW = K + 8, CPR = G / 8, UPW = G / 8, RH = GU_RH;
   constexpr int RS = GU_RS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int M, N, Kd, KS, n_xcc, fenced, rot;
-  sk_dims(dims0, dims1, M, N, Kd, KS, n_xcc, fenced, rot);
-  (void)Kd, (void)KS, (void)n_xcc, (void)fenced, (void)rot, (void)perr;
+  int M, N, Kd, KS, n_xcc, fenced;
+  sk_dims(dims0, dims1, M, N, Kd, KS, n_xcc, fenced);
+  (void)Kd, (void)KS, (void)n_xcc, (void)fenced, (void)perr;
   // rows m0 .. m0 + M - 1 of the forward: half hr of 32-row tile mt
   const int mt = blockIdx.y >> 1, hr = blockIdx.y & 1, tr0 = RH * hr;
   const int m0 = 32 * mt + tr0, M_all = M;
@@ -1012,7 +1024,7 @@ bool skinny_supported(int kind, int N, int K) {
 namespace {
 uint32_t sk_dims1(const FusedArgs& a, int KS) {
   return (uint32_t)a.M | ((uint32_t)KS << 8) | ((uint32_t)a.n_xcc << 16) |
-         ((uint32_t)(a.fenced ? 1 : 0) << 24) | ((uint32_t)a.xcc_rot << 25);
+         ((uint32_t)(a.fenced ? 1 : 0) << 24);
 }
 }  // namespace
 
