@@ -48,11 +48,23 @@ extern "C" __global__ void round_bf16_bias_kernel(float* __restrict__ y, int64_t
   }
 }
 
-extern "C" __global__ void to_bf16_kernel(const float* __restrict__ x, uint16_t* __restrict__ o,
-                                          int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    o[i] = float_to_bf16_bits(x[i]);
+// eight values per thread; the last n % 8 one by one
+extern "C" __global__ __launch_bounds__(256) void to_bf16_kernel(const float* __restrict__ x,
+                                                                 uint16_t* __restrict__ o,
+                                                                 int64_t n) {
+  const int64_t i = (blockIdx.x * (int64_t)256 + threadIdx.x) * 8;
+  if (i + 8 <= n) {
+    const f32x4 a = *(const f32x4_e*)(x + i), b = *(const f32x4_e*)(x + i + 4);
+    uint16_t h[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = float_to_bf16_bits(a[e]);
+      h[4 + e] = float_to_bf16_bits(b[e]);
+    }
+    *(u32x4_e*)(o + i) = __builtin_bit_cast(u32x4, h);
+  } else {
+    for (int64_t j = i; j < n; ++j) o[j] = float_to_bf16_bits(x[j]);
+  }
 }
 
 namespace drt {
@@ -64,8 +76,7 @@ void round_bf16_inplace(float* y, int64_t n, const uint16_t* bias, int N, hipStr
 }
 
 void to_bf16(const float* x, uint16_t* o, int64_t n, hipStream_t s) {
-  const int blocks = (int)std::min<int64_t>((n + 255) / 256, 8192);
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks), dim3(256), 0, s, x, o, n);
+  hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)((n + 2047) / 2048)), dim3(256), 0, s, x, o, n);
   DRT_HIP(hipGetLastError());
 }
 

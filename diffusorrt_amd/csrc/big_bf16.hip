@@ -343,9 +343,10 @@ int bb_tiles(int t, int M, int N) {
 // only: each at least four stages, the slices within part_floats) and, unsplit, a
 // whole number of rounds of 256 x 256 tiles with the last columns on 128 x 128 ones
 // (a second launch: 1000 x 18944 x 3584, 296 large tiles on 256 CUs, 168 us all
-// large, 154 all small, 134 mixed). reduce_us: what a slice pass costs besides its bytes.
+// large, 154 all small). reduce_us: what a slice pass costs besides its bytes;
+// split_us: the least a split call can take (the host's part of a second launch).
 BigBf16Plan big_bf16_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
-                          float reduce_us) {
+                          float reduce_us, float split_us) {
   const int n_cu = n_cu_of_current_device(), G = K / 64;
   BigBf16Plan best;
   float best_us = 1e30f;
@@ -356,6 +357,7 @@ BigBf16Plan big_bf16_plan(int M, int N, int K, int kind, int max_ks, size_t part
       if (ks > 1 && (kind != FL_STORE || G / ks < 4 || (size_t)ks * M * N > part_floats)) break;
       float us = tile_cost(t, tiles * ks, (float)((G + ks - 1) / ks), n_cu);
       if (ks > 1) us += reduce_us + (ks + 1) * 4e-6f * M * N / 4.f;  // 4 TB/s
+      us = std::max(us, ks > 1 ? split_us : 0.f);
       if (us < best_us) {
         best_us = us;
         best = BigBf16Plan{t, ks, 0};
@@ -383,7 +385,7 @@ BigBf16Plan big_bf16_plan(int M, int N, int K, int kind, int max_ks, size_t part
 bool big_bf16_supported(const FusedArgs& a, int kind) {
   // (16-byte loads straight into LDS: aligned operands only)
   if ((((uintptr_t)a.wb | (uintptr_t)a.act) & 15) != 0) return false;
-  if (!a.wb || a.qw || !a.act || a.M <= 32 || a.N % 32 || a.K % 64 || a.K < 64) return false;
+  if (!a.wb || a.qw || !a.act || a.M < 1 || a.N % 32 || a.K % 64 || a.K < 64) return false;
   if (kind == FL_SWIGLU) return a.N % 128 == 0 && a.act_fmt == ACT_BF16;
   if (kind == FL_QKV) return a.N % 128 == 0;
   return kind == FL_STORE;

@@ -150,7 +150,7 @@ struct BigBf16Plan {
 };
 bool big_bf16_supported(const FusedArgs& a, int kind);
 BigBf16Plan big_bf16_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
-                          float reduce_us);
+                          float reduce_us, float split_us = 0.f);
 void big_bf16_linear(const FusedArgs& a, int kind, const BigBf16Plan& p, hipStream_t s);
 void big_bf16_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s);
 // q|k|v projection + epilogue: split-K into `part` (when the tiles alone would

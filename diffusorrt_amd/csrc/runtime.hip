@@ -2199,6 +2199,8 @@ static size_t q4_op_act_bytes(int32_t m, int32_t k) {
   return ((size_t)2 * m * k * 2 + (size_t)m * (k / 64) * 4 + 255) / 256 * 256;
 }
 
+constexpr int OP_COUNTER_BLOCKS = 32, OP_COUNTERS = 4096;  // (see op_counters)
+
 size_t drt_op_q4_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   if (m <= 0 || k <= 0) return 0;
   size_t b = q4_op_act_bytes(m, k) + 256;
@@ -2213,7 +2215,6 @@ size_t drt_op_q4_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
 // launch, one block of OP_COUNTERS per (device, stream) so that calls on
 // different streams never share one; the XCD placement is probed once per
 // device (on a stream of its own, synchronised once).
-constexpr int OP_COUNTER_BLOCKS = 32, OP_COUNTERS = 4096;
 static __device__ int op_counters[OP_COUNTER_BLOCKS * OP_COUNTERS];
 static __device__ int op_probe[256];
 namespace {
@@ -2434,12 +2435,96 @@ int32_t drt_op_bf16_repack(const void* w, int32_t n, int32_t k, void* wb, void* 
   });
 }
 
-constexpr float BB_OP_REDUCE_US = 4.f;  // the slice sum's own launch
-// (more than 32 rows: the split-K slices)
+// the slice sum's own launch, and the least time of a call that makes it
+constexpr float BB_OP_REDUCE_US = 4.f, BB_OP_SPLIT_US = 14.f;
+// bf16 linears of few rows or outputs. Up to 64 rows and 8M weights: the one-launch split-K
+// kernel, where it takes the shape (1024 x 3072, 32 fp32 rows: 14.8 us with a cast of its
+// own before, 10.7, the host's part of a call; a second launch costs it 4 us more), unless
+// bf16 rows need no cast and the next kernel takes them (its call's host part is 0.4 us
+// shorter: no counters to look up). Else the kernel that streams a 32 x 32 tile's whole K, one launch, where its tiles fit one
+// round of the CUs and K is short enough to end before a split GEMM and its sum would
+// (bf16 rows: 512 x 3584, 200 rows 10.6 against 13.7; 3584 x 3584, 2 rows 10.3, 64 rows 12.0
+// against 13.8; but two rounds, 96 rows, 22.0 against 15.2, and K = 8192, 32 rows, 20.3
+// against 13.3, 9 rows 12.1 against 13.3). Else the shared-operand GEMM (18944 x 3584: 2
+// rows 30.5 -> 26.3, 32 rows 58 -> 29; 3584 x 18944: 91 -> 29).
+constexpr int64_t BB_SKINNY_WEIGHTS = (int64_t)8 << 20;
+static bool bf16_op_streams(int32_t m, int32_t n, int32_t k) {
+  return (int64_t)(n / 32) * ((m + 31) / 32) <= n_cu_of_current_device() &&
+         k <= (m <= 8 ? 8192 : 4096);
+}
+static bool bf16_op_skinny(int32_t m, int32_t n, int32_t k) {
+  return m <= 32 * SK_ROW_TILES && n % 32 == 0 && k % 64 == 0 &&
+         n / 32 <= OP_COUNTERS / SK_ROW_TILES && (int64_t)n * k <= BB_SKINNY_WEIGHTS &&
+         skinny_supported(FL_STORE, n, k);
+}
+static size_t bf16_op_x_bytes(int32_t m, int32_t k) { return ((size_t)m * k * 2 + 255) / 256 * 256; }
+
+// the split-K slices, or the split-K kernel's partial tiles
 size_t drt_op_bf16_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
-  if (m <= 32 || n <= 0 || k <= 0 || n % 32 || k % 64) return 256;
-  const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, SIZE_MAX, BB_OP_REDUCE_US);
+  if (m <= 0 || n <= 0 || k <= 0 || n % 32 || k % 64) return 256;
+  if (bf16_op_skinny(m, n, k)) return skinny_part_floats(n, k) * 4 * SK_ROW_TILES;
+  if (bf16_op_streams(m, n, k)) return 256;
+  const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, SIZE_MAX, BB_OP_REDUCE_US,
+                                      BB_OP_SPLIT_US);
   return p.ks > 1 ? (size_t)p.ks * m * n * 4 : 256;
+}
+
+// ... and the rows rounded to bf16 for the kernels that do not do that themselves
+size_t drt_op_bf16_linear_x_workspace_bytes(int32_t m, int32_t n, int32_t k) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  return bf16_op_x_bytes(m, k) + drt_op_bf16_linear_workspace_bytes(m, n, k);
+}
+
+// x bf16, or with xb fp32 (rounded to bf16 into xb where no kernel does it on the way)
+static void bf16_linear_into(const void* wb, const void* x, void* xb, int32_t m, int32_t n, int32_t k,
+                             const void* bias, float* y, void* workspace, size_t workspace_bytes,
+                             hipStream_t st) {
+  FusedArgs f;
+  f.wb = (const uint16_t*)wb;
+  f.bias = (const uint16_t*)bias;
+  f.M = m;
+  f.N = n;
+  f.K = k;
+  f.act = x;
+  f.rnd_bf16 = 1;  // the bf16 matmul output is bf16; the bias is added after
+  f.y = y;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  DRT_HIP(hipStreamIsCapturing(st, &cap));
+  if (bf16_op_skinny(m, n, k) && (xb || !bf16_op_streams(m, n, k)) && workspace &&
+      workspace_bytes >= skinny_part_floats(n, k) * 4 * SK_ROW_TILES &&
+      cap == hipStreamCaptureStatusNone) {
+    // one launch, its counters this stream's (a graph's replays would share them)
+    FusedArgs g = f;
+    g.x_in = xb ? 1 : 0;
+    g.part = (float*)workspace;
+    g.part_floats = skinny_part_floats(n, k);
+    g.sk_row_tiles = SK_ROW_TILES;
+    bool fenced = false;
+    g.counters = op_counters_for(st, g.n_xcc, fenced);
+    g.n_counters = OP_COUNTERS / SK_ROW_TILES;
+    g.fenced = fenced ? 1 : 0;
+    if (g.counters && skinny_linear(g, FL_STORE, st)) return;
+  }
+  if (xb) {
+    to_bf16((const float*)x, (uint16_t*)xb, (int64_t)m * k, st);
+    f.act = xb;
+  }
+  if (bf16_op_streams(m, n, k) || !big_bf16_supported(f, FL_STORE)) {
+    fused_linear(f, FL_STORE, st);
+    return;
+  }
+  // as many slices as the caller's workspace holds (none is needed)
+  const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS,
+                                      workspace ? workspace_bytes / 4 : 0, BB_OP_REDUCE_US,
+                                      BB_OP_SPLIT_US);
+  if (p.ks > 1) {
+    float* part = (float*)workspace;
+    f.y = part;
+    big_bf16_linear(f, FL_STORE, p, st);
+    sum_slices(part, p.ks, (int64_t)m * n, (const uint16_t*)bias, n, y, st, true);
+  } else {
+    big_bf16_linear(f, FL_STORE, p, st);
+  }
 }
 
 int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, int32_t k,
@@ -2448,31 +2533,22 @@ int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, 
   return guarded([&] {
     require(wb && x && y && m > 0 && n > 0 && k > 0, "bad bf16_linear arguments");
     require(n % 32 == 0 && k % 16 == 0, "bf16_linear needs n % 32 == 0 and k % 16 == 0");
-    FusedArgs f;
-    f.wb = (const uint16_t*)wb;
-    f.bias = (const uint16_t*)bias;
-    f.M = m;
-    f.N = n;
-    f.K = k;
-    f.act = x;
-    f.rnd_bf16 = 1;  // the bf16 matmul output is bf16; the bias is added after
-    f.y = y;
-    hipStream_t st = as_stream(stream);
-    if (!big_bf16_supported(f, FL_STORE)) {
-      fused_linear(f, FL_STORE, st);
-      return;
-    }
-    // as many slices as the caller's workspace holds (none is needed)
-    const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS,
-                                        workspace ? workspace_bytes / 4 : 0, BB_OP_REDUCE_US);
-    if (p.ks > 1) {
-      float* part = (float*)workspace;
-      f.y = part;
-      big_bf16_linear(f, FL_STORE, p, st);
-      sum_slices(part, p.ks, (int64_t)m * n, (const uint16_t*)bias, n, y, st, true);
-    } else {
-      big_bf16_linear(f, FL_STORE, p, st);
-    }
+    bf16_linear_into(wb, x, nullptr, m, n, k, bias, y, workspace, workspace_bytes, as_stream(stream));
+  });
+}
+
+int32_t drt_op_bf16_linear_x(const void* wb, const void* x, int32_t x_dtype, int32_t m, int32_t n,
+                             int32_t k, const void* bias, float* y, void* workspace,
+                             size_t workspace_bytes, void* stream) {
+  return guarded([&] {
+    require(wb && x && y && m > 0 && n > 0 && k > 0, "bad bf16_linear arguments");
+    require(n % 32 == 0 && k % 16 == 0, "bf16_linear needs n % 32 == 0 and k % 16 == 0");
+    require(x_dtype == DRT_F32 || x_dtype == DRT_BF16, "bf16_linear x must be F32 or BF16");
+    require(workspace && workspace_bytes >= drt_op_bf16_linear_x_workspace_bytes(m, n, k),
+            "bf16_linear workspace too small");
+    const size_t xb = bf16_op_x_bytes(m, k);
+    bf16_linear_into(wb, x, x_dtype == DRT_F32 ? workspace : nullptr, m, n, k, bias, y,
+                     (char*)workspace + xb, workspace_bytes - xb, as_stream(stream));
   });
 }
 

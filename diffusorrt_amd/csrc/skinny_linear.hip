@@ -481,13 +481,14 @@ __global__ __launch_bounds__(256) void skinny_wide_kernel(
 // in chunks of UW, each chunk's loads issued together).
 // XIN: the activation's format. 0: ACT_F16P (hi plane, lo plane at + M * K);
 // 1: fp32 rows [M][K] and 2: bf16 rows (a per-op call's input), split into the
-// hi and lo planes in registers on the way to LDS (no preparation pass).
+// hi and lo planes (bf16 weights, fp32 rows: rounded to bf16) in registers on the
+// way to LDS (no preparation pass).
 template <int WK, int EPI, int UW, int XIN>
 __global__ __launch_bounds__(256) void skinny_narrow_kernel(
     const uint32_t* __restrict__ qw, const uint32_t* __restrict__ sbp,
     const uint16_t* __restrict__ act, int* perr, uint32_t dims0, uint32_t dims1,
     const FusedArgs a) {
-  static_assert(XIN == 0 || WK == W_Q4, "fp32 / bf16 rows feed the q4 kernels only");
+  static_assert(XIN != 2 || WK == W_Q4, "bf16 rows are what the bf16 kernels take as they are");
   constexpr bool BF = WK == W_BF16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int M, N, K, KS, n_xcc, fenced;
@@ -589,6 +590,15 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
             if (XIN == 1) v[e] = xr[XIN == 1 ? i : 0][j][e >> 2][e & 3];
             else v[e] = bf16_bits_to_float(e & 1 ? craw[i][j][e >> 1] >> 16
                                                   : craw[i][j][e >> 1] & 0xffffu);
+          }
+          if (BF) {
+            u32x4 bp;
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+              bp[w] = (uint32_t)float_to_bf16_bits(v[2 * w]) |
+                      ((uint32_t)float_to_bf16_bits(v[2 * w + 1]) << 16);
+            craw[i][j] = bp;
+            continue;
           }
           u32x4 hp, lp;
 #pragma unroll
@@ -948,6 +958,7 @@ DRT_NARROW(W_BF16, EPI_RESID, 1) DRT_NARROW(W_BF16, EPI_RESID, 2)
 DRT_NARROW(W_BF16, EPI_STORE, 1) DRT_NARROW(W_BF16, EPI_STORE, 2)
 DRT_NARROW_X(W_Q4, EPI_STORE, 1, 1) DRT_NARROW_X(W_Q4, EPI_STORE, 2, 1)
 DRT_NARROW_X(W_Q4, EPI_STORE, 1, 2) DRT_NARROW_X(W_Q4, EPI_STORE, 2, 2)
+DRT_NARROW_X(W_BF16, EPI_STORE, 1, 1) DRT_NARROW_X(W_BF16, EPI_STORE, 2, 1)
 #undef DRT_NARROW_X
 #undef DRT_NARROW
 
@@ -1143,8 +1154,10 @@ static bool skinny_launch(const FusedArgs& a, int kind, hipStream_t s) {
     // two-unit staging holds one), so they run in one round instead of two.
     const bool one_unit = per_wave <= 1 || MT > 1;
     if (a.x_in != 0) {
-      if (kind != FL_STORE || bf) return false;
-      if (a.x_in == 1) {
+      if (kind != FL_STORE || (bf && a.x_in != 1)) return false;
+      if (bf) {
+        if (one_unit) DRT_SN1X(W_BF16, EPI_STORE, 1, 1) else DRT_SN1X(W_BF16, EPI_STORE, 2, 1)
+      } else if (a.x_in == 1) {
         if (one_unit) DRT_SN1X(W_Q4, EPI_STORE, 1, 1) else DRT_SN1X(W_Q4, EPI_STORE, 2, 1)
       } else {
         if (one_unit) DRT_SN1X(W_Q4, EPI_STORE, 1, 2) else DRT_SN1X(W_Q4, EPI_STORE, 2, 2)

@@ -246,6 +246,11 @@ size_t drt_op_bf16_linear_workspace_bytes(int32_t m, int32_t n, int32_t k);
 int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, int32_t k,
                            const void* bias, float* y, void* workspace, size_t workspace_bytes,
                            void* stream);
+/* The same of fp32 or bf16 rows (x_dtype): fp32 rows are rounded to bf16 on the way. */
+size_t drt_op_bf16_linear_x_workspace_bytes(int32_t m, int32_t n, int32_t k);
+int32_t drt_op_bf16_linear_x(const void* wb, const void* x, int32_t x_dtype, int32_t m, int32_t n,
+                             int32_t k, const void* bias, float* y, void* workspace,
+                             size_t workspace_bytes, void* stream);
 /* Write K/V rows ([n, hkv, 128] fp32 or bf16) into a tiled cache of one layer at
  * positions pos0..pos0+n-1. cache holds hkv * head_stride elements of kv_dtype. */
 int32_t drt_op_kv_pack(const void* k, const void* v, int32_t src_dtype, int32_t n, int32_t hkv,

@@ -165,27 +165,34 @@ def test_bf16_linear(m, n, k):
     assert rel < 1e-2
 
 
-# The large-M bf16 kernels: row and column remainders of every tile (64, 128, 256),
-# fewer 64-k stages than stage buffers, split K, whole rounds of 256 x 256 tiles with
-# the last columns on 128 x 128 ones (520 x 22400 on 256 CUs), and a K that is not
-# whole stages (the general kernel).
+# The bf16 kernels of a per-op call: the one-launch kernel (fp32 rows rounded on the way;
+# one and two units per wave, K slices, one and two row tiles), the streaming kernel (bf16
+# rows, and where that takes no such shape), the GEMM's 64-row tile for large weights;
+# then the large-M ones: row and column remainders of every tile (64, 128, 256), fewer
+# 64-k stages than stage buffers, split K, whole rounds of 256 x 256 tiles with the last
+# columns on 128 x 128 ones (520 x 22400 on 256 CUs), and a K that is not whole stages
+# (the general kernel). Each with fp32 rows and, the same values, with bf16 ones.
 @pytest.mark.parametrize("m,n,k,with_ws", [
-    (33, 32, 64, True), (64, 160, 128, True), (65, 992, 192, True), (129, 1024, 3072, True),
-    (129, 1024, 3072, False), (257, 4064, 1024, True), (520, 22400, 1024, True),
+    (1, 32, 64, True), (31, 1024, 1024, True), (32, 96, 3072, True), (32, 96, 3072, False),
+    (5, 512, 3584, True), (9, 3584, 3584, True), (3, 18944, 3584, True),
+    (33, 32, 64, True), (48, 1024, 2048, True), (64, 160, 128, True), (64, 3072, 1024, False),
+    (200, 512, 3584, True), (9, 512, 8192, True), (65, 4064, 64, True), (100, 2720, 192, True),
+    (300, 1024, 3072, True), (300, 1024, 3072, False), (257, 4064, 1024, True), (520, 22400, 1024, True),
     (70, 256, 80, True)])
-def test_bf16_linear_large_m(m, n, k, with_ws):
+def test_bf16_linear_kernels(m, n, k, with_ws):
     import ctypes as C
 
     from diffusorrt_amd import _lib, kernels
 
-    _say("bf16_linear large M", m, n, k, "workspace" if with_ws else "no workspace")
+    _say("bf16_linear", m, n, k, "workspace" if with_ws else "no workspace")
     gen = torch.Generator().manual_seed(12)
     wt = (torch.randn((n, k), generator=gen) * 0.02).to(torch.bfloat16)
     bias = torch.randn((n,), generator=gen).to(torch.bfloat16)
     x = torch.randn((m, k), generator=gen)
     w = kernels.DeviceBF16Weight(wt.cuda())
     if with_ws:
-        y = kernels.linear(x.cuda(), w, bias.cuda())
+        ys = [kernels.linear(x.cuda(), w, bias.cuda()),
+              kernels.linear(x.to(torch.bfloat16).cuda(), w, bias.cuda())]
     else:  # the entry point needs no workspace: it then does not split K
         xb, bd = x.to(torch.bfloat16).cuda(), bias.cuda()
         y = torch.empty((m, n), device="cuda")
@@ -193,15 +200,17 @@ def test_bf16_linear_large_m(m, n, k, with_ws):
             C.c_void_p(w.wb.data_ptr()), C.c_void_p(xb.data_ptr()), m, n, k,
             C.c_void_p(bd.data_ptr()), C.c_void_p(y.data_ptr()), None, 0,
             C.c_void_p(torch.cuda.current_stream().cuda_stream)))
-    y = y.cpu().numpy().astype(np.float64)
+        ys = [y]
     exact = x.to(torch.bfloat16).double().numpy() @ wt.double().numpy().T
-    err = np.abs((y - bias.double().numpy()) - exact)
     # half a bf16 ulp of the product (2^-8 of it), the fp32 sums' own error ahead of the
     # rounding, and the fp32 addition of the bias
     mag = np.abs(x.to(torch.bfloat16).double().numpy()) @ np.abs(wt.double().numpy()).T
-    bound = np.abs(exact) * 2.0 ** -8 + mag * k * 2.0 ** -24 + 2.0 ** -22 * (1 + np.abs(y))
-    _say(f"  worst error / bound {np.max(err / bound):.3f}")
-    assert (err <= bound).all()
+    for y in ys:
+        y = y.cpu().numpy().astype(np.float64)
+        err = np.abs((y - bias.double().numpy()) - exact)
+        bound = np.abs(exact) * 2.0 ** -8 + mag * k * 2.0 ** -24 + 2.0 ** -22 * (1 + np.abs(y))
+        _say(f"  worst error / bound {np.max(err / bound):.3f}")
+        assert (err <= bound).all()
 
 
 # The large-M q4 kernels: both tiles, unsplit and split, the split last round beside one
