@@ -110,7 +110,7 @@ DRT_DEV void store_attn8(const f32x4 v0, const f32x4 v1, int row, int n_rows, in
 
 // Long-query attention: a wave owns one 32-vector query tile, the QW waves of a
 // key group share 32-key K/V tiles, streamed by direct-to-LDS loads into a ring of
-// three 16 KiB slots (tile t + 2 is issued once tile t has arrived and every wave is
+// three slots of 16 KiB per key group (tile t + 2 is issued once tile t has arrived and every wave is
 // done with t - 1: one barrier per tile, no registers held by the loads). Two or three
 // waves per SIMD overlap one's softmax (VALU) with another's products (MFMA): either
 // alone takes about as long as the other. The
@@ -121,7 +121,10 @@ DRT_DEV void store_attn8(const f32x4 v0, const f32x4 v1, int row, int n_rows, in
 // OUT: a single split writes the attention itself (out_fmt as in
 // attn_combine_kernel) instead of a partial for the combine.
 // KG: key groups of a work-group, each with its own QW waves over a contiguous share of
-// the keys; their parts meet in LDS at the end.
+// the keys; their parts meet in LDS at the end. Four groups of two query tiles (two slots,
+// so one iteration of prefetch) put twice the work-groups on the chip where two groups of
+// four leave CUs idle: 1000 x 16 heads over 1000 keys, 256 work-groups instead of 128, 24.2
+// -> 18.0 us.
 // 2048 rows x 16 heads over 4096 keys, bf16: 135 -> 77 us with the combine (671 TFLOP/s; K/V
 // staged through registers, products with a zero lo plane, a mask test per score before).
 template <typename T, int QW, int KG, bool LO, bool OUT>
@@ -154,7 +157,8 @@ DRT_DEV void attn_split_tile(
   constexpr int SLOT = KG * TILE_BYTES;
   __shared__ __align__(1024) char ring0[SLOT];
   __shared__ __align__(1024) char ring1[SLOT];
-  __shared__ __align__(1024) char ring2[SLOT];
+  constexpr int SLOTS = KG > 2 ? 2 : 3;  // (three of 64 KiB would not fit)
+  __shared__ __align__(1024) char ring2[SLOTS > 2 ? SLOT : 16];
   __shared__ float2 ml[KG > 1 ? KG * QW * 32 : 1];
 
   // This lane's query (B operand of S^T) and its absolute position.
@@ -257,25 +261,28 @@ DRT_DEV void attn_split_tile(
     }
     l_run += psum;
   };
-  // iteration it in slot it % 3; at most one later slot's loads are in flight while its
-  // own are awaited
-  auto step = [&](int it, char* here, char* two_on) {
-    if (it + 1 < n_it) __builtin_amdgcn_s_waitcnt(0x0F70 | LD);  // vmcnt(LD): its tile is here
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
+  // iteration it in slot it % SLOTS; with three slots one later slot's loads are in flight
+  // while its own are awaited
+  auto step = [&](int it, char* here, char* freed) {
+    if (SLOTS > 2 && it + 1 < n_it)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | LD);  // vmcnt(LD): its tile is here
+    else
+      __builtin_amdgcn_s_waitcnt(0x0F70);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (it + 2 < n_it) issue(it + 2, two_on);
+    if (it + SLOTS - 1 < n_it) issue(it + SLOTS - 1, freed);
     compute(it, here);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave is done reading the slot
   };
   if (n_it > 0) issue(0, ring0);
-  if (n_it > 1) issue(1, ring1);
+  if (SLOTS > 2 && n_it > 1) issue(1, ring1);
   asm volatile("" ::: "memory");
-  for (int it = 0; it < n_it; it += 3) {
-    step(it, ring0, ring2);
+  for (int it = 0; it < n_it; it += SLOTS) {
+    step(it, ring0, SLOTS > 2 ? ring2 : ring1);
     if (it + 1 >= n_it) break;
     step(it + 1, ring1, ring0);
+    if (SLOTS < 3) continue;
     if (it + 2 >= n_it) break;
     step(it + 2, ring2, ring1);
   }
@@ -1073,18 +1080,28 @@ AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, int mask_kind,
   const int wgs = Hkv * p.qgroups;
   int splits = 1;
   if (mask_kind == 1) {
-    // one iteration over two tiles takes about 1.1 us, a split adds the combine's 8 us
-    // and its partials' bytes (1000 x 1000 keys: 24 us unsplit, 29 with two; 100 x 4100:
-    // 68 and 23 with eight)
+    // one iteration over two tiles takes about 1.1 us, over four (of half the queries)
+    // 1.3, a split adds the combine's 8 us and its partials' bytes (two groups, 1000 x 1000
+    // keys: 24 us unsplit, 29 with two; 100 x 4100: 68 and 23 with eight; four groups: 18
+    // and, with five, 21; 500 x 500 17.4 -> 14.1, 1000 x 4000 56 -> 48, 1000 x 8000 91 -> 89)
     p.kg = wgs > 256 ? 1 : 2;
-    const float iters = (float)((n_tiles + 1) / 2), part_us = (float)n_rows * Hq * 1024.f / 4e6f;
-    float best = 1.1f * iters;
-    for (int sp = 2; sp <= std::min({256 / wgs, (n_tiles + 1) / 2, 64}); ++sp) {
-      const float us = 1.1f * std::ceil(iters / sp) + 8.f + part_us * sp;  // (the combine reads <= 64)
-      if (us < best) {
-        best = us;
-        splits = sp;
+    const int wgs2 = Hkv * ((qtiles + 1) / 2);
+    const float part_us = (float)n_rows * Hq * 1024.f / 4e6f;
+    float best = 1e30f;
+    for (int kg = p.kg; kg <= (wgs2 <= 256 ? 4 : p.kg); kg += 2) {
+      const float iters = (float)((n_tiles + kg - 1) / kg), it_us = kg > 2 ? 1.3f : 1.1f;
+      for (int sp = 1; sp <= std::max(1, std::min({256 / (kg > 2 ? wgs2 : wgs), (int)iters, 64})); ++sp) {
+        const float us = it_us * std::ceil(iters / sp) + (sp > 1 ? 8.f + part_us * sp : 0.f);
+        if (us < best) {  // (the combine reads <= 64)
+          best = us;
+          splits = sp;
+          p.kg = kg;
+        }
       }
+    }
+    if (p.kg > 2) {
+      p.qw = 2;
+      p.qgroups = (qtiles + 1) / 2;
     }
     splits *= p.kg;
   } else {
@@ -1143,6 +1160,7 @@ void attention(bool bf16, const void* q, const void* kv_layer, int64_t kv_head_s
 #define DRT_ATTN(T)                                                                             \
   {                                                                                             \
     if (plan.qw == 2 && plan.kg == 1) DRT_ATTN3(T, 2, 1)                                        \
+    else if (plan.kg == 4) DRT_ATTN3(T, 2, 4)                                                   \
     else if (plan.qw == 2) DRT_ATTN3(T, 2, 2)                                                   \
     else if (plan.kg == 1) DRT_ATTN3(T, 4, 1)                                                   \
     else DRT_ATTN3(T, 4, 2)                                                                     \

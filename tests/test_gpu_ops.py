@@ -341,6 +341,8 @@ def test_block_attention_many_key_ranges(hq, hkv):
                                               ("d2f_hybrid", 97, 31, 128),
                                               ("bidirectional", 65, 0, 65),
                                               ("d2f_hybrid", 128, 4000, 4128),
+                                              ("d2f_hybrid", 160, 0, 160),
+                                              ("d2f_hybrid", 300, 0, 300),
                                               ("d2f_hybrid", 1000, 24, 1024),
                                               ("d2f_hybrid", 2100, 0, 2100),
                                               ("d2f_hybrid", 32, 8192, 8224),
