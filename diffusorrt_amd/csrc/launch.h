@@ -181,6 +181,7 @@ struct AttnPlan {
 AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, int mask_kind,
                         size_t part_budget_bytes);
 size_t attention_part_bytes(const AttnPlan& p, int n_rows, int Hq, int Hkv);
+size_t attention_part_bytes_max(int n_rows, int Hq, int Hkv, int n_keys, size_t part_budget_bytes);
 void attention(bool bf16, const void* q, const void* kv_layer, int64_t kv_head_stride,
                int n_rows, int Hq, int Hkv, int n_keys, int row_pos0, int mask_kind,
                int mask_prompt_len, int mask_block, const AttnPlan& plan, float* o_part,

@@ -2568,11 +2568,7 @@ int32_t drt_op_kv_pack(const void* k, const void* v, int32_t src_dtype, int32_t 
 
 size_t drt_op_attention_workspace_bytes(int32_t rows, int32_t hq, int32_t hkv, int32_t n_keys) {
   if (rows <= 0 || hq <= 0 || hkv <= 0 || hq % hkv || n_keys <= 0) return 0;
-  size_t general = 0;  // of either mask kind
-  for (int mask = 0; mask < 2; ++mask)
-    general = std::max(general, attention_part_bytes(plan_attention(rows, hq, hkv, n_keys, mask,
-                                                                    (size_t)256 << 20),
-                                                     rows, hq, hkv));
+  const size_t general = attention_part_bytes_max(rows, hq, hkv, n_keys, (size_t)256 << 20);
   const size_t decode = attention_decode_part_bytes(attention_decode_ranges(n_keys, hkv), hkv, rows * (hq / hkv));
   // + the kernels' Q operand: the caller's Q as the hi plane and a zero lo plane
   const size_t q_planes = ((size_t)2 * rows * hq * 128 * 2 + 255) / 256 * 256;
