@@ -118,6 +118,10 @@ DRT_DEV void store_attn8(const f32x4 v0, const f32x4 v1, int row, int n_rows, in
 // score: the scale is folded into the exponent's fma and the mask is tested only in
 // tiles that not every row of the wave sees whole. LO: Q has a lo plane (without it
 // the products with it are left out).
+// MASK: the d2f_hybrid mask. Without one the scores are scaled ahead of the max, one
+// rounding and 16 multiplies a tile more: the probabilities of a canvas stay those it always
+// had, and with them the token of a row whose two best logits are all but equal (one of a few
+// thousand rows otherwise).
 // OUT: a single split writes the attention itself (out_fmt as in
 // attn_combine_kernel) instead of a partial for the combine.
 // KG: key groups of a work-group, each with its own QW waves over a contiguous share of
@@ -127,14 +131,14 @@ DRT_DEV void store_attn8(const f32x4 v0, const f32x4 v1, int row, int n_rows, in
 // -> 18.0 us.
 // 2048 rows x 16 heads over 4096 keys, bf16: 135 -> 77 us with the combine (671 TFLOP/s; K/V
 // staged through registers, products with a zero lo plane, a mask test per score before).
-template <typename T, int QW, int KG, bool LO, bool OUT>
+template <typename T, int QW, int KG, bool LO, bool OUT, bool MASK>
 DRT_DEV void attn_split_tile(
     const T* __restrict__ q,       // [n_rows][Hq][128]
     const T* __restrict__ q_lo,    // its lo plane (the same layout; LO)
     const T* __restrict__ kv,      // this layer: [Hkv][tile_cap][8192]
     int64_t kv_head_stride,        // elements between kv heads
     int n_rows, int Hq, int Hkv, int n_keys, int row_pos0,
-    int mask_kind, int mask_prompt_len, int mask_block, int tiles_per_split,
+    int mask_prompt_len, int mask_block, int tiles_per_split,
     float* __restrict__ o_part,    // [splits][Hkv][n_qv][128]
     float* __restrict__ ml_part,   // [splits][Hkv][n_qv][2]
     float scale, const AttnOut& ao) {
@@ -175,12 +179,13 @@ DRT_DEV void attn_split_tile(
       if (LO) qfl[LO ? i : 0] = *(const vec*)(q_lo + qo + 16 * i);
     }
   }
-  const float c = scale * 1.44269504088896340736f;  // scores to base-2 exponents
+  const float cs = scale * 1.44269504088896340736f;  // scores to base-2 exponents
+  const float c = MASK ? cs : 1.f;  // (an fma by one subtracts the base)
   // d2f_hybrid: a query sees exactly the keys before the end of its own block
   // (the whole prompt, then whole blocks up to its own), so visibility is one
   // compare per key against the row's end, which never falls from row to row.
   auto key_end = [&](int row) {
-    if (mask_kind != 1) return n_keys;
+    if (!MASK) return n_keys;
     const int e = eff_block(row_pos0 + row, mask_prompt_len, mask_block);
     return min(n_keys, e < 0 ? mask_prompt_len : mask_prompt_len + (e + 1) * mask_block);
   };
@@ -192,7 +197,7 @@ DRT_DEV void attn_split_tile(
   const int wg_end = key_end(min(n_rows - 1, ((int)blockIdx.y * QW * 32 + QW * 32 - 1) / G));
   const int t_stop = min(t_end, (wg_end + 31) >> 5);
   // this key group's tiles: a contiguous share of the split's (masked) range
-  const int per = mask_kind == 1 ? (max(0, t_stop - t_begin) + KG - 1) / KG : tiles_per_split / KG;
+  const int per = MASK ? (max(0, t_stop - t_begin) + KG - 1) / KG : tiles_per_split / KG;
   const int kt0 = t_begin + kg * per, kt1 = min(t_stop, kt0 + per);
   const int n_it = min(per, t_stop - t_begin);  // iterations (every group's)
 
@@ -223,6 +228,10 @@ DRT_DEV void attn_split_tile(
       const vec kf = *(const vec*)(kt + (i * 64 + lane) * 8);
       s = MfmaT<T>::mma(kf, qf[i], s);
       if (LO) s = MfmaT<T>::mma(kf, qfl[LO ? i : 0], s);
+    }
+    if (!MASK) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] *= cs;
     }
     if (key0 + 32 > wave_full) {
 #pragma unroll
@@ -355,15 +364,15 @@ DRT_DEV void attn_split_tile(
 }
 
 // (the buffer resource type is not known to the host pass: the body is a device function)
-template <typename T, int QW, int KG, bool LO, bool OUT>
+template <typename T, int QW, int KG, bool LO, bool OUT, bool MASK>
 __global__ __launch_bounds__(64 * QW * KG, QW * KG == 2 ? 1 : KG == 1 ? 3 : QW == 4 ? 2 : 1) void attn_split_kernel(
     const T* __restrict__ q, const T* __restrict__ q_lo, const T* __restrict__ kv,
-    int64_t kv_head_stride, int n_rows, int Hq, int Hkv, int n_keys, int row_pos0, int mask_kind,
+    int64_t kv_head_stride, int n_rows, int Hq, int Hkv, int n_keys, int row_pos0,
     int mask_prompt_len, int mask_block, int tiles_per_split, float* __restrict__ o_part,
     float* __restrict__ ml_part, float scale, const AttnOut ao) {
-  attn_split_tile<T, QW, KG, LO, OUT>(q, q_lo, kv, kv_head_stride, n_rows, Hq, Hkv, n_keys, row_pos0,
-                                  mask_kind, mask_prompt_len, mask_block, tiles_per_split, o_part,
-                                  ml_part, scale, ao);
+  attn_split_tile<T, QW, KG, LO, OUT, MASK>(q, q_lo, kv, kv_head_stride, n_rows, Hq, Hkv, n_keys,
+                                            row_pos0, mask_prompt_len, mask_block, tiles_per_split,
+                                            o_part, ml_part, scale, ao);
 }
 
 // Decode attention: rows of one mask segment (every key in [0, n_keys) is
@@ -1106,12 +1115,12 @@ AttnPlan plan_attention(int n_rows, int Hq, int Hkv, int n_keys, int mask_kind,
     splits *= p.kg;
   } else {
     // every row sees every key: as many equal key ranges as fill the chip with one
-    // work-group each (two for long key ranges), neighbouring pairs of them in one
-    // work-group (the ranges, and with them the rounding of the probabilities, are
-    // those of separate work-groups)
+    // work-group each (two for long key ranges); two of them in one work-group, which adds
+    // them in the order and with the roundings of the combine (a canvas of 512 tokens: one
+    // launch less per layer). More would be added in pairs first, other sums.
     splits = std::max(1, (n_tiles <= 64 ? 256 : 512) / wgs);
     splits = std::min({splits, n_tiles, 64});
-    p.kg = splits % 2 == 0 ? 2 : 1;
+    p.kg = splits == 2 ? 2 : 1;
   }
   // keep the fp32 partials within budget
   const size_t per_split = (size_t)Hkv * n_rows * G * 130 * 4;
@@ -1154,31 +1163,37 @@ void attention(bool bf16, const void* q, const void* kv_layer, int64_t kv_head_s
   const AttnOut ao{out, xsum, err, out_fmt};
   // algorithmic bytes of this launch: Q read + the K/V of n_keys keys
   const double bytes = 2.0 * n_rows * Hq * 128 + 4.0 * n_keys * Hkv * 128;
-#define DRT_ATTN4(T, QW, KG, LO, OUT)                                                           \
-  DRT_LAUNCH(Profiler::ATTN, bytes, (attn_split_kernel<T, QW, KG, LO, OUT>), grid, block, 0, s, \
-             (const T*)q, LO ? (const T*)q + (int64_t)n_rows * Hq * 128 : (const T*)nullptr,    \
-             (const T*)kv_layer, kv_head_stride, n_rows, Hq, Hkv, n_keys, row_pos0, mask_kind,  \
+#define DRT_ATTN4(T, QW, KG, LO, OUT, MASK)                                                     \
+  DRT_LAUNCH(Profiler::ATTN, bytes, (attn_split_kernel<T, QW, KG, LO, OUT, MASK>), grid, block, \
+             0, s, (const T*)q, LO ? (const T*)q + (int64_t)n_rows * Hq * 128 : (const T*)nullptr, \
+             (const T*)kv_layer, kv_head_stride, n_rows, Hq, Hkv, n_keys, row_pos0,             \
              mask_prompt_len, mask_block, plan.tiles_per_split, o_part, ml_part, scale, ao)
-#define DRT_ATTN3(T, QW, KG)                                                                    \
+#define DRT_ATTN3(T, QW, KG, MASK)                                                              \
   {                                                                                             \
     if (q_has_lo) {                                                                             \
-      if (plan.splits == 1) DRT_ATTN4(T, QW, KG, true, true);                                   \
-      else DRT_ATTN4(T, QW, KG, true, false);                                                   \
+      if (plan.splits == 1) DRT_ATTN4(T, QW, KG, true, true, MASK);                             \
+      else DRT_ATTN4(T, QW, KG, true, false, MASK);                                             \
     } else {                                                                                    \
-      if (plan.splits == 1) DRT_ATTN4(T, QW, KG, false, true);                                  \
-      else DRT_ATTN4(T, QW, KG, false, false);                                                  \
+      if (plan.splits == 1) DRT_ATTN4(T, QW, KG, false, true, MASK);                            \
+      else DRT_ATTN4(T, QW, KG, false, false, MASK);                                            \
     }                                                                                           \
+  }
+#define DRT_ATTN2(T, MASK)                                                                      \
+  {                                                                                             \
+    if (plan.qw == 2 && plan.kg == 1) DRT_ATTN3(T, 2, 1, MASK)                                  \
+    else if (plan.qw == 2) DRT_ATTN3(T, 2, 2, MASK)                                             \
+    else if (plan.kg == 1) DRT_ATTN3(T, 4, 1, MASK)                                             \
+    else DRT_ATTN3(T, 4, 2, MASK)                                                               \
   }
 #define DRT_ATTN(T)                                                                             \
   {                                                                                             \
-    if (plan.qw == 2 && plan.kg == 1) DRT_ATTN3(T, 2, 1)                                        \
-    else if (plan.kg == 4) DRT_ATTN3(T, 2, 4)                                                   \
-    else if (plan.qw == 2) DRT_ATTN3(T, 2, 2)                                                   \
-    else if (plan.kg == 1) DRT_ATTN3(T, 4, 1)                                                   \
-    else DRT_ATTN3(T, 4, 2)                                                                     \
+    if (mask_kind != 1) DRT_ATTN2(T, false)                                                     \
+    else if (plan.kg == 4) DRT_ATTN3(T, 2, 4, true)                                             \
+    else DRT_ATTN2(T, true)                                                                     \
   }
   if (bf16) DRT_ATTN(__bf16) else DRT_ATTN(_Float16)
 #undef DRT_ATTN
+#undef DRT_ATTN2
 #undef DRT_ATTN3
 #undef DRT_ATTN4
   DRT_HIP(hipGetLastError());

@@ -151,6 +151,11 @@ struct Runtime {
   bool streaming = false;
   int sk_n_counters = 0;
   int n_xcc = 1;
+  // The gate|up projection of large q4 forwards splits its last round along K: where the
+  // stream's work-group 0 ran on XCD 0 at creation (a process with one hardware queue).
+  // Elsewhere such forwards always ran without it, and the split would change their sums
+  // and with them a token now and then (see big_q4_forward_plan).
+  bool split_last = false;
   bool fenced = false;           // split-K exchange through device-scope fences (no placement assumed)
   // scratch of the placement's probe, and whether it was probed (not overridden)
   DevBuf xcc_probe;
@@ -490,7 +495,11 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
       }
       // the gate|up projection's split last round shares the workspace (it runs
       // between the q|k|v and down projections, which use it too)
-      bf = std::max(bf, (size_t)n_cu_of_current_device() * 128 * 256);
+      for (int mt = 1; mt <= (M + 127) / 128; ++mt) {
+        const BigQ4Plan p =
+            big_q4_forward_plan(std::min(M, mt * 128), 2 * F, d, FL_SWIGLU, 1, SIZE_MAX, true);
+        bf = std::max(bf, (size_t)(mt * ((2 * F + 255) / 256) - p.full) * p.kt * 128 * 256);
+      }
       rt->big_part_floats = bf;
       rt->big_part.alloc(bf * 4);
       rt->big_tail_count.alloc((size_t)BIG_TAIL_COUNTERS * 4);
@@ -513,10 +522,15 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
       rt->n_xcc = atoi(nx_env);
     } else {
       rt->xcc_probe.alloc(256 * sizeof(int));
-      rt->fenced = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s) < 0;
+      const int rot = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s);
+      rt->fenced = rot < 0;
       rt->xcc_probed = true;
+      rt->split_last = rot == 0 && rt->n_xcc == 8;
     }
-    if (getenv("DRT_SPLITK_FENCED") != nullptr) rt->fenced = true;
+    if (getenv("DRT_SPLITK_FENCED") != nullptr) {
+      rt->fenced = true;
+      rt->split_last = false;
+    }
     rt->placement_err.alloc(8);
     DRT_HIP(hipMemsetAsync(rt->placement_err.p, 0, 8, s));
     DRT_HIP(hipHostMalloc((void**)&rt->placement_host, 4, hipHostMallocCoherent));
@@ -788,7 +802,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       big_bf16_linear(f, FL_STORE, bp, s);
       return bp.ks;
     }
-    const BigQ4Plan bp = big_q4_plan(M, f.N, f.K, FL_STORE, max_ks, rt.big_part_floats, 0.f, false);
+    const BigQ4Plan bp = big_q4_forward_plan(M, f.N, f.K, FL_STORE, max_ks, 0, false);
     require((size_t)bp.ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
     big_linear(f, FL_STORE, bp, s);
     return bp.ks;
@@ -895,8 +909,8 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       fg.act_fmt = fmt;
       if (rt.q4)
         big_linear(fg, FL_SWIGLU,
-                   big_q4_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats, 0.f,
-                               !rt.fenced && rt.n_xcc == 8),
+                   big_q4_forward_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats,
+                                       rt.split_last),
                    s, bpart, rt.big_tail_count.as<int>());
       else
         big_bf16_linear(fg, FL_SWIGLU, big_bf16_plan(M, fg.N, fg.K, FL_SWIGLU, 1, 0, 0.f), s);

@@ -6,6 +6,7 @@ kernel still runs to completion:
   raises, and the GPU is then fine for a new runtime;
 * the fenced split-K exchange (``DRT_SPLITK_FENCED=1``, what a runtime falls
   back to when its placement probe fails) gives bit-identical results;
+* the scores and tokens of a q4 canvas, bit for bit;
 * hardware queues that come into being after a runtime and move where its stream's
   work-groups land: the same results as before;
 * the fp16 range of the activations: a first-layer norm weight that pushes the
@@ -78,6 +79,40 @@ def test_fenced_split_k_exchange_is_bit_identical():
     s1, t1, f1 = _propose(model, {"DRT_SPLITK_FENCED": "1"})
     assert (t1, f1) == (t0, f0)
     assert np.array_equal(np.asarray(s1), np.asarray(s0))
+
+
+# Scores and tokens of a q4 canvas, bit for bit as they always were: every fp32 sum of such a
+# forward is cut along K where the shape says (big_q4_forward_plan) and its probabilities are
+# rounded one way (attn_split_tile), whatever the kernels' tiles and launches. Otherwise a row
+# whose two best logits are all but equal takes its other token. 512 rows attend in two key
+# ranges (met in one work-group), 257 in four, 100 in more; the gate|up projection stays below
+# two work-groups per CU, where nothing depends on the process's hardware queues.
+_CANVAS_DIGESTS = {100: "f94f169c64e44037", 257: "bfa80cbd6e0fcbd8", 512: "0738386d73833c8b"}
+
+
+@pytest.mark.parametrize("n", sorted(_CANVAS_DIGESTS))
+def test_canvas_results_are_bit_stable(n):
+    import hashlib
+
+    from diffusorrt_amd import synthetic as syn
+    from diffusorrt_amd.runtime import Runtime, fixed_quota_session_config
+
+    from helpers import tiny_dream_geometry
+
+    _say("canvas bits", n)
+    g = tiny_dream_geometry(hidden_size=1024, intermediate_size=3072, num_heads=14, num_kv_heads=2,
+                            vocab_size=4096)
+    rt = Runtime(syn.build_model(g, "q4", seed=55), max_forward_rows=512, max_positions=512)
+    toks = [(7 * i) % 900 for i in range(n - n // 2)] + [g.mask_token_id] * (n // 2)
+    with rt.session(fixed_quota_session_config(64, 64, n)) as s:
+        s.start_device(toks, prompt_len=n - n // 2, block_size=64, mask_token_id=g.mask_token_id,
+                       exact_kv=False, steps=8)
+        scores, tokens, _ = s.propose_device(list(range(n - n // 2, n)), window_end=n,
+                                             frozen_prefix=0)
+    rt.close()
+    h = hashlib.sha256(np.asarray(scores, dtype="<f8").tobytes() +
+                       np.asarray(tokens, dtype="<i4").tobytes()).hexdigest()[:16]
+    assert h == _CANVAS_DIGESTS[n]
 
 
 _LATER_QUEUES = """
