@@ -130,7 +130,7 @@ DRT_DEV void big_q4_tile(const FusedArgs& a, int KS, const BgTail& tail) {
       // raises the placement error (the host then fails the forward)
       if (threadIdx.x == 0 && a.placement_err) {
         const int xcc = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xf);  // HW_REG_XCC_ID
-        const int r = (xcc - b) & 7;
+        const int r = drt::xcd_rotation(xcc, b, 8);
         if (r != a.placement_err[1])
           __hip_atomic_fetch_or(a.placement_err, 1 | drt::placement_bit(r), __ATOMIC_RELAXED,
                                 __HIP_MEMORY_SCOPE_AGENT);

@@ -60,7 +60,7 @@ extern "C" __global__ __launch_bounds__(256) void embed_kernel(
   const int m = blockIdx.x, c = threadIdx.x, ng = d >> 5;
   const bool live = c < ng;
   if (rot && m == 0 && c == 0)  // where this launch's work-group 0 runs (see probe_round_robin)
-    *rot = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0x7);  // HW_REG_XCC_ID
+    *rot = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xf);  // HW_REG_XCC_ID
   if (row_desc) tokens += row_desc->row0;
   float* ss_row = ss_out ? ss_out + (int64_t)(m >> 5) * d + (m & 31) : nullptr;
   float* xs_row = pre ? pre_xs + (int64_t)(m >> 5) * d + (m & 31) : nullptr;

@@ -1,6 +1,7 @@
 // Arguments and modes of the fused linear kernel (fused_linear.hip).
 #pragma once
 #include "common.h"
+#include "placement.h"
 
 enum { W_Q4 = 0, W_BF16 = 1 };
 enum { PRO_ACT = 0, PRO_NORM = 1 };
@@ -114,9 +115,6 @@ size_t skinny_part_floats(int N, int K);
 // -1 where there is none (scratch_dev: >= 256 ints). It is the hardware queue's: 0 in a
 // process with one queue, another for each queue once there are several.
 int probe_round_robin(int n_xcc, int* scratch_dev, hipStream_t s);
-// What a work-group that finds itself on XCD xcc, a launch's rotation r away from its
-// place x, reports besides the placement bit.
-constexpr int placement_bit(int r) { return 1 << (8 + r); }
 int skinny_counters(int N);
 // Whether the split-K kernels take a linear of this kind and shape (given
 // workspaces sized by skinny_part_floats / skinny_counters).

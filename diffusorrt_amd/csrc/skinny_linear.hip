@@ -94,7 +94,7 @@ DRT_DEV bool sk_place(int n_xcc, int n_blocks, int KS, int& blk, int& ks) {
 DRT_DEV void sk_check(int n_xcc, int fenced, int* perr) {
   if (n_xcc > 1 && !fenced && threadIdx.x == 0 && perr) {
     const int xcc = (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xf);  // HW_REG_XCC_ID
-    const int r = (xcc - (int)blockIdx.x % n_xcc) & 7;
+    const int r = drt::xcd_rotation(xcc, (int)blockIdx.x, n_xcc);
     if (r != perr[1])
       __hip_atomic_fetch_or(perr, 1 | drt::placement_bit(r), __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);

@@ -1,0 +1,44 @@
+"""The host's and the kernels' reckoning of work-group placement (``csrc/placement.h``), on the
+CPU: the header is compiled into a small program that counts what it finds wrong."""
+from __future__ import annotations
+
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "diffusorrt_amd",
+                    "csrc")
+
+
+def _run(tmp_path, body, *headers):
+    src = tmp_path / "t.cpp"
+    src.write_text("#include <cstdio>\n#include <initializer_list>\n" + "".join(f'#include "{h}"\n' for h in headers) +
+                   "int main() {\n  int wrong = 0;\n" + body + "  return wrong != 0;\n}\n")
+    exe = tmp_path / "t"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, str(src), "-o", str(exe), "-pthread"],
+                   check=True, capture_output=True, text=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout
+
+
+@pytest.mark.parametrize("n_xcc", [1, 2, 4, 8])
+def test_rotation_is_the_same_for_every_work_group(tmp_path, n_xcc):
+    _run(tmp_path, """
+  const int n = %d;
+  for (int r = 0; r < n; ++r)
+    for (int i = 0; i < 512; ++i)
+      if (drt::xcd_rotation((i + r) %% n, i, n) != r) { ++wrong; std::printf("r %%d i %%d\\n", r, i); }
+""" % n_xcc, "placement.h")
+
+
+def test_a_wrong_xcd_count_shows(tmp_path):
+    # eight XCDs taken for four or two: some of the first eight work-groups disagree
+    _run(tmp_path, """
+  for (int n : {2, 4})
+    for (int r = 0; r < 8; ++r) {
+      bool differs = false;
+      for (int i = 0; i < 8; ++i) differs = differs || drt::xcd_rotation((i + r) % 8, i, n) != r;
+      wrong += !differs;
+    }
+""", "placement.h")
