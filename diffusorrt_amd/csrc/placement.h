@@ -15,4 +15,12 @@ constexpr int xcd_rotation(int xcc, int i, int n_xcc) {
 // error word besides bit 0, the placement's.
 constexpr int placement_bit(int r) { return 1 << (8 + r); }
 
+// A drained stream's error word without its placement reports, if every one of them names the
+// rotation that the stream has now; other kernels' bits stay. Else the word as it is.
+constexpr int settled_word(int word, int rotation) {
+  constexpr int any = ((1 << 16) - 1) << 8;
+  if (rotation < 0 || (word & any) != placement_bit(rotation)) return word;
+  return word & ~(1 | placement_bit(rotation));
+}
+
 }  // namespace drt

@@ -163,6 +163,7 @@ struct Runtime {
   DevBuf placement_err;          // int, set by a kernel that finds itself on an unexpected XCD,
                                  // and this forward's rotation (written by its embedding)
   int* placement_host = nullptr; // pinned copy, read after each synchronized forward
+  int test_seen = 0;  // (DRT_PLACEMENT_WORD)
   // pinned landing area of a forward's scores and tokens, written by the LM head's
   // last kernel (the caller's arrays are pageable)
   char* out_host = nullptr;
@@ -535,6 +536,14 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     DRT_HIP(hipMemsetAsync(rt->placement_err.p, 0, 8, s));
     DRT_HIP(hipHostMalloc((void**)&rt->placement_host, 4, hipHostMallocCoherent));
     *rt->placement_host = 0;
+    // DRT_PLACEMENT_WORD=seen,word (a test hook): the first check of the error word sees
+    // `seen`, while the device's already holds `word`, as with a block queued behind
+    if (const char* w = getenv("DRT_PLACEMENT_WORD")) {
+      char* rest = nullptr;
+      rt->test_seen = (int)strtol(w, &rest, 10);
+      const int word = *rest == ',' ? (int)strtol(rest + 1, nullptr, 10) : 0;
+      DRT_HIP(hipMemcpy(rt->placement_err.p, &word, 4, hipMemcpyHostToDevice));
+    }
   }
   DRT_HIP(hipStreamSynchronize(s));
   size_t total = rt->embed.bytes + rt->final_norm.bytes + rt->lm_head.qw.bytes +
@@ -985,16 +994,20 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
 void check_placement(Runtime& rt) {
   // the placement first: a split-K exchange across XCDs produces garbage, which
   // may also trip the other two checks
-  int e = *rt.placement_host;
+  int e = rt.test_seen;
+  rt.test_seen = 0;
+  if (e == 0) e = *rt.placement_host;
   if ((e & 1) && rt.xcc_probed && !rt.fenced) {
     // Another rotation from some kernel on (every report the same, and what the stream has
     // now): a hardware queue created during the forward moved this one. What the exchange
-    // needs, equal i % n_xcc on one XCD, held all along.
+    // needs, equal i % n_xcc on one XCD, held all along. The probe drains the stream, a
+    // block queued behind included: the word is read again, and keeps what that reported.
     const int r = probe_round_robin(rt.n_xcc, rt.xcc_probe.as<int>(), rt.stream);
-    if (r >= 0 && (e & ~(1 | placement_bit(r))) == 0 && (e & placement_bit(r))) {
-      DRT_HIP(hipMemsetAsync(rt.placement_err.p, 0, 4, rt.stream));
-      e = *rt.placement_host = 0;
-    }
+    DRT_HIP(hipMemcpyAsync(rt.placement_host, rt.placement_err.p, 4, hipMemcpyDeviceToHost, rt.stream));
+    DRT_HIP(hipStreamSynchronize(rt.stream));
+    e = *rt.placement_host = settled_word(*rt.placement_host, r);
+    DRT_HIP(hipMemcpyAsync(rt.placement_err.p, rt.placement_host, 4, hipMemcpyHostToDevice, rt.stream));
+    DRT_HIP(hipStreamSynchronize(rt.stream));
   }
   if (e & 1)
     fail(INTERNAL_ERROR,

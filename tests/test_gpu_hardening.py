@@ -9,6 +9,8 @@ kernel still runs to completion:
 * the scores and tokens of a q4 canvas, bit for bit;
 * hardware queues that come into being after a runtime and move where its stream's
   work-groups land: the same results as before;
+* a placement report of a rotation that the stream has taken (``DRT_PLACEMENT_WORD``) is
+  settled, and what a block queued behind it reported meanwhile is not lost;
 * the fp16 range of the activations: a first-layer norm weight that pushes the
   normalized activation past 65504 raises the range error, one that keeps it
   near 4e4 (checked on the CPU) does not.
@@ -113,6 +115,32 @@ def test_canvas_results_are_bit_stable(n):
     h = hashlib.sha256(np.asarray(scores, dtype="<f8").tobytes() +
                        np.asarray(tokens, dtype="<i4").tobytes()).hexdigest()[:16]
     assert h == _CANVAS_DIGESTS[n]
+
+
+def test_a_settled_rotation_keeps_other_reports():
+    from diffusorrt_amd import synthetic as syn
+
+    model = syn.build_model(tiny_geometry(), "q4", seed=56)
+    s0, t0, f0 = _propose(model)
+
+    def outcome(word, seen=None):
+        try:
+            s, t, f = _propose(model, {"DRT_PLACEMENT_WORD": f"{seen or word},{word}"})
+        except RuntimeError as e:
+            return str(e)
+        assert (t, f) == (t0, f0) and np.array_equal(np.asarray(s), np.asarray(s0))
+        return "settled"
+
+    _say("settled rotation, and other reports")
+    moved = [1 | 1 << (8 + r) for r in range(8)]
+    plain = [outcome(w) for w in moved]
+    assert "settled" in plain  # (the stream's rotation; a queue's may differ from run to run)
+    assert all(o == "settled" or "unexpected XCD" in o for o in plain)
+    for bit, text in ((2, "bounded wait"), (4, "fp16 range")):
+        late = [outcome(w | bit, seen=w) for w in moved]  # reported after the host looked
+        assert any(text in o for o in late)
+        assert all(text in o or "unexpected XCD" in o for o in late)
+    assert "unexpected XCD" in outcome(moved[0] | moved[1])
 
 
 _LATER_QUEUES = """

@@ -32,6 +32,25 @@ def test_rotation_is_the_same_for_every_work_group(tmp_path, n_xcc):
 """ % n_xcc, "placement.h")
 
 
+def test_settled_word_keeps_other_reports(tmp_path):
+    # 2: a bounded wait, 4: the fp16 range
+    _run(tmp_path, """
+  for (int r = 0; r < 8; ++r)
+    for (int other : {0, 2, 4, 6}) {
+      const int moved = 1 | drt::placement_bit(r);
+      wrong += drt::settled_word(other, r) != other;
+      wrong += drt::settled_word(moved | other, r) != other;
+      for (int q = 0; q < 8; ++q) {
+        if (q == r) continue;
+        wrong += drt::settled_word(moved | other, q) != (moved | other);
+        const int two = moved | drt::placement_bit(q) | other;
+        wrong += drt::settled_word(two, r) != two || drt::settled_word(two, q) != two;
+      }
+      wrong += drt::settled_word(moved | other, -1) != (moved | other);
+    }
+""", "placement.h")
+
+
 def test_a_wrong_xcd_count_shows(tmp_path):
     # eight XCDs taken for four or two: some of the first eight work-groups disagree
     _run(tmp_path, """
