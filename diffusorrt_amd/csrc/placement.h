@@ -16,10 +16,15 @@ constexpr int xcd_rotation(int xcc, int i, int n_xcc) {
 constexpr int placement_bit(int r) { return 1 << (8 + r); }
 
 // A drained stream's error word without its placement reports, if every one of them names the
-// rotation that the stream has now; other kernels' bits stay. Else the word as it is.
-constexpr int settled_word(int word, int rotation) {
+// rotation that the stream has now and every arrival counter is back at zero (at_rest); other
+// kernels' bits stay. Else the word as it is.
+// The counters tell a rotation that moved between launches from one that moved inside one:
+// there a block's slices counted in two XCDs' L2s, neither reached the block's count, and
+// what either wrote back is neither zero nor the count. Every later launch then ends its
+// block early by as much and leaves the same remainder.
+constexpr int settled_word(int word, int rotation, bool at_rest) {
   constexpr int any = ((1 << 16) - 1) << 8;
-  if (rotation < 0 || (word & any) != placement_bit(rotation)) return word;
+  if (rotation < 0 || !at_rest || (word & any) != placement_bit(rotation)) return word;
   return word & ~(1 | placement_bit(rotation));
 }
 

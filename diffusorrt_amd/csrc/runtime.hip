@@ -536,13 +536,18 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     DRT_HIP(hipMemsetAsync(rt->placement_err.p, 0, 8, s));
     DRT_HIP(hipHostMalloc((void**)&rt->placement_host, 4, hipHostMallocCoherent));
     *rt->placement_host = 0;
-    // DRT_PLACEMENT_WORD=seen,word (a test hook): the first check of the error word sees
-    // `seen`, while the device's already holds `word`, as with a block queued behind
+    // DRT_PLACEMENT_WORD=seen,word[,count] (a test hook): the first check of the error word
+    // sees `seen`, while the device's already holds `word`, as with a block queued behind,
+    // and the last arrival counter (of a second row tile) `count`
     if (const char* w = getenv("DRT_PLACEMENT_WORD")) {
       char* rest = nullptr;
       rt->test_seen = (int)strtol(w, &rest, 10);
-      const int word = *rest == ',' ? (int)strtol(rest + 1, nullptr, 10) : 0;
-      DRT_HIP(hipMemcpy(rt->placement_err.p, &word, 4, hipMemcpyHostToDevice));
+      const int word = *rest == ',' ? (int)strtol(rest + 1, &rest, 10) : 0;
+      const int count = *rest == ',' ? (int)strtol(rest + 1, nullptr, 10) : 0;
+      DRT_HIP(hipMemcpyAsync(rt->placement_err.p, &word, 4, hipMemcpyHostToDevice, s));
+      DRT_HIP(hipMemcpyAsync(rt->sk_counters.as<char>() + rt->sk_counters.bytes - 4, &count, 4,
+                             hipMemcpyHostToDevice, s));
+      DRT_HIP(hipStreamSynchronize(s));
     }
   }
   DRT_HIP(hipStreamSynchronize(s));
@@ -991,6 +996,18 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
 // that observed otherwise left a flag (read back with the forward's results).
 // Bit 2 of the same flag: a wave of the decode attention gave up waiting for a K/V
 // tile (its bounded wait ran out), so that forward's attention is not valid.
+bool counters_at_rest(const Runtime& rt) {
+  for (const DevBuf* b : {&rt.sk_counters, &rt.big_tail_count}) {
+    std::vector<int> c(b->bytes / 4);
+    if (c.empty()) continue;
+    DRT_HIP(hipMemcpyAsync(c.data(), b->p, c.size() * 4, hipMemcpyDeviceToHost, rt.stream));
+    DRT_HIP(hipStreamSynchronize(rt.stream));
+    for (int v : c)
+      if (v != 0) return false;
+  }
+  return true;
+}
+
 void check_placement(Runtime& rt) {
   // the placement first: a split-K exchange across XCDs produces garbage, which
   // may also trip the other two checks
@@ -1000,12 +1017,13 @@ void check_placement(Runtime& rt) {
   if ((e & 1) && rt.xcc_probed && !rt.fenced) {
     // Another rotation from some kernel on (every report the same, and what the stream has
     // now): a hardware queue created during the forward moved this one. What the exchange
-    // needs, equal i % n_xcc on one XCD, held all along. The probe drains the stream, a
+    // needs, equal i % n_xcc on one XCD, held in every launch if it moved between two, and
+    // then every counter is zero again (see settled_word). The probe drains the stream, a
     // block queued behind included: the word is read again, and keeps what that reported.
     const int r = probe_round_robin(rt.n_xcc, rt.xcc_probe.as<int>(), rt.stream);
     DRT_HIP(hipMemcpyAsync(rt.placement_host, rt.placement_err.p, 4, hipMemcpyDeviceToHost, rt.stream));
     DRT_HIP(hipStreamSynchronize(rt.stream));
-    e = *rt.placement_host = settled_word(*rt.placement_host, r);
+    e = *rt.placement_host = settled_word(*rt.placement_host, r, counters_at_rest(rt));
     DRT_HIP(hipMemcpyAsync(rt.placement_err.p, rt.placement_host, 4, hipMemcpyHostToDevice, rt.stream));
     DRT_HIP(hipStreamSynchronize(rt.stream));
   }

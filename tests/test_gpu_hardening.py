@@ -123,9 +123,9 @@ def test_a_settled_rotation_keeps_other_reports():
     model = syn.build_model(tiny_geometry(), "q4", seed=56)
     s0, t0, f0 = _propose(model)
 
-    def outcome(word, seen=None):
+    def outcome(word, seen=None, count=0):
         try:
-            s, t, f = _propose(model, {"DRT_PLACEMENT_WORD": f"{seen or word},{word}"})
+            s, t, f = _propose(model, {"DRT_PLACEMENT_WORD": f"{seen or word},{word},{count}"})
         except RuntimeError as e:
             return str(e)
         assert (t, f) == (t0, f0) and np.array_equal(np.asarray(s), np.asarray(s0))
@@ -141,6 +141,8 @@ def test_a_settled_rotation_keeps_other_reports():
         assert any(text in o for o in late)
         assert all(text in o or "unexpected XCD" in o for o in late)
     assert "unexpected XCD" in outcome(moved[0] | moved[1])
+    # slices of one block that counted on two XCDs
+    assert all("unexpected XCD" in outcome(w, count=1) for w in moved)
 
 
 _LATER_QUEUES = """

@@ -38,16 +38,40 @@ def test_settled_word_keeps_other_reports(tmp_path):
   for (int r = 0; r < 8; ++r)
     for (int other : {0, 2, 4, 6}) {
       const int moved = 1 | drt::placement_bit(r);
-      wrong += drt::settled_word(other, r) != other;
-      wrong += drt::settled_word(moved | other, r) != other;
+      wrong += drt::settled_word(other, r, true) != other;
+      wrong += drt::settled_word(moved | other, r, true) != other;
+      wrong += drt::settled_word(moved | other, r, false) != (moved | other);
       for (int q = 0; q < 8; ++q) {
         if (q == r) continue;
-        wrong += drt::settled_word(moved | other, q) != (moved | other);
+        wrong += drt::settled_word(moved | other, q, true) != (moved | other);
         const int two = moved | drt::placement_bit(q) | other;
-        wrong += drt::settled_word(two, r) != two || drt::settled_word(two, q) != two;
+        wrong += drt::settled_word(two, r, true) != two || drt::settled_word(two, q, true) != two;
       }
-      wrong += drt::settled_word(moved | other, -1) != (moved | other);
+      wrong += drt::settled_word(moved | other, -1, true) != (moved | other);
     }
+""", "placement.h")
+
+
+def test_a_launch_cut_in_two_leaves_a_counter(tmp_path):
+    # KS slices of a block count in one L2, or (one launch) some in another: each L2 works on
+    # its own copy of the counter and either may be the one written back last. The last of a
+    # block sets it to zero. Later launches run whole; no remainder may come back to zero.
+    _run(tmp_path, """
+  for (int KS = 2; KS <= 16; ++KS)
+    for (int a = 1; a < KS; ++a)
+      for (int back = 0; back < 2; ++back) {
+        int c = back ? a : KS - a;
+        for (int launch = 0; launch < 64; ++launch) {
+          wrong += c == 0;
+          const int ks = 2 + (7 * KS + 5 * launch) % 15;  // another linear's slices
+          for (int i = 0; i < ks; ++i)
+            if (c++ == ks - 1) c = 0;
+        }
+        wrong += c == 0;
+      }
+  int c = 0;
+  for (int i = 0; i < 5; ++i) if (c++ == 4) c = 0;
+  wrong += c != 0;
 """, "placement.h")
 
 
