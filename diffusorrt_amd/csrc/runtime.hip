@@ -29,6 +29,7 @@
 #include "../../include/drt_rocm.h"
 #include "fused.h"
 #include "launch.h"
+#include "op_blocks.h"
 
 namespace drt {
 
@@ -2244,8 +2245,6 @@ static size_t q4_op_act_bytes(int32_t m, int32_t k) {
   return ((size_t)2 * m * k * 2 + (size_t)m * (k / 64) * 4 + 255) / 256 * 256;
 }
 
-constexpr int OP_COUNTER_BLOCKS = 32, OP_COUNTERS = 4096;  // (see op_counters)
-
 size_t drt_op_q4_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   if (m <= 0 || k <= 0) return 0;
   size_t b = q4_op_act_bytes(m, k) + 256;
@@ -2255,59 +2254,57 @@ size_t drt_op_q4_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   return b;
 }
 
-// The split-K store kernel of the per-op path (<= 32 rows): its arrival counters
-// live in a device array of the library, zero from load and left zero by every
-// launch, one block of OP_COUNTERS per (device, stream) so that calls on
-// different streams never share one; the XCD placement is probed once per
-// device (on a stream of its own, synchronised once).
+// The per-op calls whose work-groups meet through counters - the one-launch split-K kernel
+// (q4 up to 32 rows, bf16 up to 64) and the split last round of larger q4 calls - find them
+// in a device array of the library, zero from load and left zero by every launch, one block
+// of OP_COUNTERS per (device, stream). A stream's first such call probes its placement,
+// which waits for the stream once.
 static __device__ int op_counters[OP_COUNTER_BLOCKS * OP_COUNTERS];
-static __device__ int op_probe[256];
+static __device__ int op_probe[OP_COUNTER_BLOCKS * 256];
 namespace {
 struct OpDevice {
+  std::once_flag once;
   int* counters = nullptr;
+  int* probe = nullptr;
   int n_xcc = 1;
-  bool fenced = false;
-  std::map<hipStream_t, int> blocks;
+  CounterBlocks blocks;
 };
-std::mutex g_op_mu;
-std::map<int, OpDevice> g_op_dev;
+constexpr int OP_DEVICES = 64;
+OpDevice g_op_dev[OP_DEVICES];
 
-// The counter block of (current device, stream) and the device's placement,
-// or nullptr when every block is taken (the caller then takes another path).
+// The counter block of (current device, stream) and the form of its exchange, or nullptr
+// without a block.
 int* op_counters_for(hipStream_t stream, int& n_xcc, bool& fenced) {
   int dev = -1;
   DRT_HIP(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(g_op_mu);
-  OpDevice& d = g_op_dev[dev];
-  if (!d.counters) {
+  if (dev >= OP_DEVICES) return nullptr;
+  OpDevice* d = &g_op_dev[dev];
+  std::call_once(d->once, [&] {  // (a call that throws leaves it to the next)
     void* c = nullptr;
     void* pr = nullptr;
     DRT_HIP(hipGetSymbolAddress(&c, HIP_SYMBOL(op_counters)));
     DRT_HIP(hipGetSymbolAddress(&pr, HIP_SYMBOL(op_probe)));
     int nx = 1;
     if (hipDeviceGetAttribute(&nx, hipDeviceAttributeNumberOfXccs, dev) != hipSuccess) nx = 1;
-    d.n_xcc = std::max(1, nx);
-    hipStream_t ps = nullptr;
-    DRT_HIP(hipStreamCreateWithFlags(&ps, hipStreamNonBlocking));
-    int rot = -1;
-    try {
-      rot = probe_round_robin(d.n_xcc, (int*)pr, ps);
-    } catch (...) {
-      (void)hipStreamDestroy(ps);
-      throw;
-    }
-    DRT_HIP(hipStreamDestroy(ps));
-    d.fenced = rot < 0;  // (any rotation keeps equal i % n_xcc on one XCD, on any stream)
-    d.counters = (int*)c;
-  }
-  n_xcc = d.n_xcc;
-  fenced = d.fenced;
-  auto it = d.blocks.find(stream);
-  if (it == d.blocks.end()) {
-    if ((int)d.blocks.size() >= OP_COUNTER_BLOCKS) return nullptr;
-    it = d.blocks.emplace(stream, (int)d.blocks.size()).first;
-  }
-  return d.counters + (size_t)it->second * OP_COUNTERS;
+    d->n_xcc = std::max(1, nx);
+    d->probe = (int*)pr;
+    d->counters = (int*)c;
+  });
+  CounterBlocks::Block* b = d->blocks.of((uintptr_t)stream);
+  if (!b) return nullptr;
+  n_xcc = d->n_xcc;
+  fenced = CounterBlocks::fenced(
+      *b,
+      [&] {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+          (void)hipGetLastError();
+          return true;
+        }
+        return cap != hipStreamCaptureStatusNone;
+      },
+      [&] { return probe_round_robin(d->n_xcc, d->probe + 256 * b->index, stream); });
+  return d->counters + (size_t)b->index * OP_COUNTERS;
 }
 }  // namespace
 

@@ -220,10 +220,12 @@ int32_t drt_op_q4_quantize(const void* w, int32_t w_dtype, int32_t n, int32_t k,
 int32_t drt_op_cast_bf16(const float* x, void* y, int64_t n, void* stream);
 /* linear(x, QuantizedWeight, bias) (mlx_ops.py:97-130): y fp32 [m, n] from x fp32 or
  * bf16 [m, k]; bias bf16 [n] or NULL. Needs drt_op_q4_linear_workspace_bytes(m, n, k).
- * m <= 32: one split-K launch that reads x as it is; its arrival counters are a block of a
+ * m <= 32: one split-K launch that reads x as it is; m > 32: the tiles past whole rounds of
+ * the device may be split along K in the same launch. Both count arrivals in a block of a
  * library array reserved for (device, stream) on first use (32 per device; a further
- * stream's calls take a two-launch path), so calls on different streams never share
- * counters. Calls that overlap must not share a workspace. */
+ * stream's calls take a path without counters), so calls on different streams never share
+ * counters. A stream's first call probes where its work-groups run and waits for the stream
+ * once, unless the stream is being captured. Calls that overlap must not share a workspace. */
 size_t drt_op_q4_linear_workspace_bytes(int32_t m, int32_t n, int32_t k);
 int32_t drt_op_q4_linear(const void* qw, const void* sb, const void* x, int32_t x_dtype,
                          int32_t m, int32_t n, int32_t k, const void* bias, float* y,
@@ -241,7 +243,10 @@ int32_t drt_op_q4_linear_noalloc(const void* qw, const void* sb, const void* x, 
                                  void* stream);
 /* bf16 weight W [n, k] -> device tile layout wb (same size). */
 int32_t drt_op_bf16_repack(const void* w, int32_t n, int32_t k, void* wb, void* stream);
-/* linear(x, bf16 W): y = bf16(bf16(x) @ W^T) as fp32 [m, n]; x bf16 [m, k]. */
+/* linear(x, bf16 W): y = bf16(bf16(x) @ W^T) as fp32 [m, n]; x bf16 [m, k]. A workspace of
+ * drt_op_bf16_linear_workspace_bytes holds K slices; with a smaller one, or NULL, K is not
+ * split. Calls that overlap must not share a workspace. m <= 64 with a workspace: arrival
+ * counters and a first call as drt_op_q4_linear's (a captured call does without). */
 size_t drt_op_bf16_linear_workspace_bytes(int32_t m, int32_t n, int32_t k);
 int32_t drt_op_bf16_linear(const void* wb, const void* x, int32_t m, int32_t n, int32_t k,
                            const void* bias, float* y, void* workspace, size_t workspace_bytes,

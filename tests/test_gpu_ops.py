@@ -255,6 +255,47 @@ def test_q4_linear_large_m_plans(m, n, k):
         assert bool(((yg.double() - (exact + bd.double())).abs() <= bound).all())
 
 
+def _counting_linears():
+    """Calls whose work-groups meet through counters, with their results on this stream: the
+    one-launch kernel for both weight types and the split last round (296 tiles on 256 CUs)."""
+    from diffusorrt_amd import kernels
+
+    calls = []
+    for kind, m, n, k in [("q4", 32, 3072, 1024), ("bf16", 32, 1024, 3072), ("q4", 500, 18944, 1024)]:
+        gen, q = _q4_case(n, k, seed=36)
+        w = (kernels.DeviceQ4Weight(q.w_q.cuda(), q.scales.cuda(), q.biases.cuda()) if kind == "q4"
+             else kernels.DeviceBF16Weight((torch.randn((n, k), generator=gen) * 0.02).bfloat16().cuda()))
+        x = torch.randn((m, k), generator=gen).cuda()
+        calls.append((x, w, kernels.linear(x, w)))
+    torch.cuda.synchronize()
+    return calls
+
+
+def test_linears_on_fresh_streams():
+    from diffusorrt_amd import kernels
+
+    _say("linears on fresh streams, eager and captured first")
+    calls = _counting_linears()
+    for _ in range(6):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for x, w, y in calls:
+                assert torch.equal(kernels.linear(x, w), y)
+    for x, w, y in calls[:1]:  # captured before any call on its stream: the same bits
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            yg = kernels.linear(x, w)
+        for _ in range(3):
+            yg.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(yg, y)
+            with torch.cuda.stream(stream):
+                assert torch.equal(kernels.linear(x, w), y)
+            torch.cuda.synchronize()
+
+
 # ---------------------------------------------------------------- attention (config 2)
 
 def _attention_inputs(L, seed=1, rows=32, hq=16, hkv=8):

@@ -1,5 +1,6 @@
-"""The host's and the kernels' reckoning of work-group placement (``csrc/placement.h``), on the
-CPU: the header is compiled into a small program that counts what it finds wrong."""
+"""The host's and the kernels' reckoning of work-group placement (``csrc/placement.h``) and the
+per-op calls' counter blocks (``csrc/op_blocks.h``), on the CPU: the header is compiled into a
+small program that counts what it finds wrong."""
 from __future__ import annotations
 
 import os
@@ -13,7 +14,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 def _run(tmp_path, body, *headers):
     src = tmp_path / "t.cpp"
-    src.write_text("#include <cstdio>\n#include <initializer_list>\n" + "".join(f'#include "{h}"\n' for h in headers) +
+    src.write_text("#include <cstdio>\n#include <initializer_list>\n" + "".join(f'#include {h if h[0] == "<" else chr(34) + h + chr(34)}\n' for h in headers) +
                    "int main() {\n  int wrong = 0;\n" + body + "  return wrong != 0;\n}\n")
     exe = tmp_path / "t"
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, str(src), "-o", str(exe), "-pthread"],
@@ -85,3 +86,48 @@ def test_a_wrong_xcd_count_shows(tmp_path):
       wrong += !differs;
     }
 """, "placement.h")
+
+
+def test_the_exchange_is_probed_on_each_stream(tmp_path):
+    # stream 16 is round-robin, stream 32 (a CU mask, say) is not; one being captured is not
+    # probed, takes the fenced form, and is probed by its next call
+    _run(tmp_path, """
+  drt::CounterBlocks blocks;
+  int probes = 0;
+  bool capturing = false;
+  auto fenced = [&](std::uintptr_t s) {
+    auto* b = blocks.of(s);
+    return drt::CounterBlocks::fenced(*b, [&] { return capturing; },
+                                      [&] { ++probes; return s == 32 ? -1 : 5; });
+  };
+  for (int i = 0; i < 3; ++i) wrong += fenced(16) || !fenced(32);
+  wrong += probes != 2;
+  capturing = true;
+  wrong += !fenced(48) || probes != 2;
+  wrong += fenced(16) || !fenced(32);
+  capturing = false;
+  wrong += fenced(48) || probes != 3;
+  wrong += blocks.of(16)->index == blocks.of(32)->index || blocks.of(16) != blocks.of(16);
+  for (std::uintptr_t s = 64; s < 64 + 29; ++s) wrong += !blocks.of(s);
+  wrong += blocks.of(1000) != nullptr || !blocks.of(64);
+""", "op_blocks.h")
+
+
+def test_threads_on_one_stream_share_its_block_and_probe(tmp_path):
+    _run(tmp_path, """
+  drt::CounterBlocks blocks;
+  std::atomic<int> probes{0}, odd{0};
+  std::vector<std::thread> ts;
+  for (int t = 0; t < 8; ++t)
+    ts.emplace_back([&] {
+      for (int i = 0; i < 200; ++i) {
+        auto* b = blocks.of(16);
+        if (drt::CounterBlocks::fenced(*b, [] { return false; },
+                                       [&] { ++probes; std::this_thread::yield(); return 0; }) ||
+            b->index != 0)
+          ++odd;
+      }
+    });
+  for (auto& t : ts) t.join();
+  wrong += odd + (probes != 1);
+""", "op_blocks.h", "<thread>", "<vector>")
