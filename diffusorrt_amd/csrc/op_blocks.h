@@ -21,9 +21,11 @@ class CounterBlocks {
     std::mutex mu;
   };
 
-  // The block of a stream handle; null when every block is taken: the caller then takes a
-  // path without counters.
+  // The block of a stream handle; null when every block is taken, or for the handle that
+  // stands for another stream in each thread (two of them would count in one block at the
+  // same time): the caller then takes a path without counters.
   Block* of(uintptr_t stream) {
+    if (stream == PER_THREAD) return nullptr;
     std::lock_guard<std::mutex> lock(mu_);
     auto it = blocks_.find(stream);
     if (it == blocks_.end()) {
@@ -50,6 +52,8 @@ class CounterBlocks {
     }
     return b.form == FENCED;
   }
+
+  static constexpr uintptr_t PER_THREAD = 2;  // hipStreamPerThread
 
  private:
   std::mutex mu_;

@@ -223,7 +223,7 @@ int32_t drt_op_cast_bf16(const float* x, void* y, int64_t n, void* stream);
  * m <= 32: one split-K launch that reads x as it is; m > 32: the tiles past whole rounds of
  * the device may be split along K in the same launch. Both count arrivals in a block of a
  * library array reserved for (device, stream) on first use (32 per device; a further
- * stream's calls take a path without counters), so calls on different streams never share
+ * stream's calls, and those on hipStreamPerThread, take a path without counters), so calls on different streams never share
  * counters. A stream's first call probes where its work-groups run and waits for the stream
  * once, unless the stream is being captured. Calls that overlap must not share a workspace. */
 size_t drt_op_q4_linear_workspace_bytes(int32_t m, int32_t n, int32_t k);

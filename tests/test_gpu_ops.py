@@ -296,6 +296,60 @@ def test_linears_on_fresh_streams():
             torch.cuda.synchronize()
 
 
+def test_linears_of_two_threads_on_the_per_thread_stream():
+    import ctypes as C
+    import threading
+
+    from diffusorrt_amd import _lib, kernels
+
+    _say("linears on hipStreamPerThread from two threads")
+    lib, per_thread = _lib.load(), C.c_void_p(2)
+    calls = _counting_linears()
+
+    def ptr(t):
+        return C.c_void_p(t.data_ptr())
+
+    jobs = []
+    for x, w, y in calls * 2:  # each thread its own outputs and workspaces, filled ahead
+        (m, k), n = x.shape, y.shape[1]
+        q4 = isinstance(w, kernels.DeviceQ4Weight)
+        ws = (lib.drt_op_q4_linear_workspace_bytes if q4
+              else lib.drt_op_bf16_linear_x_workspace_bytes)(m, n, k)
+        jobs.append((x, w, y, [torch.full_like(y, float("nan")) for _ in range(8)],
+                     [torch.empty(ws, dtype=torch.uint8, device="cuda") for _ in range(8)]))
+    torch.cuda.synchronize()
+    errors, start = [], threading.Barrier(2)
+
+    def work(mine):
+        try:
+            start.wait(timeout=20)
+            for i in range(8):
+                for x, w, y, outs, spaces in mine:
+                    (m, k), n = x.shape, y.shape[1]
+                    args = (_lib.F32, m, n, k, None, ptr(outs[i]), ptr(spaces[i]), spaces[i].numel(),
+                            per_thread)
+                    if isinstance(w, kernels.DeviceQ4Weight):
+                        _lib.check(lib.drt_op_q4_linear(ptr(w.qw), ptr(w.sb), ptr(x), *args))
+                    else:
+                        _lib.check(lib.drt_op_bf16_linear_x(ptr(w.wb), ptr(x), *args))
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(jobs[i::2],)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    torch.cuda.synchronize()
+    assert not errors
+    for x, w, y, outs, _ in jobs:
+        for o in outs:
+            # another kernel: fp32 sums in another order, and for bf16 one bf16 step of a result
+            tol = 2e-6 if isinstance(w, kernels.DeviceQ4Weight) else 2.0 ** -8
+            assert torch.equal(o, outs[0])
+            assert ((o - y).norm() <= tol * y.norm()).item()
+
+
 # ---------------------------------------------------------------- attention (config 2)
 
 def _attention_inputs(L, seed=1, rows=32, hq=16, hkv=8):

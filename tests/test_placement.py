@@ -131,3 +131,11 @@ def test_threads_on_one_stream_share_its_block_and_probe(tmp_path):
   for (auto& t : ts) t.join();
   wrong += odd + (probes != 1);
 """, "op_blocks.h", "<thread>", "<vector>")
+
+
+def test_the_per_thread_handle_has_no_block(tmp_path):
+    # one handle, as many streams as threads: they would count in one block at the same time
+    _run(tmp_path, """
+  drt::CounterBlocks blocks;
+  wrong += blocks.of(2) != nullptr || !blocks.of(0) || !blocks.of(1);
+""", "op_blocks.h")
