@@ -537,10 +537,11 @@ __global__ __launch_bounds__(256) void skinny_narrow_kernel(
       for (int j = 0; j < 4; ++j) {
         const int64_t off = (int64_t)min(8 * j + (lane >> 3), M - 1) * K + u * 64 + (lane & 7) * 8;
         if (XIN == 1) {
-          xr[XIN == 1 ? i : 0][j][0] = *(const f32x4*)(x32 + off);
-          xr[XIN == 1 ? i : 0][j][1] = *(const f32x4*)(x32 + off + 4);
+          // (a caller's rows: a view into a larger buffer is aligned to its element)
+          xr[XIN == 1 ? i : 0][j][0] = *(const f32x4_e*)(x32 + off);
+          xr[XIN == 1 ? i : 0][j][1] = *(const f32x4_e*)(x32 + off + 4);
         } else {
-          craw[i][j] = *(const u32x4*)(act + off);  // XIN == 2: 8 bf16 values
+          craw[i][j] = *(const u32x4_e*)(act + off);  // XIN == 2: 8 bf16 values
           if (!BF && XIN == 0) crawl[i][j] = *(const u32x4*)(act_lo + off);
         }
       }

@@ -734,6 +734,28 @@ def test_q4_linear_activation_offsets(m, off, dtype):
     assert torch.equal(y, kernels.linear(flat[off:].view(m, 2048).contiguous().cuda(), w).cpu())
 
 
+# fp32 rows read by the one-launch kernel and cast for the others, bf16 rows as they are: the
+# one-launch, streaming, general (K of 80) and GEMM kernels
+@pytest.mark.parametrize("m,n,k,off", [(32, 1024, 3072, 1), (64, 3072, 1024, 3), (9, 3584, 3584, 1),
+                                       (3, 18944, 3584, 5), (33, 256, 80, 1), (300, 1024, 3072, 1)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_bf16_linear_activation_offsets(m, n, k, off, dtype):
+    from diffusorrt_amd import kernels
+
+    _say("bf16_linear activation", m, n, k, dtype, "offset", off)
+    gen = torch.Generator().manual_seed(37)
+    wt = (torch.randn((n, k), generator=gen) * 0.02).to(torch.bfloat16)
+    flat = torch.randn(m * k + off, generator=gen)
+    flat = flat.to(torch.bfloat16) if dtype == "bf16" else flat
+    w = kernels.DeviceBF16Weight(wt.cuda())
+    x = flat[off:].view(m, k)
+    y = kernels.linear(flat.cuda()[off:].view(m, k), w).double()
+    xd, wd = x.to(torch.bfloat16).double().cuda(), wt.double().cuda()
+    exact, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    # half a bf16 ulp of the product, and the fp32 sums' own error ahead of the rounding
+    assert bool(((y - exact).abs() <= exact.abs() * 2.0 ** -8 + mag * k * 2.0 ** -24).all())
+
+
 @pytest.mark.parametrize("pos0,n,src,kv", [(0, 32, "f32", "f16"), (5, 3, "f32", "f16"),
                                            (30, 70, "bf16", "bf16"), (64, 33, "bf16", "f16"),
                                            (17, 15, "f32", "bf16")])
