@@ -206,16 +206,19 @@ DRT_DEV void attn_split_tile(
 #pragma unroll
   for (int hb = 0; hb < 4; ++hb) o[hb] = f32x16{};
 
-  const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(kv + (int64_t)kvh * kv_head_stride), 0, (uint32_t)n_tiles * TILE_BYTES, 0x00020000);
   constexpr int LD = TILE_BYTES / 1024 / QW;  // 1 KiB loads per wave and slot
-  // tile it of this wave's key group (past the cache's last tile: zeros, never used)
+  // tile it of this wave's key group, a buffer of its own (a head's keys may pass the 4 GiB of
+  // one); past the cache's last tile an empty one: zeros, never used
   auto issue = [&](int it, char* dst) {
+    const int t = kt0 + it;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(kv + (int64_t)kvh * kv_head_stride + (int64_t)t * KV_TILE_ELEMS), 0,
+        t < n_tiles ? TILE_BYTES : 0, 0x00020000);
 #pragma unroll
     for (int i = 0; i < LD; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           src, (__attribute__((address_space(3))) void*)(dst + (wave * LD + i) * 1024), 16,
-          (uint32_t)((kt0 + it) * TILE_BYTES + (qw * LD + i) * 1024 + lane * 16), 0, 0, 0);
+          (uint32_t)((qw * LD + i) * 1024 + lane * 16), 0, 0, 0);
   };
   auto compute = [&](int it, const char* slot) {
     const int t = kt0 + it, key0 = t * 32;
@@ -1157,7 +1160,6 @@ void attention(bool bf16, const void* q, const void* kv_layer, int64_t kv_head_s
   require(Hq % Hkv == 0, "attention needs Hq % Hkv == 0");
   require(n_keys >= 1 && n_rows >= 1, "attention needs at least one query row and key");
   const float scale = 1.0f / sqrtf(128.0f);
-  require((size_t)((n_keys + 31) / 32) * 16384 <= 0xFFFFFFFFu, "attention: too many keys");
   const dim3 grid(plan.splits * Hkv, plan.qgroups);
   const dim3 block(64 * plan.qw * plan.kg);
   const AttnOut ao{out, xsum, err, out_fmt};

@@ -429,6 +429,31 @@ def test_block_attention_many_key_ranges(hq, hkv):
     assert mean_rel < 6e-3
 
 
+def test_attention_over_more_keys_than_4_gib_hold():
+    from diffusorrt_amd import kernels
+
+    keys, rows = (1 << 23) + 4096, 160  # 512 bytes a key: one head's K and V pass 4 GiB
+    _say("attention over", keys, "keys")
+    cache = kernels.PrefixKVCache(1, 1, keys, dtype="f16")
+    # K is zero, so every key weighs the same; V differs from zero in the last 4096 keys only
+    v = torch.randn((4096, 1, 128), generator=torch.Generator().manual_seed(38)).cuda() * 1000
+    cache.store(0, torch.zeros_like(v), v, keys - 4096)
+    q = torch.randn((rows, 1, 128), device="cuda").half()
+    want = v[:, 0].half().double().sum(0) / keys
+    for kind, geometry in (("full", None), ("d2f_hybrid", (0, 32))):
+        y = cache.attention(0, q, n_keys=keys, row_pos0=keys - rows, kind=kind,
+                            mask_geometry=geometry).double()
+        # every weight is one and their count exact below 2^24; V is summed over 128 tiles of 32
+        # keys, 2^-24 of the magnitudes each (here at most a few hundred times the sum's). The
+        # mask takes up to 128 keys from a row
+        some = want if geometry is None else None
+        for r in range(0, rows, 32):
+            if geometry is not None:
+                n = keys - rows + r + 32
+                some = v[:4096 - (keys - n), 0].half().double().sum(0) / n
+            assert ((y[r:r + 32] - some).norm(dim=1) <= 1e-4 * some.norm()).all()
+
+
 @pytest.mark.parametrize("kind,rows,pos0,L", [("d2f_hybrid", 96, 64, 160),
                                               # one tile, a ragged last tile, an odd tile count,
                                               # more key tiles than a key group's share
