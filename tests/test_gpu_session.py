@@ -92,6 +92,70 @@ def test_bd3_execute_window_and_propose(kind):
     rt.close()
 
 
+@pytest.mark.parametrize("prompt_len,n", [
+    (0, 160),   # chunks of 96 and 32 rows, the last with the block's 32: one forward
+    (0, 224),   # two whole chunks: the second and the block do not fit one forward
+    (20, 148),  # a chunk cut back to a block's start (84 rows), then 32 and the block
+    (20, 160),  # a block of 12 rows behind two chunks of whole blocks
+])
+def test_bf16_window_over_several_chunks(prompt_len, n):
+    """The last commit chunk and the active block as one forward (or two), and the K/V that
+    it committed reused by the next window."""
+    from diffusorrt_amd import synthetic as syn
+    from diffusorrt_amd.runtime import Runtime, bd3_session_config
+
+    _say("bf16 window over chunks", prompt_len, n)
+    geom = tiny_geometry()
+    model = syn.build_model(geom, "bf16", 57)
+    rt = Runtime(model, max_forward_rows=96, max_positions=512)
+    W, cfg = _oracle(model)
+    rng = np.random.default_rng(7)
+    ids = rng.integers(0, 900, n).tolist()
+    first = prompt_len + (n - 1 - prompt_len) // 32 * 32  # the last block's start
+    with rt.session(bd3_session_config(32, 8, n + 64)) as s:
+        before, done = s.device_metrics(), 0
+        for step in range(2):
+            end = n if step == 0 else first + 64
+            scope = list(range(first + 32 * step, end))
+            ids = (ids + rng.integers(0, 900, 64).tolist())[:end]
+            got = s.execute_window(ids, scope, mask_geometry=(prompt_len, 32))
+            ref = F.forward_full(W, cfg, ids, mask_kind="d2f_hybrid",
+                                 mask_geometry=(prompt_len, 32), output_rows=scope)
+            assert rel_err_rows(got.array(), ref).max() < LOGITS_REL_TOL
+            m = s.device_metrics()
+            frozen = first + 32 * step
+            assert got.forwarded_rows == end - done
+            assert m["rocm_kv_cache_len"] == frozen
+            assert m["rocm_commit_rows"] - before["rocm_commit_rows"] == frozen - done
+            assert m["rocm_active_rows"] - before["rocm_active_rows"] == end - frozen
+            before, done = m, frozen
+    rt.close()
+
+
+@pytest.mark.parametrize("n", [700, 1100])
+def test_bf16_window_large_tiles(n):
+    """Row counts and widths whose linears take the large tiles: 700 rows, gate|up in whole
+    rounds of 256 x 256 tiles with the last columns on 128 x 128 ones; 1100 rows, all 256 x
+    256, and q|k|v on two-buffer 128 x 128 tiles (on 256 CUs). Every row is scored."""
+    from diffusorrt_amd import synthetic as syn
+    from diffusorrt_amd.runtime import Runtime, bd3_session_config
+
+    _say("bf16 window, large tiles", n)
+    geom = tiny_geometry(num_heads=24, num_kv_heads=4, intermediate_size=11520)
+    model = syn.build_model(geom, "bf16", 58)
+    rt = Runtime(model, max_forward_rows=1152, max_positions=1152)
+    W, cfg = _oracle(model)
+    ids = np.random.default_rng(8).integers(0, 900, n).tolist()
+    with rt.session(bd3_session_config(32, 8, n)) as s:
+        got = s.execute_window(ids, list(range(n)), mask_geometry=(n, 32)).array()
+    ref = F.forward_full(W, cfg, ids, mask_kind="d2f_hybrid", mask_geometry=(n, 32),
+                         output_rows=list(range(n)))
+    err = rel_err_rows(got, ref)
+    _say(f"  rel err max={err.max():.2e}")
+    assert err.max() < LOGITS_REL_TOL
+    rt.close()
+
+
 @pytest.mark.parametrize("kind", ["q4", "bf16"])
 def test_bd3_full_decode_teacher_forced(kind):
     from diffusorrt_amd import decode
