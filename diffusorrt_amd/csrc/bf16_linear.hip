@@ -1,5 +1,6 @@
-// bf16-weight linear support for gfx950 (the GEMM itself is fused_linear.hip up to 32
-// rows, big_bf16.hip above):
+// bf16-weight linear support for gfx950 (the products themselves: skinny_linear.hip and
+// fused_linear.hip for few rows, big_bf16.hip for more, or for large weights; a model's
+// forwards go by their rows, the per-op calls by tiles, K and weights, bf16_linear_into):
 // y = bf16(x) @ W^T with fp32 accumulation, rounded to bf16 like the reference's
 // bf16 matmul output (backends/mlx_ops.py:122-125).
 //
@@ -38,16 +39,6 @@ void bf16_repack(const uint16_t* w, int N, int K, uint16_t* wb, hipStream_t s) {
 }  // namespace drt
 
 // ---- small fp32 <-> bf16 helpers used by the per-op entry points ----
-extern "C" __global__ void round_bf16_bias_kernel(float* __restrict__ y, int64_t n,
-                                                  const uint16_t* __restrict__ bias, int N) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    float v = round_bf16(y[i]);
-    if (bias) v += bf16_bits_to_float(bias[i % N]);
-    y[i] = v;
-  }
-}
-
 // eight values per thread; the last n % 8 one by one
 extern "C" __global__ __launch_bounds__(256) void to_bf16_kernel(const float* __restrict__ x,
                                                                  uint16_t* __restrict__ o,
@@ -68,12 +59,6 @@ extern "C" __global__ __launch_bounds__(256) void to_bf16_kernel(const float* __
 }
 
 namespace drt {
-
-void round_bf16_inplace(float* y, int64_t n, const uint16_t* bias, int N, hipStream_t s) {
-  const int blocks = (int)std::min<int64_t>((n + 255) / 256, 8192);
-  hipLaunchKernelGGL(round_bf16_bias_kernel, dim3(blocks), dim3(256), 0, s, y, n, bias, N);
-  DRT_HIP(hipGetLastError());
-}
 
 void to_bf16(const float* x, uint16_t* o, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)((n + 2047) / 2048)), dim3(256), 0, s, x, o, n);

@@ -1,12 +1,13 @@
-// Large-M bf16-weight linear for gfx950 (more than 32 rows): y = bf16(x) @ W^T with
-// fp32 accumulation, rounded to bf16 like the reference's bf16 matmul output
+// bf16-weight linear on shared operands for gfx950 (a model's forwards of more than 64 rows;
+// per-op calls where no kernel for few rows is faster): y = bf16(x) @ W^T with fp32
+// accumulation, rounded to bf16 like the reference's bf16 matmul output
 // (backends/mlx_ops.py:122-125).
 //
 // At these sizes the contraction is MFMA bound, so both operands are shared
 // through LDS: a work-group of WVM x WVN waves owns 32*TM*WVM rows x 32*TN*WVN
 // columns, and every byte it loads feeds 128 or 256 rows / columns.
 //   A (ACT_BF16, [M][K]) and B (the bf16 tile layout of bf16_linear.hip) are
-//     loaded per 64-k stage straight into LDS (global_load_lds), double buffered.
+//     loaded per 64-k stage straight into LDS (buffer loads to LDS), double buffered.
 //     A rows (128 B per stage) are stored with the 16-byte chunks of row r permuted
 //     (chunk c at position c ^ (r & 7) ^ ((r >> 3) & 1)): the MFMA fragment reads
 //     of 8 or 16 consecutive rows hit distinct bank groups. B is already in
@@ -15,8 +16,8 @@
 //     being read from the one being filled and waits for no load in flight.
 // k step t + 1's fragments are read while step t's MFMAs run; the stage after next
 // is issued at the last step's barrier, a whole stage of MFMAs ahead of its use.
-// Split-K over blockIdx.z (KS slices) writes fp32 partial slices y + ks * M * N that
-// a reduce pass sums and rounds.
+// Split-K (KS slices, the slowest index of the one-dimensional grid) writes fp32 partial
+// slices y + ks * M * N that a reduce pass sums and rounds.
 // Epilogues:
 //   EPI_STORE : y = bf16(tile) (+ bias); slices of a split, or without rnd_bf16: the
 //               fp32 sums

@@ -1,4 +1,5 @@
-// Large-M q4 linear for gfx950: the forwards of more than 32 rows (Dream's
+// Large-M q4 linear for gfx950: per-op calls of more than 32 rows and forwards of more than
+// 64 (Dream's
 // full canvas, BD3 prefix commits). At these sizes the contraction is MFMA
 // bound, so the weights are dequantized once per work-group into fp16 MFMA
 // operands (w = s * q + b, one fp16 rounding; backends/mlx_ops.py:97-130 for the

@@ -26,7 +26,7 @@ struct FusedArgs {
   int fenced = 0;
   int* placement_err = nullptr;
   // PRO_ACT: activation [M][K] (ACT_F16P + xsum[M][K/64], or ACT_BF16); for
-  // the split-K q4 store kernel also fp32 (x_in 1) or bf16 (x_in 2) rows
+  // the split-K store kernel also fp32 (x_in 1) or, q4 weights, bf16 (x_in 2) rows
   const void* act = nullptr;
   int x_in = 0;
   const float* act_xsum = nullptr;
@@ -140,7 +140,7 @@ void big_linear(const FusedArgs& a, int kind, const BigQ4Plan& p, hipStream_t s,
                 float* tail_part = nullptr, int* tail_count = nullptr);
 constexpr int BIG_TAIL_COUNTERS = 512;  // split tiles a caller's counters cover
 constexpr int BG_TAIL_KT_MAX = 8;       // K slices of one
-// The large-M bf16-weight kernels (M > 32, K % 64 == 0; big_bf16.hip): ACT_BF16
+// The bf16-weight kernels on shared operands (K % 64 == 0; big_bf16.hip): ACT_BF16
 // activation in, kinds FL_QKV, FL_SWIGLU (ACT_BF16 out) and FL_STORE (rounded with
 // the bias; ks > 1, or without rnd_bf16: fp32 slices y + ks * M * N for a reduce pass).
 struct BigBf16Plan {

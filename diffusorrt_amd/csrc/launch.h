@@ -239,7 +239,6 @@ void block_commit(const double* scores_d, const int32_t* tokens_d, const int32_t
                   StepDesc* advance = nullptr, const int32_t* quota_tab = nullptr);
 
 // y = round_bf16(y) (+ bias after rounding); x fp32 -> bf16 bits.
-void round_bf16_inplace(float* y, int64_t n, const uint16_t* bias, int N, hipStream_t s);
 void to_bf16(const float* x, uint16_t* o, int64_t n, hipStream_t s);
 
 // Per-op fp32 helpers (KernelTable seam).

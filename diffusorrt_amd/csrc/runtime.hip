@@ -137,7 +137,7 @@ struct Runtime {
   // gate|up kernel reads one and writes the other)
   bool sk_pre_on = false;
   DevBuf sk_pre, sk_pre_xs, sk_pre_sc;
-  // large-M (> 32 rows) q4 forwards: the down projection's input activation and
+  // large-M forwards: the down projection's input activation and
   // the split-K partial slices of o_proj / down_proj
   DevBuf act2, big_part, big_tail_count;
   size_t big_part_floats = 0;
@@ -2483,12 +2483,13 @@ constexpr float BB_OP_REDUCE_US = 4.f, BB_OP_SPLIT_US = 14.f;
 // kernel, where it takes the shape (1024 x 3072, 32 fp32 rows: 14.8 us with a cast of its
 // own before, 10.7, the host's part of a call; a second launch costs it 4 us more), unless
 // bf16 rows need no cast and the next kernel takes them (its call's host part is 0.4 us
-// shorter: no counters to look up). Else the kernel that streams a 32 x 32 tile's whole K, one launch, where its tiles fit one
-// round of the CUs and K is short enough to end before a split GEMM and its sum would
-// (bf16 rows: 512 x 3584, 200 rows 10.6 against 13.7; 3584 x 3584, 2 rows 10.3, 64 rows 12.0
-// against 13.8; but two rounds, 96 rows, 22.0 against 15.2, and K = 8192, 32 rows, 20.3
-// against 13.3, 9 rows 12.1 against 13.3). Else the shared-operand GEMM (18944 x 3584: 2
-// rows 30.5 -> 26.3, 32 rows 58 -> 29; 3584 x 18944: 91 -> 29).
+// shorter: no counters to look up). Else the kernel that streams a 32 x 32 tile's whole K,
+// one launch, where its tiles fit one round of the CUs and K is short enough to end before a
+// split GEMM and its sum would (bf16 rows: 512 x 3584, 200 rows 10.6 against 13.7; 3584 x
+// 3584, 2 rows 10.3, 64 rows 12.0 against 13.8; but two rounds, 96 rows, 22.0 against 15.2,
+// and K = 8192, 32 rows, 20.3 against 13.3, 9 rows 12.1 against 13.3). Else the
+// shared-operand GEMM (18944 x 3584: 2 rows 30.5 -> 26.3, 32 rows 58 -> 29; 3584 x 18944:
+// 91 -> 29).
 constexpr int64_t BB_SKINNY_WEIGHTS = (int64_t)8 << 20;
 static bool bf16_op_streams(int32_t m, int32_t n, int32_t k) {
   return (int64_t)(n / 32) * ((m + 31) / 32) <= n_cu_of_current_device() &&

@@ -21,9 +21,10 @@
 // (the dispatcher's round-robin), so the grid is laid out to give every slice
 // of block b the XCD b % n_xcc. Plain stores, the L2 atomic and plain loads are
 // then coherent with each other, with no device-wide fence (an L2 writeback and
-// invalidate per work-group costs tens of microseconds). Each work-group checks
-// the XCD it runs on and raises `placement_err` if the layout assumption fails,
-// which the host turns into an error. The runtime probes the placement once at
+// invalidate per work-group costs tens of microseconds). Each work-group but
+// the last of its block checks the XCD it runs on and raises `placement_err` if the layout
+// assumption fails, which the host turns into an error (per-op calls have no error word:
+// their stream is probed). The runtime probes the placement once at
 // creation; where it does not hold, the kernels run `fenced`: each slice's
 // stores are released at device scope before a device-scope arrival atomic,
 // and the last work-group acquires before reading the slices.

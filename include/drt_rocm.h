@@ -265,7 +265,8 @@ int32_t drt_op_kv_pack(const void* k, const void* v, int32_t src_dtype, int32_t 
  * over the tiled cache: q [rows, hq, 128] of kv_dtype, keys [0, n_keys), query row r at
  * absolute position row_pos0 + r. mask_kind: DRT_MASK_BIDIRECTIONAL or DRT_MASK_D2F_HYBRID
  * (with prompt_len / block_size). out [rows, hq*128] of out_dtype (DRT_F32 or DRT_BF16).
- * q is read in place by the kernels (no staging copy). */
+ * q is read in place by the kernels (no staging copy), and the cache straight into LDS in
+ * 16-byte pieces: cache 16-byte aligned, head_stride a multiple of 8. */
 size_t drt_op_attention_workspace_bytes(int32_t rows, int32_t hq, int32_t hkv, int32_t n_keys);
 int32_t drt_op_attention(const void* q, const void* cache, int64_t head_stride, int32_t kv_dtype,
                          int32_t rows, int32_t hq, int32_t hkv, int32_t n_keys, int32_t row_pos0,
