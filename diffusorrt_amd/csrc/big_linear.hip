@@ -584,9 +584,9 @@ float bg_cost(bool wide, int n, float g, int n_cu) {
 }
 }  // namespace
 
-// The plan of a per-op linear, or of the LM head: the cheapest estimate over the two tiles
-// and, for plain stores, the K slices (each at least four groups; reduce_us: what the reduce
-// pass costs besides its bytes) and the split last round: the tiles past whole rounds of one
+// The cheapest estimate over the two tiles and, for plain stores, the K slices (each at
+// least four groups; reduce_us: what the reduce pass costs besides its bytes), and for
+// unsplit stores and gate|up the split last round: the tiles past whole rounds of one
 // or two work-groups per CU over at most one K slice per CU. part_floats bounds the
 // slices and the split tiles' partials. Measured (hi + lo MFMA rates in brackets):
 // 512 x 18944 x 3584, 296 wide tiles: 155 us as they are, 156 as 592 narrow ones, 119
@@ -614,7 +614,7 @@ BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_flo
       if (ks > 1) us += reduce_us + (2 * ks + 1) * 0.5e-6f * M * N;  // 4 bytes each at 8 TB/s
       take(us, BigQ4Plan{wide, ks, 0, 0});
     }
-    if (!tail_ok || kind != FL_STORE) continue;
+    if (!tail_ok || (kind != FL_STORE && kind != FL_SWIGLU)) continue;
     for (int unit = 1; unit <= 2; ++unit) {
       const int full = T / (unit * n_cu) * (unit * n_cu), rest = T - full;
       if (rest == 0 || rest > BIG_TAIL_COUNTERS || full % 8) continue;
@@ -631,14 +631,14 @@ BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_flo
   return best;
 }
 
-// The plan of a linear inside a model's forward. Where its sums are cut along K is fixed by
-// the shape: big_linear_splits slices, and with split_last the gate|up tiles past whole
-// rounds of two per CU over the K slices that fill one more. The estimates above, which cut
-// more to the point (512 x 37888 x 3584: 247 us, 279 here without split_last; a 512-token
-// canvas 14.1 ms, 15.2 here), round the fp32 sums otherwise, and over 28 layers that moved the token of one
-// row in a few thousand of a canvas, whose two best logits were all but equal. The tile
-// changes no sum: the cheaper one.
-BigQ4Plan big_q4_forward_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+// The plan of a linear in a canvas's forward, whose tokens are chosen from it directly. Where
+// its sums are cut along K is fixed by the shape: big_linear_splits slices, and with
+// split_last the gate|up tiles past whole rounds of two per CU over the K slices that fill one
+// more. The estimates above, which cut more to the point (512 x 37888 x 3584: 247 us, 279 here
+// without split_last; a 512-token canvas 14.1 ms, 15.2 here), round the fp32 sums otherwise,
+// and over 28 layers that moved the token of one row in a few thousand, whose two best logits
+// were all but equal. The tile changes no sum: the cheaper one.
+BigQ4Plan big_q4_canvas_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
                               bool split_last) {
   const int n_cu = n_cu_of_current_device(), G = K / 64, MT = (M + BG_WM - 1) / BG_WM;
   const int T = MT * ((N + 255) / 256), S = 2 * n_cu, full = T / S * S, rest = T - full;
@@ -723,10 +723,13 @@ void sum_slices(const float* part, int KS, int64_t n, const uint16_t* bias, int 
   DRT_HIP(hipGetLastError());
 }
 
-void big_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s) {
-  const BigQ4Plan split = big_q4_forward_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, 0, false);
+void big_qkv(const FusedArgs& a, float* part, size_t part_floats, bool canvas, hipStream_t s) {
+  // (the epilogue pass: its own launch and 6 us besides its bytes)
+  const BigQ4Plan split =
+      canvas ? big_q4_canvas_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, 0, false)
+             : big_q4_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, part ? part_floats : 0, 6.f, false);
   if (split.ks == 1 || !part || (size_t)split.ks * a.M * a.N > part_floats) {
-    big_linear(a, FL_QKV, big_q4_forward_plan(a.M, a.N, a.K, FL_QKV, 1, 0, false), s);
+    big_linear(a, FL_QKV, big_q4_plan(a.M, a.N, a.K, FL_QKV, 1, 0, 0.f, false), s);
     return;
   }
   FusedArgs g = a;

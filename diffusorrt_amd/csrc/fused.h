@@ -134,7 +134,7 @@ struct BigQ4Plan {
 };
 BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
                       float reduce_us, bool tail_ok);
-BigQ4Plan big_q4_forward_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+BigQ4Plan big_q4_canvas_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
                               bool split_last);
 void big_linear(const FusedArgs& a, int kind, const BigQ4Plan& p, hipStream_t s,
                 float* tail_part = nullptr, int* tail_count = nullptr);
@@ -155,7 +155,7 @@ void big_bf16_linear(const FusedArgs& a, int kind, const BigBf16Plan& p, hipStre
 void big_bf16_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s);
 // q|k|v projection + epilogue: split-K into `part` (when the tiles alone would
 // leave CUs idle and part_floats suffices) and a separate epilogue pass.
-void big_qkv(const FusedArgs& a, float* part, size_t part_floats, hipStream_t s);
+void big_qkv(const FusedArgs& a, float* part, size_t part_floats, bool canvas, hipStream_t s);
 // The per-head q|k|v epilogue (bias, q/k norm, RoPE, Q out, K/V into the cache)
 // of a projection given as ks <= BG_QKV_MAX_KS fp32 slices [ks][M][N].
 void qkv_epilogue_slices(const FusedArgs& a, const float* part, int ks, hipStream_t s);

@@ -152,10 +152,10 @@ struct Runtime {
   bool streaming = false;
   int sk_n_counters = 0;
   int n_xcc = 1;
-  // The gate|up projection of large q4 forwards splits its last round along K: where the
+  // The gate|up projection of q4 canvases splits its last round along K: where the
   // stream's work-group 0 ran on XCD 0 at creation (a process with one hardware queue).
   // Elsewhere such forwards always ran without it, and the split would change their sums
-  // and with them a token now and then (see big_q4_forward_plan).
+  // and with them a token now and then (see big_q4_canvas_plan).
   bool split_last = false;
   bool fenced = false;           // split-K exchange through device-scope fences (no placement assumed)
   // scratch of the placement's probe, and whether it was probed (not overridden)
@@ -499,9 +499,10 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
       // between the q|k|v and down projections, which use it too)
       for (int mt = 1; mt <= (M + 127) / 128; ++mt) {
         const BigQ4Plan p =
-            big_q4_forward_plan(std::min(M, mt * 128), 2 * F, d, FL_SWIGLU, 1, SIZE_MAX, true);
+            big_q4_canvas_plan(std::min(M, mt * 128), 2 * F, d, FL_SWIGLU, 1, SIZE_MAX, true);
         bf = std::max(bf, (size_t)(mt * ((2 * F + 255) / 256) - p.full) * p.kt * 128 * 256);
       }
+      bf = std::max(bf, (size_t)n_cu_of_current_device() * 128 * 256);
       rt->big_part_floats = bf;
       rt->big_part.alloc(bf * 4);
       rt->big_tail_count.alloc((size_t)BIG_TAIL_COUNTERS * 4);
@@ -763,6 +764,8 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
   // (ACT_F16P, or ACT_BF16 for bf16 weights), the RMSNorms run as their own passes,
   // fused with the split-K reduce and residual add of the projection before them
   const bool big = M > 32 * SK_ROW_TILES;
+  // no mask: a canvas, whose sums are cut by shape alone (big_q4_canvas_plan)
+  const bool canvas = a.mask_kind == 0;
   // <= 32-row forwards of 7B-class layers: the weight-streaming linears (fp32 K
   // slices, reduced by small passes: residual add + row statistics, q|k|v
   // epilogue, SwiGLU; the RMSNorms run inside the next linear's staging)
@@ -817,7 +820,9 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       big_bf16_linear(f, FL_STORE, bp, s);
       return bp.ks;
     }
-    const BigQ4Plan bp = big_q4_forward_plan(M, f.N, f.K, FL_STORE, max_ks, 0, false);
+    const BigQ4Plan bp =
+        canvas ? big_q4_canvas_plan(M, f.N, f.K, FL_STORE, max_ks, 0, false)
+               : big_q4_plan(M, f.N, f.K, FL_STORE, max_ks, rt.big_part_floats, 0.f, false);
     require((size_t)bp.ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
     big_linear(f, FL_STORE, bp, s);
     return bp.ks;
@@ -875,7 +880,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       }
       if (big) {
         f.act = rt.act.p;
-        if (rt.q4) big_qkv(f, bpart, rt.big_part_floats, s);
+        if (rt.q4) big_qkv(f, bpart, rt.big_part_floats, canvas, s);
         else big_bf16_qkv(f, bpart, rt.big_part_floats, s);
       } else if (stream) {  // normed from the residual stream while staged
         qkv_epilogue_slices(f, bpart, slices(f, ST_QKV_MAX_KS), s);
@@ -924,8 +929,10 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       fg.act_fmt = fmt;
       if (rt.q4)
         big_linear(fg, FL_SWIGLU,
-                   big_q4_forward_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats,
-                                       rt.split_last),
+                   canvas ? big_q4_canvas_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats,
+                                               rt.split_last)
+                          : big_q4_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats, 0.f,
+                                        !rt.fenced && rt.n_xcc == 8),
                    s, bpart, rt.big_tail_count.as<int>());
       else
         big_bf16_linear(fg, FL_SWIGLU, big_bf16_plan(M, fg.N, fg.K, FL_SWIGLU, 1, 0, 0.f), s);
