@@ -631,14 +631,18 @@ BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_flo
   return best;
 }
 
-// The plan of a linear in a canvas's forward, whose tokens are chosen from it directly. Where
-// its sums are cut along K is fixed by the shape: big_linear_splits slices, and with
-// split_last the gate|up tiles past whole rounds of two per CU over the K slices that fill one
-// more. The estimates above, which cut more to the point (512 x 37888 x 3584: 247 us, 279 here
-// without split_last; a 512-token canvas 14.1 ms, 15.2 here), round the fp32 sums otherwise,
-// and over 28 layers that moved the token of one row in a few thousand, whose two best logits
-// were all but equal. The tile changes no sum: the cheaper one.
-BigQ4Plan big_q4_canvas_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+// The plan that cuts a linear's sums along K by its shape alone: big_linear_splits slices,
+// and with split_last the gate|up tiles past whole rounds of two per CU over the K slices that
+// fill one more. The tile changes no sum: the cheaper one.
+// For a canvas's forward, whose tokens are chosen from it directly: the estimates above, which
+// cut more to the point there (512 x 37888 x 3584: 247 us, 279 here without split_last; a
+// 512-token canvas 14.1 ms, 15.2 here), round the fp32 sums otherwise, and over 28 layers that
+// moved the token of one row in a few thousand, whose two best logits were all but equal.
+// For per-op calls that take slices: with fewer, or a split last round in their place, the
+// fp32 chains are longer (error against 64 bits up to 1.7 times, 512 rows of 3584 x 18944
+// 4.5e-7 and 6.3e-7), and the estimates miss by more than they gain (300 x 3584 x 3584: 55 us,
+// 39 here; 700 x 3584 x 18944: 292 and 198; 2048 x 2048 x 1024: 31 and 37).
+BigQ4Plan big_q4_shape_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
                               bool split_last) {
   const int n_cu = n_cu_of_current_device(), G = K / 64, MT = (M + BG_WM - 1) / BG_WM;
   const int T = MT * ((N + 255) / 256), S = 2 * n_cu, full = T / S * S, rest = T - full;
@@ -726,7 +730,7 @@ void sum_slices(const float* part, int KS, int64_t n, const uint16_t* bias, int 
 void big_qkv(const FusedArgs& a, float* part, size_t part_floats, bool canvas, hipStream_t s) {
   // (the epilogue pass: its own launch and 6 us besides its bytes)
   const BigQ4Plan split =
-      canvas ? big_q4_canvas_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, 0, false)
+      canvas ? big_q4_shape_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, 0, false)
              : big_q4_plan(a.M, a.N, a.K, FL_STORE, BG_QKV_MAX_KS, part ? part_floats : 0, 6.f, false);
   if (split.ks == 1 || !part || (size_t)split.ks * a.M * a.N > part_floats) {
     big_linear(a, FL_QKV, big_q4_plan(a.M, a.N, a.K, FL_QKV, 1, 0, 0.f, false), s);

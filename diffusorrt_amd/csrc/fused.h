@@ -134,7 +134,7 @@ struct BigQ4Plan {
 };
 BigQ4Plan big_q4_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
                       float reduce_us, bool tail_ok);
-BigQ4Plan big_q4_canvas_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
+BigQ4Plan big_q4_shape_plan(int M, int N, int K, int kind, int max_ks, size_t part_floats,
                               bool split_last);
 void big_linear(const FusedArgs& a, int kind, const BigQ4Plan& p, hipStream_t s,
                 float* tail_part = nullptr, int* tail_count = nullptr);

@@ -155,7 +155,7 @@ struct Runtime {
   // The gate|up projection of q4 canvases splits its last round along K: where the
   // stream's work-group 0 ran on XCD 0 at creation (a process with one hardware queue).
   // Elsewhere such forwards always ran without it, and the split would change their sums
-  // and with them a token now and then (see big_q4_canvas_plan).
+  // and with them a token now and then (see big_q4_shape_plan).
   bool split_last = false;
   bool fenced = false;           // split-K exchange through device-scope fences (no placement assumed)
   // scratch of the placement's probe, and whether it was probed (not overridden)
@@ -499,7 +499,7 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
       // between the q|k|v and down projections, which use it too)
       for (int mt = 1; mt <= (M + 127) / 128; ++mt) {
         const BigQ4Plan p =
-            big_q4_canvas_plan(std::min(M, mt * 128), 2 * F, d, FL_SWIGLU, 1, SIZE_MAX, true);
+            big_q4_shape_plan(std::min(M, mt * 128), 2 * F, d, FL_SWIGLU, 1, SIZE_MAX, true);
         bf = std::max(bf, (size_t)(mt * ((2 * F + 255) / 256) - p.full) * p.kt * 128 * 256);
       }
       bf = std::max(bf, (size_t)n_cu_of_current_device() * 128 * 256);
@@ -764,7 +764,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
   // (ACT_F16P, or ACT_BF16 for bf16 weights), the RMSNorms run as their own passes,
   // fused with the split-K reduce and residual add of the projection before them
   const bool big = M > 32 * SK_ROW_TILES;
-  // no mask: a canvas, whose sums are cut by shape alone (big_q4_canvas_plan)
+  // no mask: a canvas, whose sums are cut by shape alone (big_q4_shape_plan)
   const bool canvas = a.mask_kind == 0;
   // <= 32-row forwards of 7B-class layers: the weight-streaming linears (fp32 K
   // slices, reduced by small passes: residual add + row statistics, q|k|v
@@ -821,7 +821,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       return bp.ks;
     }
     const BigQ4Plan bp =
-        canvas ? big_q4_canvas_plan(M, f.N, f.K, FL_STORE, max_ks, 0, false)
+        canvas ? big_q4_shape_plan(M, f.N, f.K, FL_STORE, max_ks, 0, false)
                : big_q4_plan(M, f.N, f.K, FL_STORE, max_ks, rt.big_part_floats, 0.f, false);
     require((size_t)bp.ks * M * f.N <= rt.big_part_floats, "large-M partials exceed the workspace");
     big_linear(f, FL_STORE, bp, s);
@@ -929,7 +929,7 @@ void launch_forward(Runtime& rt, void* kv, int64_t head_stride, int64_t layer_st
       fg.act_fmt = fmt;
       if (rt.q4)
         big_linear(fg, FL_SWIGLU,
-                   canvas ? big_q4_canvas_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats,
+                   canvas ? big_q4_shape_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats,
                                                rt.split_last)
                           : big_q4_plan(M, fg.N, fg.K, FL_SWIGLU, 1, rt.big_part_floats, 0.f,
                                         !rt.fenced && rt.n_xcc == 8),
@@ -2397,20 +2397,24 @@ static void q4_linear_into(const void* qw, const void* sb, const void* x, int32_
       stream_linear(g, sp, st);
       sum_slices(part, sp.KS, (int64_t)m * n, (const uint16_t*)bias, n, y, st);
     } else if (m > 32) {
-      // planned within the slices the workspace rule provides (the same plan whichever
-      // workspace is passed); the split last round needs a counter block of this stream,
-      // which a graph capture cannot own (its replays may run beside the stream's calls)
+      // as many slices as the shape says (and the workspace rule provides), or unsplit; then
+      // the split last round needs a counter block of this stream, which a graph capture
+      // cannot own (its replays may run beside the stream's calls)
       float* part = (float*)(ws + q4_op_act_bytes(m, k));
-      const size_t part_floats = (size_t)big_linear_splits(m, n, k, BG_OP_MAX_KS) * m * n;
-      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-      DRT_HIP(hipStreamIsCapturing(st, &cap));
+      const int ks = big_linear_splits(m, n, k, BG_OP_MAX_KS);
       FusedArgs g = f;
       int* count = nullptr;
       bool fenced = true;
-      if (cap == hipStreamCaptureStatusNone) count = op_counters_for(st, g.n_xcc, fenced);
+      if (ks == 1) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        DRT_HIP(hipStreamIsCapturing(st, &cap));
+        if (cap == hipStreamCaptureStatusNone) count = op_counters_for(st, g.n_xcc, fenced);
+      }
       g.fenced = fenced ? 1 : 0;
-      const BigQ4Plan p = big_q4_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, part_floats, 2.5f,
-                                      count && !fenced && g.n_xcc == 8);
+      const BigQ4Plan p =
+          ks > 1 ? big_q4_shape_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, 0, false)
+                 : big_q4_plan(m, n, k, FL_STORE, 1, (size_t)m * n, 0.f,
+                               count && !fenced && g.n_xcc == 8);
       if (p.ks > 1) {  // slices, summed (+ bias) into y in a fixed order
         g.bias = nullptr;
         g.y = part;

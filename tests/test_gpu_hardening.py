@@ -84,7 +84,7 @@ def test_fenced_split_k_exchange_is_bit_identical():
 
 
 # Scores and tokens of a q4 canvas, bit for bit as they always were: every fp32 sum of such a
-# forward is cut along K where the shape says (big_q4_canvas_plan) and its probabilities are
+# forward is cut along K where the shape says (big_q4_shape_plan) and its probabilities are
 # rounded one way (attn_split_tile), whatever the kernels' tiles and launches. Otherwise a row
 # whose two best logits are all but equal takes its other token. 512 rows attend in two key
 # ranges (met in one work-group), 257 in four, 100 in more; the gate|up projection stays below

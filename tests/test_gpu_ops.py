@@ -350,6 +350,26 @@ def test_linears_of_two_threads_on_the_per_thread_stream():
             assert ((o - y).norm() <= tol * y.norm()).item()
 
 
+# Sums over as many K slices as the shape says (big_q4_shape_plan: 8, 6, 6 and 2), bit for bit
+# as they always were: with fewer the fp32 chains are longer and the results further off.
+_SLICED_DIGESTS = {(300, 3584, 3584): "0c4da08d30913597", (700, 3584, 3584): "192c3c7b1c3859f8",
+                   (41, 18944, 3584): "ebd33d7484cdaee7", (1000, 2048, 1024): "f56ff14fd4cde433"}
+
+
+@pytest.mark.parametrize("m,n,k", sorted(_SLICED_DIGESTS))
+def test_q4_linear_sums_are_cut_by_shape(m, n, k):
+    import hashlib
+
+    from diffusorrt_amd import kernels
+
+    _say("q4_linear bits", m, n, k)
+    gen, q = _q4_case(n, k, seed=39)
+    x = torch.randn((m, k), generator=gen)
+    w = kernels.DeviceQ4Weight(q.w_q.cuda(), q.scales.cuda(), q.biases.cuda())
+    y = kernels.linear(x.cuda(), w).cpu().numpy()
+    assert hashlib.sha256(y.tobytes()).hexdigest()[:16] == _SLICED_DIGESTS[(m, n, k)]
+
+
 # ---------------------------------------------------------------- attention (config 2)
 
 def _attention_inputs(L, seed=1, rows=32, hq=16, hkv=8):
