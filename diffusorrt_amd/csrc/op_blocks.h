@@ -43,14 +43,16 @@ class CounterBlocks {
   // (the same bits). Only calls on the same stream wait for its probe.
   template <class Capturing, class Probe>
   static bool fenced(Block& b, Capturing&& capturing, Probe&& probe) {
-    if (b.form == UNKNOWN) {
+    int form = b.form.load(std::memory_order_relaxed);
+    if (form == UNKNOWN) {
       std::lock_guard<std::mutex> lock(b.mu);
-      if (b.form == UNKNOWN) {
+      form = b.form;
+      if (form == UNKNOWN) {
         if (capturing()) return true;
-        b.form = probe() < 0 ? FENCED : IN_L2;
+        b.form = form = probe() < 0 ? FENCED : IN_L2;
       }
     }
-    return b.form == FENCED;
+    return form == FENCED;
   }
 
   static constexpr uintptr_t PER_THREAD = 2;  // hipStreamPerThread

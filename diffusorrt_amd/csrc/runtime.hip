@@ -16,6 +16,7 @@
 // re-associated.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
@@ -2270,13 +2271,13 @@ static __device__ int op_counters[OP_COUNTER_BLOCKS * OP_COUNTERS];
 static __device__ int op_probe[OP_COUNTER_BLOCKS * 256];
 namespace {
 struct OpDevice {
-  std::once_flag once;
-  int* counters = nullptr;
+  std::atomic<int*> counters{nullptr};  // (set last)
   int* probe = nullptr;
   int n_xcc = 1;
   CounterBlocks blocks;
 };
 constexpr int OP_DEVICES = 64;
+std::mutex g_op_mu;
 OpDevice g_op_dev[OP_DEVICES];
 
 // The counter block of (current device, stream) and the form of its exchange, or nullptr
@@ -2286,17 +2287,22 @@ int* op_counters_for(hipStream_t stream, int& n_xcc, bool& fenced) {
   DRT_HIP(hipGetDevice(&dev));
   if (dev >= OP_DEVICES) return nullptr;
   OpDevice* d = &g_op_dev[dev];
-  std::call_once(d->once, [&] {  // (a call that throws leaves it to the next)
+  int* counters = d->counters.load(std::memory_order_acquire);
+  if (!counters) {
+    std::lock_guard<std::mutex> lock(g_op_mu);
     void* c = nullptr;
     void* pr = nullptr;
     DRT_HIP(hipGetSymbolAddress(&c, HIP_SYMBOL(op_counters)));
     DRT_HIP(hipGetSymbolAddress(&pr, HIP_SYMBOL(op_probe)));
     int nx = 1;
     if (hipDeviceGetAttribute(&nx, hipDeviceAttributeNumberOfXccs, dev) != hipSuccess) nx = 1;
-    d->n_xcc = std::max(1, nx);
-    d->probe = (int*)pr;
-    d->counters = (int*)c;
-  });
+    if (!d->counters.load(std::memory_order_relaxed)) {
+      d->n_xcc = std::max(1, nx);
+      d->probe = (int*)pr;
+      d->counters.store((int*)c, std::memory_order_release);
+    }
+    counters = (int*)c;
+  }
   CounterBlocks::Block* b = d->blocks.of((uintptr_t)stream);
   if (!b) return nullptr;
   n_xcc = d->n_xcc;
@@ -2311,7 +2317,7 @@ int* op_counters_for(hipStream_t stream, int& n_xcc, bool& fenced) {
         return cap != hipStreamCaptureStatusNone;
       },
       [&] { return probe_round_robin(d->n_xcc, d->probe + 256 * b->index, stream); });
-  return d->counters + (size_t)b->index * OP_COUNTERS;
+  return counters + (size_t)b->index * OP_COUNTERS;
 }
 }  // namespace
 
@@ -2513,20 +2519,26 @@ static bool bf16_op_skinny(int32_t m, int32_t n, int32_t k) {
 }
 static size_t bf16_op_x_bytes(int32_t m, int32_t k) { return ((size_t)m * k * 2 + 255) / 256 * 256; }
 
-// the split-K slices, or the split-K kernel's partial tiles
-size_t drt_op_bf16_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
+// the split-K slices, or the split-K kernel's partial tiles (f32: of fp32 rows)
+static size_t bf16_op_part_bytes(int32_t m, int32_t n, int32_t k, bool f32) {
   if (m <= 0 || n <= 0 || k <= 0 || n % 32 || k % 64) return 256;
-  if (bf16_op_skinny(m, n, k)) return skinny_part_floats(n, k) * 4 * SK_ROW_TILES;
-  if (bf16_op_streams(m, n, k)) return 256;
+  const bool streams = bf16_op_streams(m, n, k);
+  if ((f32 || !streams) && bf16_op_skinny(m, n, k))
+    return skinny_part_floats(n, k) * 4 * SK_ROW_TILES;
+  if (streams) return 256;
   const BigBf16Plan p = big_bf16_plan(m, n, k, FL_STORE, BG_OP_MAX_KS, SIZE_MAX, BB_OP_REDUCE_US,
                                       BB_OP_SPLIT_US);
   return p.ks > 1 ? (size_t)p.ks * m * n * 4 : 256;
 }
 
+size_t drt_op_bf16_linear_workspace_bytes(int32_t m, int32_t n, int32_t k) {
+  return bf16_op_part_bytes(m, n, k, false);
+}
+
 // ... and the rows rounded to bf16 for the kernels that do not do that themselves
 size_t drt_op_bf16_linear_x_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  return bf16_op_x_bytes(m, k) + drt_op_bf16_linear_workspace_bytes(m, n, k);
+  return bf16_op_x_bytes(m, k) + bf16_op_part_bytes(m, n, k, true);
 }
 
 // x bf16, or with xb fp32 (rounded to bf16 into xb where no kernel does it on the way)
@@ -2542,11 +2554,15 @@ static void bf16_linear_into(const void* wb, const void* x, void* xb, int32_t m,
   f.act = x;
   f.rnd_bf16 = 1;  // the bf16 matmul output is bf16; the bias is added after
   f.y = y;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  DRT_HIP(hipStreamIsCapturing(st, &cap));
-  if (bf16_op_skinny(m, n, k) && (xb || !bf16_op_streams(m, n, k)) && workspace &&
-      workspace_bytes >= skinny_part_floats(n, k) * 4 * SK_ROW_TILES &&
-      cap == hipStreamCaptureStatusNone) {
+  const bool streams = bf16_op_streams(m, n, k);
+  bool counters = (xb || !streams) && workspace && bf16_op_skinny(m, n, k) &&
+                  workspace_bytes >= skinny_part_floats(n, k) * 4 * SK_ROW_TILES;
+  if (counters) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    DRT_HIP(hipStreamIsCapturing(st, &cap));
+    counters = cap == hipStreamCaptureStatusNone;
+  }
+  if (counters) {
     // one launch, its counters this stream's (a graph's replays would share them)
     FusedArgs g = f;
     g.x_in = xb ? 1 : 0;
@@ -2563,7 +2579,7 @@ static void bf16_linear_into(const void* wb, const void* x, void* xb, int32_t m,
     to_bf16((const float*)x, (uint16_t*)xb, (int64_t)m * k, st);
     f.act = xb;
   }
-  if (bf16_op_streams(m, n, k) || !big_bf16_supported(f, FL_STORE)) {
+  if (streams || !big_bf16_supported(f, FL_STORE)) {
     fused_linear(f, FL_STORE, st);
     return;
   }

@@ -105,13 +105,17 @@ def linear(x, weight, bias=None):
                                         _lib.BF16 if x.dtype == torch.bfloat16 else _lib.F32,
                                         m, n, k, bptr, _ptr(y), _ptr(ws), ws_bytes, _stream(x)))
     elif isinstance(weight, DeviceBF16Weight):
-        if x.dtype != torch.float32:
-            x = x.to(torch.bfloat16).contiguous()
-        ws_bytes = lib.drt_op_bf16_linear_x_workspace_bytes(m, n, k)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-        _lib.check(lib.drt_op_bf16_linear_x(_ptr(weight.wb), _ptr(x),
-                                            _lib.F32 if x.dtype == torch.float32 else _lib.BF16,
-                                            m, n, k, bptr, _ptr(y), _ptr(ws), ws_bytes, _stream(x)))
+        if x.dtype == torch.float32:  # rounded to bf16 on the way
+            ws_bytes = lib.drt_op_bf16_linear_x_workspace_bytes(m, n, k)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+            _lib.check(lib.drt_op_bf16_linear_x(_ptr(weight.wb), _ptr(x), _lib.F32, m, n, k, bptr,
+                                                _ptr(y), _ptr(ws), ws_bytes, _stream(x)))
+        else:
+            xb = x.to(torch.bfloat16).contiguous()
+            ws_bytes = lib.drt_op_bf16_linear_workspace_bytes(m, n, k)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+            _lib.check(lib.drt_op_bf16_linear(_ptr(weight.wb), _ptr(xb), m, n, k, bptr, _ptr(y),
+                                              _ptr(ws), ws_bytes, _stream(x)))
     else:
         raise ValueError("linear weight must be a DeviceQ4Weight or DeviceBF16Weight")
     return y
