@@ -2,8 +2,8 @@
 //
 // Queries of one KV head are flattened to query vectors qv = row * G + gi
 // (G = Hq / Hkv, head = kvh * G + gi) and processed in 32-vector tiles, one
-// tile per wave. Keys come in 32-key tiles staged through LDS (double
-// buffered) and shared by the QW waves of a work-group.
+// tile per wave. Keys come in 32-key tiles streamed into LDS and shared by the QW
+// waves of a key group.
 //
 // Per 32x32 tile the wave computes S^T = K Q^T (8 MFMAs over head_dim 128), so
 // lane l owns query (l & 31) and 16 of its 32 keys; the partner lane l ^ 32
@@ -129,8 +129,8 @@ DRT_DEV void store_attn8(const f32x4 v0, const f32x4 v1, int row, int n_rows, in
 // so one iteration of prefetch) put twice the work-groups on the chip where two groups of
 // four leave CUs idle: 1000 x 16 heads over 1000 keys, 256 work-groups instead of 128, 24.2
 // -> 18.0 us.
-// 2048 rows x 16 heads over 4096 keys, bf16: 135 -> 77 us with the combine (671 TFLOP/s; K/V
-// staged through registers, products with a zero lo plane, a mask test per score before).
+// 2048 rows x 16 heads over 4096 keys, bf16: 134 -> 73 us (711 TFLOP/s; K/V staged through
+// registers, products with a zero lo plane, a mask test per score before).
 template <typename T, int QW, int KG, bool LO, bool OUT, bool MASK>
 DRT_DEV void attn_split_tile(
     const T* __restrict__ q,       // [n_rows][Hq][128]
