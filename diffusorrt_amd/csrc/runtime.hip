@@ -521,12 +521,13 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     // keys 1565 against 1255 us) - and where there is none the split-K exchange runs
     // fenced (DRT_SPLITK_FENCED=1 forces that). The rotation itself is taken anew by each
     // forward's first kernel: queues created later move it.
+    int rot = -1;
     const char* nx_env = getenv("DRT_N_XCC");
     if (nx_env && atoi(nx_env) >= 1) {
       rt->n_xcc = atoi(nx_env);
     } else {
       rt->xcc_probe.alloc(256 * sizeof(int));
-      const int rot = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s);
+      rot = probe_round_robin(rt->n_xcc, rt->xcc_probe.as<int>(), s);
       rt->fenced = rot < 0;
       rt->xcc_probed = true;
       rt->split_last = rot == 0 && rt->n_xcc == 8;
@@ -541,11 +542,15 @@ std::shared_ptr<Runtime> create_runtime(const drt_engine_config& e, const drt_mo
     *rt->placement_host = 0;
     // DRT_PLACEMENT_WORD=seen,word[,count] (a test hook): the first check of the error word
     // sees `seen`, while the device's already holds `word`, as with a block queued behind,
-    // and the last arrival counter (of a second row tile) `count`
+    // and the last arrival counter (of a second row tile) `count`. A placement report (1)
+    // without a rotation gets the stream's.
     if (const char* w = getenv("DRT_PLACEMENT_WORD")) {
       char* rest = nullptr;
-      rt->test_seen = (int)strtol(w, &rest, 10);
-      const int word = *rest == ',' ? (int)strtol(rest + 1, &rest, 10) : 0;
+      auto report = [rot](int v) {
+        return (v & 1) && v < placement_bit(0) && rot >= 0 ? v | placement_bit(rot) : v;
+      };
+      rt->test_seen = report((int)strtol(w, &rest, 10));
+      const int word = report(*rest == ',' ? (int)strtol(rest + 1, &rest, 10) : 0);
       const int count = *rest == ',' ? (int)strtol(rest + 1, nullptr, 10) : 0;
       DRT_HIP(hipMemcpyAsync(rt->placement_err.p, &word, 4, hipMemcpyHostToDevice, s));
       DRT_HIP(hipMemcpyAsync(rt->sk_counters.as<char>() + rt->sk_counters.bytes - 4, &count, 4,
